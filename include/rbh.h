@@ -115,9 +115,10 @@ typedef struct rbh_step_log {
 typedef struct rbh_tuning {
   int unit_size;          /* contact positions per colouring unit window (default 64) */
   int lanes_per_scene;    /* sweep lanes of a batched scene, about one per wavefront (default 4) */
-  int resident_contacts;  /* most contacts of a solve group kept in LDS (multiple of 64; at most 384, FP64 192) */
-  int resident_bodies;    /* most bodies of a solve group kept in LDS (multiple of 64; same bounds) */
-  int lanes_per_group;    /* a single scene's cooperative grid: lanes per workgroup (default 4) */
+  int resident_contacts;  /* most contacts of a solve group kept in LDS (multiple of 64; at most 384, FP64 192;
+                             default: what fits) */
+  int resident_bodies;    /* most bodies of a solve group kept in LDS (multiple of 64; same bounds and default) */
+  int lanes_per_group;    /* a single scene's cooperative grid: lanes per workgroup (default 1) */
   int waves_per_group;    /* wavefronts per workgroup of the batched solve: 4 (default) or 8 */
   int color_lds_contacts; /* most contacts of a colouring unit whose colouring state is kept in LDS
                              (default and upper bound 4096; larger units keep it in global memory) */

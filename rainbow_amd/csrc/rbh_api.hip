@@ -13,6 +13,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <cstdio>
 #include <cstddef>
@@ -175,7 +176,7 @@ struct rbh_ctx {
   int unit_T = 64;          // contacts per colouring unit (a scene's units are windows of this size)
   rbh_tuning tune{};        // rbh_set_tuning (0 fields: defaults)
   // resident solve groups: LDS capacities (contacts, bodies, colour offsets) and the launch's dynamic LDS
-  int res_cap_c = 0, res_cap_b = 0, res_cap_o = 0;
+  int res_cap_c = 0, res_cap_b = 0;
   size_t solve_lds = 0, solve_lds_half = 0;   // full and half layouts (one or two workgroups per CU)
   int max_iter_batch = 1, coop_max = 0, last_units = 0;
   bool multi_ok = false;
@@ -544,7 +545,7 @@ template <typename R> Dev<R> make_dev(rbh_ctx* c, double dt, int flags, bool mul
   d.s_loc = P(int2*, s_loc); d.s_W = P(V4<R>*, s_W);
   d.s_JL = P(V4<R>*, s_JL); d.s_JA = P(V4<R>*, s_JA); d.s_JB = P(V4<R>*, s_JB);
   d.xr0 = P(R*, xr0); d.xr1 = P(R*, xr1);
-  d.res_cap_c = c->res_cap_c; d.res_cap_b = c->res_cap_b; d.res_cap_o = c->res_cap_o;
+  d.res_cap_c = c->res_cap_c; d.res_cap_b = c->res_cap_b;
   d.l_cnt = P(int*, l_cnt); d.l_base = P(int*, l_base); d.n_lanes = P(int*, n_lanes);
   d.l_start = P(int*, l_start); d.l_end = P(int*, l_end); d.l_ncol = P(int*, l_ncol); d.l_bs = P(int*, l_bs);
   d.u_start = P(int*, u_start); d.u_end = P(int*, u_end); d.u_ncol = P(int*, u_ncol);
@@ -875,15 +876,13 @@ int first_step_index(rbh_ctx* c, int slot, int* out) {
   return 0;
 }
 
-// Dynamic LDS of the solve kernels: the resident layout (FP32: 384 contacts,
-// 384 bodies, ~130 KB; FP64: half) or the velocity-only layout,
-// whichever is larger; the kernels' limit is raised to it.
+// Dynamic LDS of the solve kernels: a CU's (full layout) or half of it, less
+// their static LDS; the kernels' limit is raised to it.  A group is resident
+// if its bodies, contacts and schedule fit (and the tuning's bounds, if set).
 template <typename R> int setup_solve_lds(rbh_ctx* c) {
-  c->res_cap_c = c->tune.resident_contacts > 0 ? std::min(c->tune.resident_contacts, ResCap<R>::C) : ResCap<R>::C;
-  c->res_cap_b = c->tune.resident_bodies > 0 ? std::min(c->tune.resident_bodies, ResCap<R>::B) : ResCap<R>::B;
-  c->res_cap_o = ResCap<R>::O;
-  const size_t bytes = std::max<size_t>(SOLVE_LDS_BYTES, ResCap<R>::BYTES);
-  const size_t half = std::max<size_t>(SOLVE_LDS_BYTES, ResCap<R, 1>::BYTES);
+  c->res_cap_c = c->tune.resident_contacts > 0 ? std::min(c->tune.resident_contacts, ResCap<R>::C) : INT_MAX;
+  c->res_cap_b = c->tune.resident_bodies > 0 ? std::min(c->tune.resident_bodies, ResCap<R>::B) : INT_MAX;
+  const size_t bytes = ResCap<R>::LDS, half = ResCap<R, 1>::LDS;
   const void* ks[5] = {reinterpret_cast<const void*>(k_solve<R, SOLVE_BLOCK, 0>),
                        reinterpret_cast<const void*>(k_solve<R, 512, 0>),
                        reinterpret_cast<const void*>(k_solve_multi<R>),
@@ -939,8 +938,10 @@ template <typename R> int run_steps(rbh_ctx* c, int n_steps, double dt, int flag
   bool multi = c->multi_ok && !use_graph;
   if (flags & RBH_STEP_FORCE_SINGLE) multi = false;
   if ((flags & RBH_STEP_FORCE_MULTI) && c->multi_ok && !use_graph) multi = true;
-  // cooperative grid: about one unit per wavefront, from the unit count of the last step seen
-  const int lpw = c->tune.lanes_per_group > 0 ? c->tune.lanes_per_group : SOLVE_BLOCK / 64;
+  // cooperative grid, from the unit count of the last step seen: one lane per workgroup while the device
+  // has room for them, so that a lane's wavefront shares its CU's LDS with no other and few groups outgrow
+  // the resident layout (4096 spheres: solve 875 us, with four lanes per workgroup 1137)
+  const int lpw = c->tune.lanes_per_group > 0 ? c->tune.lanes_per_group : 1;
   auto grid_of = [&](int units) { return std::max(1, std::min((units + lpw - 1) / lpw, c->coop_max)); };
   int multi_grid = grid_of(c->last_units > 1 ? c->last_units : 64);
   int done = 0;

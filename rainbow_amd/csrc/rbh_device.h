@@ -247,6 +247,24 @@ template <typename R> __device__ __forceinline__ void prox_sphere(R zs, R zt, R 
   os = zs * scale; ot = zt * scale; orr = zr * scale;
 }
 
+// prox_sphere for a lane that holds one of the three values: z projected, sq
+// the sum of the three squares (added in prox_sphere's order).  The same
+// result; in FP32 by selects (a branch costs a lone wavefront more than the
+// arithmetic), in FP64 past a branch, since its square root and division are
+// long sequences.
+template <typename R> __device__ __forceinline__ R prox_sphere_row(R z, R sq, R mu, R xn) {
+  const R radius = mu * xn;
+  if constexpr (sizeof(R) == 4) {
+    const R f = sq <= radius * radius ? R(1) : radius * __builtin_amdgcn_rsqf(sq);
+    const R v = z * f;
+    return xn <= R(0) ? R(0) : v;
+  } else {
+    if (xn <= R(0)) return R(0);
+    if (sq <= radius * radius) return z;
+    return z * (radius / sqrt(sq));
+  }
+}
+
 // First term of a velocity-change sum: FP64 starts from 0 as the reference's
 // sparse products do (0 + p only differs from p for p = -0); FP32 starts from p.
 template <typename R> __device__ __forceinline__ R sum_first(R p) {

@@ -136,7 +136,7 @@ template <typename R> struct Dev {
   // solver arrays (colour order)
   int* perm; int2* s_id; V4<R>* s_n; V4<R>* s_rA; V4<R>* s_rB; V4<R>* s_b; V4<R>* s_r0; V4<R>* x0; V4<R>* x1;
   int2* s_loc;                         // body slots (u_blist index) of the two bodies (-1: fixed)
-  int res_cap_c, res_cap_b, res_cap_o; // LDS capacities of a resident solve group (contacts, bodies, colour offsets)
+  int res_cap_c, res_cap_b;            // most contacts and bodies of a resident solve group (rbh_tuning)
   V4<R>* s_W;                          // 4 per position: W0, W1 of body A, then of body B (zero if fixed)
   V4<R>* s_JL; V4<R>* s_JA; V4<R>* s_JB;   // rows 4 pos + r of J: (lin_r, b_r), (angA_r, r0_r), (angB_r, mu_r)
   R* xr0; R* xr1;                      // iterates by row (4 pos + r), for the row-major sweeps

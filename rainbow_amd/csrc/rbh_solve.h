@@ -1756,11 +1756,11 @@ __device__ void solve_group(const Dev<R>& d, const int slot, const Group& gr, V4
 
 // value of lane K of each quad (DPP quad_perm(K, K, K, K))
 template <int K> __device__ __forceinline__ float quad_bcast(float v) {
-  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), K * 0x55, 0xf, 0xf, false));
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), K * 0x55, 0xf, 0xf, true));
 }
 template <int K> __device__ __forceinline__ double quad_bcast(double v) {
-  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), K * 0x55, 0xf, 0xf, false);
-  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), K * 0x55, 0xf, 0xf, false);
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), K * 0x55, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), K * 0x55, 0xf, 0xf, true);
   return __hiloint2double(hi, lo);
 }
 
@@ -1888,24 +1888,24 @@ __device__ __forceinline__ void load_quad(const V4<R>* JL, const V4<R>* JA, cons
   it.lc = make_int2((lc.x >= 0 ? lc.x - b0 : zs) * rec_bytes<R>(), (lc.y >= 0 ? lc.y - b0 : zs) * rec_bytes<R>());
 }
 
-// natural-map residual parts of contact i (FP64) from its rows and the
-// accepted velocity changes; the impulses' final values
-template <typename R>
+// natural-map residual parts of a contact (FP64) from its rows (row r at JL[S r],
+// JA[S r], JB[S r]), its final values xs[0..3] and the accepted velocity changes
+template <typename R, int S>
 __device__ __forceinline__ void quad_finish_contact(const ProxParams& pp, const V4<R>* JL, const V4<R>* JA,
-                                                    const V4<R>* JB, const R* xs, int i, const V4<R>& lA,
-                                                    const V4<R>& aA, const V4<R>& lB, const V4<R>& aB, V4<R>& x,
-                                                    double& rloc, double& xmax) {
-  x = V4<R>{xs[4 * (size_t)i], xs[4 * (size_t)i + 1], xs[4 * (size_t)i + 2], xs[4 * (size_t)i + 3]};
+                                                    const V4<R>* JB, const R* xs, const V4<R>& lA, const V4<R>& aA,
+                                                    const V4<R>& lB, const V4<R>& aB, V4<R>& x, double& rloc,
+                                                    double& xmax) {
+  x = V4<R>{xs[0], xs[1], xs[2], xs[3]};
   ContactRow<R> J;
   V4<R> bb, r0;
   R* bp = &bb.x;
   R* rp = &r0.x;
   for (int r = 0; r < 4; ++r) {
-    const V4<R> a = JL[4 * (size_t)i + r], e = JA[4 * (size_t)i + r], f = JB[4 * (size_t)i + r];
+    const V4<R> a = JL[S * r], e = JA[S * r], f = JB[S * r];
     J.lin[r] = xyz(a); J.angA[r] = xyz(e); J.angB[r] = xyz(f);
     bp[r] = a.w; rp[r] = e.w;
   }
-  const V4<R> mu = {JB[4 * (size_t)i + 1].w, JB[4 * (size_t)i + 2].w, JB[4 * (size_t)i + 3].w, R(0)};
+  const V4<R> mu = {JB[S].w, JB[2 * S].w, JB[3 * S].w, R(0)};
   const V4<R> y = contact_prox(pp, J, x, bb, r0, mu, xyz(lA), xyz(aA), xyz(lB), xyz(aB), false);
   rloc = fmax(rloc, absmax4((double)x.x - (double)y.x, (double)x.y - (double)y.y, (double)x.z - (double)y.z,
                             (double)x.w - (double)y.w));
@@ -1913,57 +1913,69 @@ __device__ __forceinline__ void quad_finish_contact(const ProxParams& pp, const 
 }
 
 // ---- resident layout
-// Per contact i the four rows r of J (row 4i + r: JL = (lin_r, b_r),
-// JA = (angA_r, r0_r), JB = (angB_r, mu_r), mu_1..3 the friction
-// coefficients) and the iterates X0/X1[4i + r] are staged in LDS once per
-// solve; so are the group's bodies.  A sweep issues no global memory access.
-// Body arrays hold cb + 2 entries: slot cb stays zero and stands for every
-// fixed body, slot cb + 1 takes the discarded updates of fixed bodies, so a
-// contact's loads and stores never branch on fixed bodies.  Contact entry cc
-// is the null contact (zero rows and iterates, both bodies in the zero slot):
-// a quad with no contact in a colour updates it, which changes nothing.
-template <typename R> __host__ __device__ constexpr size_t res_lds_bytes(int cc, int cb, int co, int cl) {
-  return (size_t)(cc + 1) * (12 * sizeof(V4<R>) + 8 * sizeof(R) + sizeof(int2)) +
-         (size_t)(cb + 2) * 6 * sizeof(V4<R>) + (size_t)co * 4 + (size_t)cl * 16;
-}
+// Everything a sweep touches lies in LDS, staged once per solve: the group's
+// bodies (one record each, slot nb the zero record of fixed bodies, slot nb + 1
+// the discard record), one record per contact, and a schedule.  A sweep issues
+// no global memory access.
+//
+// A contact's record: row r of J at r * ROW as (lin_r, b_r | angA_r, r0_r |
+// angB_r, mu_r), both iterates, and the LDS offsets of its bodies' records: A
+// and B to read, A and B to write (a fixed body is written to the discard
+// record).  Under the isotropic projection every row's mu_r is mu_1, the only
+// one it reads.  Record nc is the null contact (zero rows and iterates, both
+// bodies fixed), which changes nothing.
+//
+// The schedule lists, phase by phase, the record of each quad's contact (in
+// units of 16 bytes; the null contact where a quad has none).  A phase is at
+// most 16 contacts of one colour, so a wavefront needs no test of positions
+// against colour ends, no loop over a wide colour, and no branch.
+template <typename R> struct Rec {
+  static constexpr int ROW = 12 * (int)sizeof(R);
+  static constexpr int X0 = 4 * ROW, X1 = X0 + 4 * (int)sizeof(R), LOC = X1 + 4 * (int)sizeof(R);
+  static constexpr int BYTES = (LOC + 16 + 4 * (int)sizeof(R) - 1) / (4 * (int)sizeof(R)) * (4 * (int)sizeof(R));
+};
 
 constexpr int RES_LANES = 64;   // lanes of a resident group
+constexpr int PHASE_Q = 16;     // quads of a wavefront: contacts per phase
+constexpr int PHASE_B = 2 * PHASE_Q;   // bytes of one phase of the schedule
+constexpr int PHASE_PAD = 4;    // phases read past a lane's last one
 
-// LDS capacities of the resident layout (compile-time, so array offsets fold
-// into the LDS instructions); Dev::res_cap_c/b may set lower fit limits.
-// H = 1: the half layout (FP32 ~68 KB), so that two solve workgroups share a
-// CU when a batch has more scenes than the device has CUs.
+// LDS of a solve workgroup and the most contacts and bodies a tuning may ask
+// for.  H = 1: the half layout, so that two solve workgroups share a CU when a
+// batch has more scenes than the device has CUs.
 template <typename R, int H = 0> struct ResCap {
-  static constexpr int C = (sizeof(R) == 4 ? 384 : 192) >> H;   // contacts
-  static constexpr int B = C;                             // bodies
-  static constexpr int O = 4 * C;                         // colour offsets (nc + 3 per lane)
-  static constexpr size_t BYTES = res_lds_bytes<R>(C, B, O, RES_LANES);
+  static constexpr int C = (sizeof(R) == 4 ? 384 : 192) >> H;   // contacts: limit of rbh_tuning.resident_contacts
+  static constexpr int B = C;                                   // bodies: limit of rbh_tuning.resident_bodies
+  static constexpr size_t LDS = (size_t)(H ? 80 : 160) * 1024 - 512;   // dynamic LDS of the launch
+  static constexpr size_t BYTES = LDS - 128;                            // of it for the layouts (solve_scratch has the rest)
   // the streaming layout keeps only bodies (and the zero and discard slots) in the same LDS
   static constexpr int VB = (int)(BYTES / (6 * sizeof(V4<R>))) - 2;
 };
 
-template <typename R, int H = 0> struct ResLds {
-  V4<R> *JL, *JA, *JB;                     // per contact row (4 per contact)
-  R *x0, *x1;                              // per contact row
-  BodyLds<R> B;                            // per body (slot - b_lo), zero slot zs, discard slot ts
-  int2* loc;                               // a contact's two bodies (slot - b_lo; zs: fixed)
-  int4* lt;                                // per lane: first contact, K, colours, first colour offset
-  int* coff;
-  static constexpr int zs = ResCap<R, H>::B;
-  static constexpr int ts = ResCap<R, H>::B + 1;
-  static constexpr int zsb = zs * rec_bytes<R>(), tsb = ts * rec_bytes<R>();   // their records' byte offsets
-  static constexpr int nul = ResCap<R, H>::C;
-  __device__ explicit ResLds(unsigned char* p) {
-    constexpr int cc = ResCap<R, H>::C + 1, nbs = ResCap<R, H>::B + 2;
-    V4<R>* v = reinterpret_cast<V4<R>*>(p);
-    JL = v; JA = JL + 4 * cc; JB = JA + 4 * cc;
-    B.at(JB + 4 * cc);
-    x0 = reinterpret_cast<R*>(JB + 4 * cc + BODY_REC * nbs); x1 = x0 + 4 * cc;
-    loc = reinterpret_cast<int2*>(x1 + 4 * cc);
-    lt = reinterpret_cast<int4*>(loc + cc);
-    coff = reinterpret_cast<int*>(lt + RES_LANES);
+// LDS addresses of a group of nb bodies, nc contacts, nl lanes (plain 32-bit
+// addresses: an access costs no address arithmetic beyond its own offset)
+template <typename T> using LdsPtr = __attribute__((address_space(3))) T*;
+template <typename R> struct ResLds {
+  int body;            // first body record
+  int zsb, tsb;        // records of the zero and the discard slot
+  int rec, nul;        // first contact record, the null contact's
+  int lt, sched;       // lane table (int4: first record, contacts, first phase, phases), schedule
+  __device__ ResLds(unsigned char* p, int nb, int nc, int nl) {
+    body = (int)(unsigned)(size_t)(LdsPtr<unsigned char>)p;
+    zsb = body + nb * rec_bytes<R>();
+    tsb = zsb + rec_bytes<R>();
+    rec = tsb + rec_bytes<R>();
+    nul = rec + nc * Rec<R>::BYTES;
+    lt = nul + Rec<R>::BYTES;
+    sched = lt + nl * (int)sizeof(int4);
   }
+  static constexpr size_t bytes(int nb, int nc, int nl, int nph) {
+    return (size_t)(nb + 2) * rec_bytes<R>() + (size_t)(nc + 1) * Rec<R>::BYTES + (size_t)nl * sizeof(int4) +
+           (size_t)(nph + PHASE_PAD) * PHASE_B;
+  }
+  template <typename T> __device__ __forceinline__ T& at(int addr) const { return *(T*)(LdsPtr<T>)(size_t)(unsigned)addr; }
 };
+static_assert(ResCap<float>::BYTES / 16 < 65536, "a schedule entry addresses LDS in units of 16 bytes");
 
 // ---- streaming layout: bodies in LDS, contact rows and iterates in global memory
 template <typename R, int H = 0> struct StreamLds {
@@ -1971,15 +1983,19 @@ template <typename R, int H = 0> struct StreamLds {
   static constexpr int zs = ResCap<R, H>::VB;
   static constexpr int ts = ResCap<R, H>::VB + 1;
   __device__ explicit StreamLds(unsigned char* p) {
-    constexpr int nbs = ResCap<R, H>::VB + 2;
     V4<R>* v = reinterpret_cast<V4<R>*>(p);
-    (void)nbs;
     B.at(v);
   }
 };
 
+// most phases of a lane of K contacts in nc colours (serial: one contact each):
+// a colour of w > 0 contacts takes ceil(w / 16) <= 1 + (w - 1) / 16
+__device__ __forceinline__ int lane_phases(int K, int nc, bool serial) {
+  return serial ? K : min(K, nc + K / PHASE_Q);
+}
+
 // sizes of a group's resident data (uniform over the workgroup)
-struct GroupSize { int p0, nc, no, nl; };
+struct GroupSize { int p0, nc, nph, nl; };
 
 template <typename R> __device__ GroupSize group_size(const Dev<R>& d, const Group& gr, bool serial) {
   GroupSize g{0x7fffffff, 0, 0, 0};
@@ -1989,7 +2005,7 @@ template <typename R> __device__ GroupSize group_size(const Dev<R>& d, const Gro
     if (e <= a) continue;
     g.p0 = min(g.p0, a);
     p1 = max(p1, e);
-    g.no += serial ? 0 : d.l_ncol[l] + 3;
+    g.nph += lane_phases(e - a, d.l_ncol[l], serial);
     ++g.nl;
   }
   g.nc = g.nl ? p1 - g.p0 : 0;
@@ -1999,73 +2015,151 @@ template <typename R> __device__ GroupSize group_size(const Dev<R>& d, const Gro
 
 template <typename R, int H>
 __device__ __forceinline__ bool group_fits(const Dev<R>& d, const Group& gr, const GroupSize& g) {
-  return g.nc <= min(d.res_cap_c, ResCap<R, H>::C) && gr.b_hi - gr.b_lo <= min(d.res_cap_b, ResCap<R, H>::B) &&
-         g.no <= ResCap<R, H>::O && g.nl <= RES_LANES;
+  const int nb = gr.b_hi - gr.b_lo;
+  // (the first bounds keep the sum below from overflowing)
+  return g.nc <= min(d.res_cap_c, 4096) && nb <= min(d.res_cap_b, 4096) && g.nl <= RES_LANES &&
+         ResLds<R>::bytes(nb, g.nc, g.nl, g.nph) <= ResCap<R, H>::BYTES;
 }
 
-// One sweep of one resident lane by STRIDE threads (a wavefront or the
-// workgroup): STRIDE / 4 contacts per pass.  Colour c spans positions
-// [co[c], co[c + 1]) of the lane (SERIAL: position c alone); the lane's
-// offsets end with two repeats of co[nc], so the colours after the last are
-// empty.  The merit, max |x_new - x_old| in FP64, is taken after the sweep
-// over the lane's rows (a sweep updates each of its contacts once).
-template <typename R, int STRIDE, bool SERIAL, bool JAC, int H>
-__device__ double res_sweep(const ProxParams& pp, ResLds<R, H>& L, int4 lt, bool hybrid, const R* xa, R* xn, R rs,
-                            int tid) {
-  // the lane's table entry is the same for every thread: scalar loop control
-  const int c0 = __builtin_amdgcn_readfirstlane(lt.x), K = __builtin_amdgcn_readfirstlane(lt.y);
-  const int nc = SERIAL ? K : __builtin_amdgcn_readfirstlane(lt.z);
-  const int* co = L.coff + __builtin_amdgcn_readfirstlane(lt.w);
-  const int q = tid & 3, j = tid >> 2;
-  constexpr int PER = STRIDE / 4;
-  if (nc <= 0) return 0.0;
-  // end of colour c (a load; made scalar where it is used)
-  auto col_end = [&](int c) { return SERIAL ? min(c + 1, K) : co[c + 1]; };
-  // contact at position pos of a colour ending at end, or the null contact
-  auto pick = [&](int pos, int end) { return pos < end ? c0 + pos : ResLds<R, H>::nul; };
-  // rows, iterate and body slots of contact i (none of them change during a sweep)
-  auto load = [&](int i, QuadRow<R>& it) {
-    it.jl = L.JL[4 * i + q]; it.ja = L.JA[4 * i + q]; it.jb = L.JB[4 * i + q];
-    it.xo = xa[4 * i + q];
-    it.lc = L.loc[i];
+// What a quad's lane needs of its next contact: row q of J, rows 0..3 of the
+// block it updates, that body's inverse mass, the old iterate, and LDS offsets.
+// None of it changes during a sweep, so it is read a phase ahead.
+template <typename R> struct PhaseIn {
+  V4<R> jl, ja, jb, W0, W1;
+  V3<R> v0, v1, v2, v3;
+  R xo;
+  int oA, oB;      // the two bodies' records
+  int own, wr;     // the velocity block this lane updates: where it is read, where it is written
+  int xw;          // the new iterate
+};
+
+// One sweep of one resident lane by one wavefront: nph phases of up to 16
+// contacts, one per quad, lane q of a quad holding row q (the arithmetic and
+// its order are those of update_contact, so the iterates are bitwise the
+// same).  ISO: the isotropic projection.  JAC: Jacobi reads the accepted
+// velocity changes (jacobi_solver.py:6-57), Gauss-Seidel the working ones.
+//
+// A phase is a serial chain: velocities from LDS, the row products, the
+// projection, the velocity update, back to LDS.  With one wavefront per SIMD
+// nothing else hides its latency (measured here: 8 cycles per dependent
+// vector instruction against 4.5 per independent one, 100 per LDS round trip,
+// 33 per saveexec and branch), so:
+//  * everything but the velocities is read one phase ahead, the bodies'
+//    offsets two ahead and the schedule three ahead;
+//  * the projection and the choice between the linear and the angular block
+//    are selects, not branches;
+//  * a row keeps its own projected value: it needs the others' only through
+//    the sum of their squares;
+//  * the sign of the update (body A minus, body B plus) is applied once, at
+//    the end, and a linear update runs through the same multiply-add as an
+//    angular one (times 1/m instead of times one).
+// A phase is then ~118 instructions and ~570 cycles (0.24 us), bound by their
+// issue; with the branches, the position tests and a wait for the previous
+// phase's writes it took ~1,050.  4,096 spheres, 60 colours, 50 sweeps:
+// solve 1613 -> 875 us.
+template <typename R, bool ISO, bool JAC>
+__device__ double res_sweep(const ProxParams& pp, const ResLds<R>& L, int4 lt, bool hybrid, int acc, R rs, int lane) {
+  using X = Rec<R>;
+  constexpr int VB = (int)sizeof(V4<R>), FV = JAC ? F_SL * VB : F_WL * VB;
+  const int rec0 = __builtin_amdgcn_readfirstlane(lt.x), K = __builtin_amdgcn_readfirstlane(lt.y);
+  const int nph = __builtin_amdgcn_readfirstlane(lt.w);
+  const int q = lane & 3;
+  const bool side_b = q >= 2, ang = q & 1;   // lane 0: linear A, 1: angular A, 2: linear B, 3: angular B
+  const int row = q * X::ROW, blk = ang ? (side_b ? 2 * VB : VB) : 0, fo = ang ? VB : 0;
+  const int xa = (acc ? X::X1 : X::X0), xn = (acc ? X::X0 : X::X1);
+  const int xro = xa + q * (int)sizeof(R), xwo = xn + q * (int)sizeof(R);
+  const R sgn = side_b ? R(1) : R(-1);
+  if (nph <= 0) return 0.0;
+  int sp = L.sched + __builtin_amdgcn_readfirstlane(lt.z) * PHASE_B + 2 * (lane >> 2);
+  auto entry = [&](int ahead) { return (int)L.template at<unsigned short>(sp + ahead * PHASE_B) * 16; };
+  auto load = [&](int r, const int4& lc, PhaseIn<R>& p) {
+    const int rr = r + row, rb = r + blk;
+    p.jl = L.template at<V4<R>>(rr);
+    p.ja = L.template at<V4<R>>(rr + VB);
+    p.jb = L.template at<V4<R>>(rr + 2 * VB);
+    p.xo = L.template at<R>(r + xro);
+    p.v0 = xyz(L.template at<V4<R>>(rb));
+    p.v1 = xyz(L.template at<V4<R>>(rb + X::ROW));
+    p.v2 = xyz(L.template at<V4<R>>(rb + 2 * X::ROW));
+    p.v3 = xyz(L.template at<V4<R>>(rb + 3 * X::ROW));
+    const int own = side_b ? lc.y : lc.x;
+    p.W0 = L.template at<V4<R>>(own + F_W0 * VB);
+    p.W1 = L.template at<V4<R>>(own + F_W1 * VB);
+    p.oA = lc.x;
+    p.oB = lc.y;
+    p.own = own + fo;
+    p.wr = (side_b ? lc.w : lc.z) + fo;
+    p.xw = r + xwo;
   };
-  // Phase c knows where colours c and c + 1 end.  Behind its velocity loads
-  // it reads this quad's first contact of colour c + 1 and where colour c + 2
-  // ends, so a phase waits on one LDS round trip, not two or three.  The two
-  // row buffers take turns, so nothing is copied between phases.
-  int lo = SERIAL ? 0 : __builtin_amdgcn_readfirstlane(co[0]);
-  int hi = __builtin_amdgcn_readfirstlane(col_end(0)), hn = __builtin_amdgcn_readfirstlane(col_end(1)), c = 0;
-  QuadRow<R> ra, rb;
-  load(pick(lo + j, hi), ra);
-  auto phase = [&](const QuadRow<R>& cur, QuadRow<R>& nxt) {
-    const int i0 = pick(lo + j, hi);
-    int h2 = 0;
-    R xq;
-    quad_core<R, JAC>(pp, cur, q, rs, hybrid, L.B, L.zsb, L.tsb, L.JL, L.JA, L.JB, 4 * (size_t)i0, xq, [&] {
-      load(pick(hi + j, hn), nxt);
-      h2 = col_end(c + 2);
-    });
-    xn[4 * i0 + q] = xq;
-    // further contacts of this quad in the colour (a colour wider than the quads)
-    for (int pos = lo + j + PER; pos < hi; pos += PER) {
-      const int i = c0 + pos;
-      QuadRow<R> it;
-      load(i, it);
-      quad_core<R, JAC>(pp, it, q, rs, hybrid, L.B, L.zsb, L.tsb, L.JL, L.JA, L.JB, 4 * (size_t)i, xq, [] {});
-      xn[4 * i + q] = xq;
-    }
-    phase_sync<STRIDE>();
-    lo = hi; hi = hn; hn = __builtin_amdgcn_readfirstlane(h2); ++c;
-  };
-  while (true) {
-    phase(ra, rb);
-    if (c >= nc) break;
-    phase(rb, ra);
-    if (c >= nc) break;
+  int r1 = entry(1), e2 = entry(2);
+  PhaseIn<R> pa, pb;
+  int4 lc1;
+  {
+    const int r0 = entry(0);
+    const int4 lc0 = L.template at<int4>(r0 + X::LOC);
+    lc1 = L.template at<int4>(r1 + X::LOC);
+    load(r0, lc0, pa);
   }
+  // the reads above are done when the loop starts: a wait inside it would
+  // also wait for the previous phase's writes
+  __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0)
+  auto phase = [&](const PhaseIn<R>& c, PhaseIn<R>& n) {
+    const V4<R> lA = L.template at<V4<R>>(c.oA + FV), aA = L.template at<V4<R>>(c.oA + FV + VB);
+    const V4<R> lB = L.template at<V4<R>>(c.oB + FV), aB = L.template at<V4<R>>(c.oB + FV + VB);
+    const V4<R> old = L.template at<V4<R>>(c.own + F_WL * VB);
+    load(r1, lc1, n);
+    const int r2 = e2;
+    lc1 = L.template at<int4>(r2 + X::LOC);
+    e2 = entry(3);
+    r1 = r2;
+    sp += PHASE_B;
+    // row q of z = x - r (J w + b)  (contacts.py:77-92)
+    const R Jw = row_jw(xyz(c.jl), xyz(c.ja), xyz(c.jb), xyz(lA), xyz(aA), xyz(lB), xyz(aB));
+    const R z = row_z(c.xo, c.ja.w * rs, Jw, c.jl.w);
+    // projections (contacts.py:92-95)
+    const R z0 = fmax(R(0), z);
+    const R xnrm = quad_bcast<0>(z0);
+    R val;
+    if constexpr (ISO) {
+      const R xr = (JAC && !hybrid) ? quad_bcast<0>(c.xo) : xnrm;
+      const R zz = z * z;
+      const R sq = (quad_bcast<1>(zz) + quad_bcast<2>(zz)) + quad_bcast<3>(zz);
+      val = prox_sphere_row<R>(z, sq, c.jb.w, xr);
+    } else {
+      const R xr = (JAC && !hybrid) ? quad_bcast<0>(c.xo) : xnrm;
+      const R z1 = quad_bcast<1>(z), z2 = quad_bcast<2>(z), z3 = quad_bcast<3>(z);
+      const R mu0 = quad_bcast<1>(c.jb.w), mu1 = quad_bcast<2>(c.jb.w), mu2 = quad_bcast<3>(c.jb.w);
+      const V3<R> o = prox_ellipsoid_call<R>(z1, z2, z3, mu0, mu1, mu2, xr, pp.ell_tol, pp.ell_expansion, pp.ell_max_iter);
+      val = side_b ? (ang ? o.z : o.y) : o.x;
+    }
+    const R xq = q == 0 ? z0 : val;
+    const R dq = xq - c.xo;
+    // w += W J^T dx (contacts.py:107), this lane's block
+    const R d0 = quad_bcast<0>(dq), d1 = quad_bcast<1>(dq), d2 = quad_bcast<2>(dq), d3 = quad_bcast<3>(dq);
+    V3<R> a = {sum_first(d0 * c.v0.x), sum_first(d0 * c.v0.y), sum_first(d0 * c.v0.z)};
+    a.x = madd(d1, c.v1.x, a.x); a.y = madd(d1, c.v1.y, a.y); a.z = madd(d1, c.v1.z, a.z);
+    a.x = madd(d2, c.v2.x, a.x); a.y = madd(d2, c.v2.y, a.y); a.z = madd(d2, c.v2.z, a.z);
+    a.x = madd(d3, c.v3.x, a.x); a.y = madd(d3, c.v3.y, a.y); a.z = madd(d3, c.v3.z, a.z);
+    const R W[6] = {c.W0.x, c.W0.y, c.W0.z, c.W0.w, c.W1.x, c.W1.y};
+    const V3<R> t = sym_madd(W, a);
+    const R s = ang ? sgn : sgn * c.W1.z;
+    const V3<R> u = {ang ? t.x : a.x, ang ? t.y : a.y, ang ? t.z : a.z};
+    L.template at<V4<R>>(c.wr + F_WL * VB) = V4<R>{madd(s, u.x, old.x), madd(s, u.y, old.y), madd(s, u.z, old.z), R(0)};
+    L.template at<R>(c.xw) = xq;
+    phase_sync<64>();
+  };
+  for (int p = 0;;) {
+    phase(pa, pb);
+    if (++p >= nph) break;
+    phase(pb, pa);
+    if (++p >= nph) break;
+  }
+  // the merit, max |x_new - x_old| in FP64 (a sweep updates each contact once)
   double m = 0.0;
-  for (int r = tid; r < 4 * K; r += STRIDE)
-    m = fmax(m, fabs((double)xn[4 * c0 + r] - (double)xa[4 * c0 + r]));
+  for (int i = lane >> 2; i < K; i += PHASE_Q) {
+    const int r = rec0 + i * X::BYTES;
+    m = fmax(m, fabs((double)L.template at<R>(r + xwo) - (double)L.template at<R>(r + xro)));
+  }
   return m;
 }
 
@@ -2125,93 +2219,123 @@ __device__ void finish_group(const Dev<R>& d, SceneState& st, const SolveCtl& ct
 template <typename R, bool COOP, int NT, int H>
 __device__ void solve_group_resident(const Dev<R>& d, const int slot, const Group& gr, const GroupSize& gs,
                                      unsigned char* smem, double* sh_red, int* s_ok) {
+  using X = Rec<R>;
+  constexpr int VB = (int)sizeof(V4<R>);
   const SceneParams& sp = d.sp[slot];
   SceneState& st = d.ss[slot];
   const bool serial = sp.scheme == SCHEME_GS;
   const bool jacobi = sp.scheme == SCHEME_JACOBI || sp.scheme == SCHEME_JACOBI_HYBRID;
   const bool hybrid = sp.scheme == SCHEME_JACOBI_HYBRID;
   const ProxParams pp(sp);
-  ResLds<R, H> L(smem);
+  const bool iso = pp.friction != 1;
   const int b0 = gr.b_lo, nb = gr.b_hi - gr.b_lo;
-  // stage: lane table, colour offsets, contact rows and iterates, bodies
+  const ResLds<R> L(smem, nb, gs.nc, gs.nl);
+  BodyLds<R> B;
+  B.at(reinterpret_cast<V4<R>*>(smem));
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, nwave = blockDim.x >> 6;
+  // stage: lane table (fourth entry: the sweep lane, until its schedule is written), an empty schedule,
+  // contact records, bodies
   if (threadIdx.x == 0) {
     int t = 0, o = 0;
     for (int l = gr.l_lo; l < gr.l_hi; ++l) {
       const int a = d.l_start[l], e = d.l_end[l];
       if (e <= a) continue;
-      const int nc = serial ? 0 : d.l_ncol[l];
-      L.lt[t++] = make_int4(a - gs.p0, e - a, nc, o);
-      o += serial ? 0 : nc + 3;
+      L.template at<int4>(L.lt + 16 * t++) = make_int4(L.rec + (a - gs.p0) * X::BYTES, e - a, o, l);
+      o += lane_phases(e - a, d.l_ncol[l], serial);
     }
   }
-  __syncthreads();
-  if (!serial) {
-    int t = 0;
-    for (int l = gr.l_lo; l < gr.l_hi; ++l) {
-      if (d.l_end[l] <= d.l_start[l]) continue;
-      const int4 lt = L.lt[t++];
-      const int* src = lane_coff(d, l);
-      // offsets 0..nc, then co[nc] twice: the (empty) colours after the last
-      for (int c = threadIdx.x; c <= lt.z + 2; c += blockDim.x) L.coff[lt.w + c] = src[min(c, lt.z)];
+  for (int i = threadIdx.x; i < (gs.nph + PHASE_PAD) * PHASE_Q; i += blockDim.x)
+    L.template at<unsigned short>(L.sched + 2 * i) = (unsigned short)(L.nul / 16);
+  const V4<R> zero = {R(0), R(0), R(0), R(0)};
+  for (int r = threadIdx.x; r < 4 * (gs.nc + 1); r += blockDim.x) {
+    const int i = r >> 2, q = r & 3;
+    const int rec = L.rec + i * X::BYTES;
+    V4<R> jl = zero, ja = zero, jb = zero;
+    R x0 = R(0), x1 = R(0);
+    int2 lc = make_int2(-1, -1);
+    if (i < gs.nc) {
+      const size_t g = 4 * (size_t)gs.p0 + r;
+      jl = d.s_JL[g]; ja = d.s_JA[g]; jb = d.s_JB[g];
+      if (iso) jb.w = d.s_JB[4 * ((size_t)gs.p0 + i) + 1].w;
+      x0 = d.xr0[g]; x1 = d.xr1[g];
+      lc = d.s_loc[gs.p0 + i];
+    }
+    L.template at<V4<R>>(rec + q * X::ROW) = jl;
+    L.template at<V4<R>>(rec + q * X::ROW + VB) = ja;
+    L.template at<V4<R>>(rec + q * X::ROW + 2 * VB) = jb;
+    L.template at<R>(rec + X::X0 + q * (int)sizeof(R)) = x0;
+    L.template at<R>(rec + X::X1 + q * (int)sizeof(R)) = x1;
+    if (q == 0) {
+      const int a = L.body + (lc.x - b0) * rec_bytes<R>(), b = L.body + (lc.y - b0) * rec_bytes<R>();
+      L.template at<int4>(rec + X::LOC) = make_int4(lc.x >= 0 ? a : L.zsb, lc.y >= 0 ? b : L.zsb,
+                                                    lc.x >= 0 ? a : L.tsb, lc.y >= 0 ? b : L.tsb);
     }
   }
-  for (int r = threadIdx.x; r < 4 * gs.nc; r += blockDim.x) {
-    const size_t g = 4 * (size_t)gs.p0 + r;
-    L.JL[r] = d.s_JL[g]; L.JA[r] = d.s_JA[g]; L.JB[r] = d.s_JB[g];
-    L.x0[r] = d.xr0[g]; L.x1[r] = d.xr1[g];
-  }
-  for (int i = threadIdx.x; i < gs.nc; i += blockDim.x) {
-    const int2 lc = d.s_loc[gs.p0 + i];
-    L.loc[i] = make_int2((lc.x >= 0 ? lc.x - b0 : L.zs) * rec_bytes<R>(), (lc.y >= 0 ? lc.y - b0 : L.zs) * rec_bytes<R>());
-  }
-  // the null contact: zero rows and iterates, both bodies fixed
-  if (threadIdx.x < 4) {
-    const V4<R> z = {R(0), R(0), R(0), R(0)};
-    const int r = 4 * ResLds<R, H>::nul + threadIdx.x;
-    L.JL[r] = z; L.JA[r] = z; L.JB[r] = z;
-    L.x0[r] = R(0); L.x1[r] = R(0);
-    if (threadIdx.x == 0) L.loc[ResLds<R, H>::nul] = make_int2(L.zsb, L.zsb);
-  }
-  stage_bodies(d, L.B, b0, nb, L.zs);
+  stage_bodies(d, B, b0, nb, nb);
   __syncthreads();
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, nwave = blockDim.x >> 6;
+  // schedules: a wavefront per lane, its colours 64 at a time
+  for (int t = wave; t < gs.nl; t += nwave) {
+    const int4 lt = L.template at<int4>(L.lt + 16 * t);
+    const int nc = serial ? lt.y : d.l_ncol[lt.w];
+    const int* co = lane_coff(d, lt.w);
+    int ph = lt.z;
+    for (int c0 = 0; c0 < nc; c0 += 64) {
+      const int c = c0 + lane;
+      int lo = 0, w = 0;
+      if (c < nc) {
+        lo = serial ? c : co[c];
+        w = serial ? 1 : co[c + 1] - lo;
+      }
+      const int np = (w + PHASE_Q - 1) / PHASE_Q;
+      int inc = np;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const int v = __shfl_up(inc, o, 64);
+        if (lane >= o) inc += v;
+      }
+      const int s0 = L.sched + (ph + inc - np) * PHASE_B;
+      for (int i = 0; i < w; ++i)   // (slots of one phase are consecutive, and so are its phases)
+        L.template at<unsigned short>(s0 + 2 * i) = (unsigned short)((lt.x + (lo + i) * X::BYTES) / 16);
+      ph += __shfl(inc, 63, 64);
+    }
+    if (lane == 0) L.template at<int>(L.lt + 16 * t + 12) = ph - lt.z;
+  }
+  __syncthreads();
   SolveCtl ctl;
   ctl.iters = sp.max_iter;
   bool abort = false;
   for (int it = 0; it < sp.max_iter; ++it) {
-    const R* xa = ctl.acc ? L.x1 : L.x0;
-    R* xn = ctl.acc ? L.x0 : L.x1;
     const R rs = R(ctl.rscale);
     double m = 0.0;
     for (int t = wave; t < gs.nl; t += nwave) {
-      const int4 lt = L.lt[t];
-      if (lt.y > WAVE_LANE_MAX && !serial) continue;
-      m = fmax(m, serial   ? res_sweep<R, 64, true, false, H>(pp, L, lt, hybrid, xa, xn, rs, lane)
-                  : jacobi ? res_sweep<R, 64, false, true, H>(pp, L, lt, hybrid, xa, xn, rs, lane)
-                           : res_sweep<R, 64, false, false, H>(pp, L, lt, hybrid, xa, xn, rs, lane));
+      const int4 lt = L.template at<int4>(L.lt + 16 * t);
+      double ml;
+      if (jacobi)
+        ml = iso ? res_sweep<R, true, true>(pp, L, lt, hybrid, ctl.acc, rs, lane)
+                 : res_sweep<R, false, true>(pp, L, lt, hybrid, ctl.acc, rs, lane);
+      else
+        ml = iso ? res_sweep<R, true, false>(pp, L, lt, hybrid, ctl.acc, rs, lane)
+                 : res_sweep<R, false, false>(pp, L, lt, hybrid, ctl.acc, rs, lane);
+      m = fmax(m, ml);
     }
-    for (int t = 0; t < gs.nl; ++t) {
-      const int4 lt = L.lt[t];
-      if (lt.y <= WAVE_LANE_MAX || serial) continue;
-      m = fmax(m, jacobi ? res_sweep<R, NT, false, true, H>(pp, L, lt, hybrid, xa, xn, rs, (int)threadIdx.x)
-                         : res_sweep<R, NT, false, false, H>(pp, L, lt, hybrid, xa, xn, rs, (int)threadIdx.x));
-    }
-    const int dec = sweep_decide<R, COOP>(d, sp, ctl, m, it, gr.lead, sh_red, s_ok, L.B, nb, abort);
+    const int dec = sweep_decide<R, COOP>(d, sp, ctl, m, it, gr.lead, sh_red, s_ok, B, nb, abort);
     if (abort) return;
     if (dec & 2) { ctl.iters = it; break; }
   }
   // impulses to contact order; natural-map residual (FP64) with r0; accepted velocity changes out
-  const R* xs = ctl.acc ? L.x1 : L.x0;
   double rloc = 0.0, xmax = 0.0;
   for (int i = threadIdx.x; i < gs.nc; i += blockDim.x) {
-    const int2 lc = L.loc[i];
+    const int rec = L.rec + i * X::BYTES;
+    const int4 lc = L.template at<int4>(rec + X::LOC);
+    const R* xs = &L.template at<R>(rec + (ctl.acc ? X::X1 : X::X0));
+    const V4<R>* rows = &L.template at<V4<R>>(rec);
     V4<R> x;
-    quad_finish_contact(pp, L.JL, L.JA, L.JB, xs, i, L.B.rec(lc.x, F_SL), L.B.rec(lc.x, F_SA), L.B.rec(lc.y, F_SL),
-                        L.B.rec(lc.y, F_SA), x,
-                        rloc, xmax);
+    quad_finish_contact<R, 3>(pp, rows, rows + 1, rows + 2, xs, L.template at<V4<R>>(lc.x + F_SL * VB),
+                              L.template at<V4<R>>(lc.x + F_SA * VB), L.template at<V4<R>>(lc.y + F_SL * VB),
+                              L.template at<V4<R>>(lc.y + F_SA * VB), x, rloc, xmax);
     if (!d.post) d.c_imp[d.perm[gs.p0 + i]] = x;
   }
-  finish_group<R, COOP>(d, st, ctl, gr.lead, L.B, b0, nb, rloc, xmax, sh_red);
+  finish_group<R, COOP>(d, st, ctl, gr.lead, B, b0, nb, rloc, xmax, sh_red);
 }
 
 // One sweep of one lane in the streaming layout: rows and iterates from
@@ -2314,8 +2438,9 @@ __device__ void solve_group_stream(const Dev<R>& d, const int slot, const Group&
       const int2 lc = d.s_loc[i];
       const int sa = lc.x >= 0 ? lc.x - b0 : L.zs, sb = lc.y >= 0 ? lc.y - b0 : L.zs;
       V4<R> x;
-      quad_finish_contact(pp, d.s_JL, d.s_JA, d.s_JB, xs, i, L.B.sl[sa], L.B.sa[sa], L.B.sl[sb], L.B.sa[sb], x,
-                          rloc, xmax);
+      const size_t r = 4 * (size_t)i;
+      quad_finish_contact<R, 1>(pp, d.s_JL + r, d.s_JA + r, d.s_JB + r, xs + r, L.B.sl[sa], L.B.sa[sa], L.B.sl[sb],
+                                L.B.sa[sb], x, rloc, xmax);
       if (!d.post) d.c_imp[d.perm[i]] = x;
     }
   }
@@ -2336,12 +2461,22 @@ __device__ __forceinline__ void solve_dispatch(const Dev<R>& d, int slot, const 
   else solve_group<R, false, COOP, NT>(d, slot, gr, vs, sh_red, s_ok);
 }
 
+// The solve kernels' reduction scratch (at most 8 doubles) and flag, at the end
+// of the dynamic LDS: with no static LDS the layouts start at LDS address 0,
+// so their offsets fold into the LDS instructions.
+template <typename R, int H>
+__device__ __forceinline__ void solve_scratch(unsigned char* smem, double*& red, int*& ok) {
+  red = reinterpret_cast<double*>(smem + ResCap<R, H>::BYTES);
+  ok = reinterpret_cast<int*>(red + 8);
+}
+
 // One workgroup of NT threads (NT / 64 wavefronts, one per sweep lane) per
 // batch scene; H: the LDS layout (0 full, 1 half).
 template <typename R, int NT, int H> __global__ void __launch_bounds__(NT) k_solve(Dev<R> d) {
   extern __shared__ __align__(32) unsigned char solve_smem[];
-  __shared__ double sh_red[NT / 64];
-  __shared__ int s_ok;
+  double* sh_red;
+  int* s_ok;
+  solve_scratch<R, H>(solve_smem, sh_red, s_ok);
   if (aborted(d.err)) return;
   const int bs = d.bs_order[blockIdx.x];
   const int slot = d.bs_slot[bs];
@@ -2356,15 +2491,16 @@ template <typename R, int NT, int H> __global__ void __launch_bounds__(NT) k_sol
   }
   const int u0 = d.u_base[bs], u1 = u0 + d.u_cnt[bs];
   const Group gr{d.l_base[bs], d.l_base[bs] + d.l_cnt[bs], d.u_boff[u0], d.u_boff[u1], true};
-  solve_dispatch<R, false, NT, H>(d, slot, gr, solve_smem, sh_red, &s_ok);
+  solve_dispatch<R, false, NT, H>(d, slot, gr, solve_smem, sh_red, s_ok);
 }
 
 // A single scene (its lanes are its colouring units): the lanes split into
 // gridDim.x contiguous blocks, one per workgroup of a cooperative launch.
 template <typename R> __global__ void __launch_bounds__(SOLVE_BLOCK) k_solve_multi(Dev<R> d) {
   extern __shared__ __align__(32) unsigned char solve_smem[];
-  __shared__ double sh_red[SOLVE_BLOCK / 64];
-  __shared__ int s_ok;
+  double* sh_red;
+  int* s_ok;
+  solve_scratch<R, 0>(solve_smem, sh_red, s_ok);
   if (aborted(d.err)) return;   // uniform: the flag is set before this launch or not at all
   const int slot = d.bs_slot[0];
   const SceneParams& sp = d.sp[slot];
@@ -2380,5 +2516,5 @@ template <typename R> __global__ void __launch_bounds__(SOLVE_BLOCK) k_solve_mul
   const long long nl = *d.n_lanes, G = gridDim.x;
   const int l_lo = (int)(blockIdx.x * nl / G), l_hi = (int)((blockIdx.x + 1) * nl / G);
   const Group gr{l_lo, l_hi, d.u_boff[l_lo], d.u_boff[l_hi], blockIdx.x == 0};
-  solve_dispatch<R, true, SOLVE_BLOCK, 0>(d, slot, gr, solve_smem, sh_red, &s_ok);
+  solve_dispatch<R, true, SOLVE_BLOCK, 0>(d, slot, gr, solve_smem, sh_red, s_ok);
 }

@@ -1,0 +1,85 @@
+"""GPU: the contact solve at the edges of its schedules.
+
+A phase of a sweep is at most 16 contacts of one colour (one per quad of a
+wavefront), so colours of 15, 16, 17 and 33 contacts sit on its edges; n boxes
+apart on the ground, all in one sweep lane, give colours of n contacts.  The
+FP64 build must match the FP64 oracle within the bounds of test_gpu_parity, and
+in FP32 every layout of the solve must give bitwise the same impulses.
+"""
+import numpy as np
+import pytest
+
+import oracle.scene as OS
+import oracle.stepper as OST
+from rainbow_amd import api as API
+from rainbow_amd import math3 as Q
+from rainbow_amd import mesh as MESH
+from rainbow_amd import native, scenes
+from rainbow_amd.stepper import engine_desc, gather_state
+from test_gpu_parity import assert_fp64_parity
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def bank():
+    return scenes.ShapeBank(resolution=32)
+
+
+def row_of_boxes(bank, n, params):
+    """n unit boxes, 3 apart, 0.05 into the ground and a little tilted."""
+    eng = scenes.new_engine(bank, params)
+    scenes.set_friction(eng, 0.5)
+    API.create_gravity_force(eng, "gravity", 9.81, np.array([0.0, 1.0, 0.0]))
+    scenes.add_ground(eng, bank)
+    box = bank.get("box_shape", lambda: MESH.create_box(1.0, 1.0, 1.0))
+    for i in range(n):
+        scenes.add_body(eng, "b%d" % i, box, np.array([3.0 * (i % 8) - 12.0, 0.45, 3.0 * (i // 8) - 9.0]),
+                        q=Q.Rz(0.01 * (i % 5)), v=np.array([0.1, -0.2, 0.02 * i]))
+    return eng
+
+
+def step_with(eng, tuning, flags, precision, steps=1):
+    """(contacts, state, log) after `steps` steps of a fresh context."""
+    ctx = native.Context(0, precision)
+    try:
+        ctx.set_tuning(**tuning)
+        desc, keep = engine_desc(eng, ctx)
+        sid = ctx.scene_create(desc)
+        ctx.set_state(sid, *gather_state(list(eng.bodies.values())))
+        ctx.step([sid], steps, 0.01, flags)
+        return ctx.get_contacts(sid), ctx.get_state(sid, len(eng.bodies)), ctx.get_log(sid, eng.params.max_iterations)
+    finally:
+        ctx.close()
+
+
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 33])
+@pytest.mark.parametrize("scheme", ["gauss_seidel", "parallel_gauss_seidel", "parallel_jacobi"])
+@pytest.mark.parametrize("flags", [native.STEP_FORCE_SINGLE, native.STEP_FORCE_MULTI])
+def test_phase_edges_fp64(bank, n, scheme, flags):
+    eng = row_of_boxes(bank, n, dict(precision="fp64", max_iterations=12, proximal_solver=scheme))
+    sc = OS.from_engine(eng)
+    out = OST.step(sc, 0.01)
+    c, state, lg = step_with(eng, dict(unit_size=1024, lanes_per_scene=1), flags, "fp64")
+    assert len(c["ia"]) >= n
+    assert assert_fp64_parity(c, state, lg, out, sc)
+
+
+@pytest.mark.parametrize("n", [1, 16, 17, 33])
+@pytest.mark.parametrize("friction", ["isotropic", "anisotropic"])
+def test_layouts_bitwise_fp32(bank, n, friction):
+    eng = row_of_boxes(bank, n, dict(precision="fp32", max_iterations=20, friction_model=friction))
+    if friction == "anisotropic":
+        eng.surfaces_interactions.storage[("default", "default")].mu = np.array([0.5, 0.3, 0.05])
+    ref = None
+    for tuning in (dict(), dict(unit_size=1024, lanes_per_scene=1), dict(unit_size=32, lanes_per_scene=7),
+                   dict(resident_contacts=64, resident_bodies=64, unit_size=1024, lanes_per_scene=1),
+                   dict(waves_per_group=8), dict(solve_groups_per_cu=2)):
+        for flags in (native.STEP_FORCE_SINGLE, native.STEP_FORCE_MULTI):
+            c, state, lg = step_with(eng, tuning, flags, "fp32", steps=2)
+            got = [c["impulse"], c["color"], lg["residuals"], np.float64(lg["natural_residual"])] + list(state)
+            if ref is None:
+                ref = got
+                assert len(c["ia"]) >= n
+            for a, b in zip(got, ref):
+                assert np.array_equal(a, b), (tuning, flags)
