@@ -629,7 +629,6 @@ int build_batch(rbh_ctx* c, const int* ids, int n) {
   std::vector<int> b2f(std::max(c->bodies.cap, 1), -1);
   long long pairs_all = 0, tri_sum = 0;
   int max_iter = 1;
-  bool serial = false;
   for (int i = 0; i < n; ++i) {
     const SceneHost& s = c->scenes[want[i]];
     bsslot.push_back(want[i]);
@@ -643,7 +642,6 @@ int build_batch(rbh_ctx* c, const int* ids, int n) {
     pairs_all += (long long)s.nbody * (s.nbody - 1) / 2;
     tri_sum += s.ntri;
     max_iter = std::max(max_iter, s.params.max_iterations);
-    serial = serial || s.params.proximal_solver == RBH_SCHEME_GAUSS_SEIDEL;
   }
   bsfoff.push_back((int)bb.size());
   c->nb = (int)bb.size();
@@ -668,7 +666,7 @@ int build_batch(rbh_ctx* c, const int* ids, int n) {
   // one scene: colour small units (islands) and solve them on many
   // workgroups; batches: one workgroup per scene
   c->max_iter_batch = max_iter;
-  c->multi_ok = (n == 1 && !serial);
+  c->multi_ok = n == 1;
   c->unit_T = c->tune.unit_size > 0 ? c->tune.unit_size : 64;
   c->last_units = 0;
   // initial capacities; they grow when a step reports an overflow

@@ -83,3 +83,28 @@ def test_layouts_bitwise_fp32(bank, n, friction):
                 assert len(c["ia"]) >= n
             for a, b in zip(got, ref):
                 assert np.array_equal(a, b), (tuning, flags)
+
+
+@pytest.mark.parametrize("n", [3, 40, 60])
+@pytest.mark.parametrize("scheme", ["gauss_seidel", "parallel_gauss_seidel", "parallel_jacobi_hybrid"])
+def test_sweep_order_bitwise_fp32(bank, n, scheme):
+    """Lanes swept by dependency level (unit_size 32) and lanes too large for the level tables, swept by colour or
+    contact index (unit_size 4096: n = 60 gives ~2,700 contacts in one lane), end in the same impulses and states."""
+    eng = scenes.new_engine(bank, dict(precision="fp32", max_iterations=8, proximal_solver=scheme))
+    scenes.set_friction(eng, 0.3)
+    API.create_gravity_force(eng, "gravity", 9.81, np.array([0.0, 1.0, 0.0]))
+    scenes.add_ground(eng, bank)
+    sphere = bank.get("sphere_shape", lambda: MESH.create_sphere(0.5, 16, 16))
+    rng = np.random.default_rng(n)
+    for i in range(n):   # a layer of spheres sunk into the ground and, some of them, into each other
+        p = np.array([0.72 * (i % 8), 0.46, 0.72 * (i // 8)]) + rng.uniform(-0.05, 0.05, 3) * (1.0, 0.2, 1.0)
+        scenes.add_body(eng, "s%d" % i, sphere, p, q=Q.identity(), v=rng.normal(0.0, 0.2, 3))
+    ref = None
+    for tuning in (dict(unit_size=32), dict(unit_size=4096, lanes_per_scene=1)):
+        for flags in (native.STEP_FORCE_SINGLE, native.STEP_FORCE_MULTI):
+            c, state, lg = step_with(eng, tuning, flags, "fp32", steps=2)
+            got = [c["impulse"], c["color"], lg["residuals"], np.float64(lg["natural_residual"])] + list(state)
+            ref = ref or got
+            for a, b in zip(got, ref):
+                assert np.array_equal(a, b), (tuning, flags)
+    assert len(c["ia"]) > 30 * n
