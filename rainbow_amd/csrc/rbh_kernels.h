@@ -125,10 +125,10 @@ template <typename R> struct Dev {
   int* bc_cnt; int* bc_off; int* bc_fill; int* bc_list;   // flat body -> unit-order positions
   unsigned* pal;                       // PALW words per unit-order position
   int* g_pc; unsigned char* g_done;    // colouring state of units too large for LDS
-  int* col_off;                        // colour offsets of lane l at 2 * (l_start[l] + l)
+  int* col_off;                        // level offsets of lane l at 2 * (l_start[l] + l)
   int* l_pos;                          // per unit-order position p (contact uperm[p]): its position in colour order within its lane
-  int items_nb;                        // a batch scene of more bodies than this solves from the per-contact
-                                       // items (s_n .. s_W, x0, x1); -1: any group may
+  int items_nb;                        // a scene of more bodies in contact than this may solve from the
+                                       // per-contact items (s_n .. s_W, x0, x1); -1: any may
   int* big_list;                       // [0]: count, then the units left to k_color_units
   // a scene solved by several workgroups: per sweep and workgroup, the bits
   // of that workgroup's merit (all ones until it publishes them)
@@ -138,8 +138,10 @@ template <typename R> struct Dev {
   int2* s_loc;                         // body slots (u_blist index) of the two bodies (-1: fixed)
   int res_cap_c, res_cap_b;            // most contacts and bodies of a resident solve group (rbh_tuning)
   V4<R>* s_W;                          // 4 per position: W0, W1 of body A, then of body B (zero if fixed)
-  V4<R>* s_JL; V4<R>* s_JA; V4<R>* s_JB;   // rows 4 pos + r of J: (lin_r, b_r), (angA_r, r0_r), (angB_r, mu_r)
-  R* xr0; R* xr1;                      // iterates by row (4 pos + r), for the row-major sweeps
+  unsigned char* s_rec;                // per position its record (Rec<R>), then the null contact's (at cap_contacts)
+  unsigned* l_phase; int* l_nph;       // per lane, from l_start: its phases (first position, contacts); 2 * their
+                                       // number + 1 if the workgroup sweeps it together
+  int solve_quads;                     // quads of a solve workgroup
   // hinges (constraints/hinges.py): static per hinge, then per-step rows and iterates
   const int4* h_ids;                   // (parent, child) arena bodies, (parent, child) hinge-body slots
   const V4<R>* h_geo;                  // 4 per hinge: arm_p, arm_c, axis_p, axis_c (body frames)

@@ -1103,6 +1103,38 @@ __device__ __forceinline__ void contact_rows(V4<R> n4, V4<R> rA4, V4<R> rB4, Con
 }
 
 // ------------------------------------------------------------ sweep order
+// A contact's record in sweep order (s_rec): row r of J at r * ROW as (lin_r,
+// b_r | angA_r, r0_r | angB_r, mu_r), both iterates, and the LDS addresses of
+// its bodies' records (written by the solve).  mu_1..3 are the friction
+// coefficients; under the isotropic projection every row's mu_r is mu_1, the
+// only one it reads.  The record after the last contact's stays zero: the null
+// contact, which a quad without a contact updates to no effect.
+template <typename R> struct Rec {
+  static constexpr int ROW = 12 * (int)sizeof(R);
+  static constexpr int X0 = 4 * ROW, X1 = X0 + 4 * (int)sizeof(R), LOC = X1 + 4 * (int)sizeof(R);
+  static constexpr int BYTES = (LOC + 16 + 4 * (int)sizeof(R) - 1) / (4 * (int)sizeof(R)) * (4 * (int)sizeof(R));
+};
+static_assert(Rec<float>::BYTES == 240 && Rec<double>::BYTES == 480, "records are whole vec4s");
+// 32-bit offsets reach every record of c contacts and the null one
+template <typename R> __host__ __device__ constexpr bool rec_addressable(int c) {
+  return c < (1 << 24) && ((unsigned long long)c + 1) * Rec<R>::BYTES < (1ull << 32);
+}
+
+constexpr int PHASE_Q = 16;      // quads of a wavefront: contacts per phase of a wavefront's sweep
+constexpr int PHASE_BITS = 8;    // low bits of an entry of l_phase: contacts of the phase (at most 128); the rest: its first position
+// most phases of a lane of K contacts in nc levels: a level of w > 0 contacts
+// takes ceil(w / 16) <= 1 + (w - 1) / 16
+__device__ __forceinline__ int lane_phases(int K, int nc) { return min(K, nc + K / PHASE_Q); }
+
+__device__ __forceinline__ int wave_inclusive_sum(int v) {
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int y = __shfl_up(v, o, 64);
+    if ((int)(threadIdx.x & 63) >= o) v += y;
+  }
+  return v;
+}
+
 // A free body's slot (index into u_blist); -1 for a fixed one.
 template <typename R> __device__ __forceinline__ int body_slot(const Dev<R>& d, int b) {
   if (d.b_fixed[b]) return -1;
@@ -1113,7 +1145,7 @@ template <typename R> __device__ __forceinline__ int body_slot(const Dev<R>& d, 
 // Gather one contact into the solver arrays at position `pos`; s_loc holds
 // the bodies' slots (index into u_blist; -1 for a fixed body).
 // ITEMS: also the per-contact items of the global layout
-template <typename R> __device__ __forceinline__ void gather_contact(const Dev<R>& d, int pos, int k, bool items) {
+template <typename R> __device__ __forceinline__ void gather_contact(const Dev<R>& d, int pos, int k, bool items, bool iso) {
   const V4<R> mu = d.c_mu[k];
   const V4<R> n = d.c_n[k], rA = d.c_rA[k], rB = d.c_rB[k];
   const int A = d.c_ia[k], B = d.c_ib[k];
@@ -1137,18 +1169,22 @@ template <typename R> __device__ __forceinline__ void gather_contact(const Dev<R
     d.x0[pos] = z;
     d.x1[pos] = z;
   }
-  // the rows of J once per step, for the row-major (quad) sweeps
+  // the contact's record, for the quad sweeps
+  using X = Rec<R>;
   ContactRow<R> J;
   contact_rows(V4<R>{n.x, n.y, n.z, R(0)}, rA, rB, J);
   const V4<R> bb = d.c_b[k], r0 = d.c_r0[k];
-  const R bv[4] = {bb.x, bb.y, bb.z, bb.w}, rv[4] = {r0.x, r0.y, r0.z, r0.w}, mv[4] = {R(0), mu.x, mu.y, mu.z};
+  const R bv[4] = {bb.x, bb.y, bb.z, bb.w}, rv[4] = {r0.x, r0.y, r0.z, r0.w};
+  const R mv[4] = {iso ? mu.x : R(0), mu.x, iso ? mu.x : mu.y, iso ? mu.x : mu.z};
+  unsigned char* rec = d.s_rec + (size_t)pos * X::BYTES;
+  V4<R>* row = reinterpret_cast<V4<R>*>(rec);
+  R* x = reinterpret_cast<R*>(rec + X::X0);
   for (int r = 0; r < 4; ++r) {
-    const size_t row = 4 * (size_t)pos + r;
-    d.s_JL[row] = V4<R>{J.lin[r].x, J.lin[r].y, J.lin[r].z, bv[r]};
-    d.s_JA[row] = V4<R>{J.angA[r].x, J.angA[r].y, J.angA[r].z, rv[r]};
-    d.s_JB[row] = V4<R>{J.angB[r].x, J.angB[r].y, J.angB[r].z, mv[r]};
-    d.xr0[row] = R(0);
-    d.xr1[row] = R(0);
+    row[3 * r] = V4<R>{J.lin[r].x, J.lin[r].y, J.lin[r].z, bv[r]};
+    row[3 * r + 1] = V4<R>{J.angA[r].x, J.angA[r].y, J.angA[r].z, rv[r]};
+    row[3 * r + 2] = V4<R>{J.angB[r].x, J.angB[r].y, J.angB[r].z, mv[r]};
+    x[r] = R(0);
+    x[4 + r] = R(0);
   }
 }
 
@@ -1177,15 +1213,14 @@ template <typename R> __global__ void k_post_rows(Dev<R> d) {
     d.s_n[pos] = n; d.s_rA[pos] = ra; d.s_rB[pos] = rb;
     d.x0[pos] = V4<R>{zero, zero, zero, zero};
     d.x1[pos] = V4<R>{zero, zero, zero, zero};
+    unsigned char* rec = d.s_rec + (size_t)pos * Rec<R>::BYTES;
+    V4<R>* row = reinterpret_cast<V4<R>*>(rec);
+    R* x = reinterpret_cast<R*>(rec + Rec<R>::X0);
     for (int r = 0; r < 4; ++r) {
-      const size_t row = 4 * (size_t)pos + r;
-      V4<R> jl = d.s_JL[row], jb = d.s_JB[row];
-      jl.w = (r == 0 && deep) ? g : zero;
-      jb.w = zero;
-      d.s_JL[row] = jl;
-      d.s_JB[row] = jb;
-      d.xr0[row] = zero;
-      d.xr1[row] = zero;
+      row[3 * r].w = (r == 0 && deep) ? g : zero;
+      row[3 * r + 2].w = zero;
+      x[r] = zero;
+      x[4 + r] = zero;
     }
     if (deep) d.ss[slot].post_active = 1;
   }
@@ -1239,17 +1274,38 @@ __device__ __forceinline__ void order_scan(OrderLds& s, int n, int* coff) {
     for (int c0 = 0; c0 < n; c0 += 64) {
       const int c = c0 + (int)threadIdx.x;
       const int v = c < n ? s.cnt[c] : 0;
-      int x = v;
-#pragma unroll
-      for (int o = 1; o < 64; o <<= 1) {
-        const int y = __shfl_up(x, o, 64);
-        if ((int)threadIdx.x >= o) x += y;
-      }
+      const int x = wave_inclusive_sum(v);
       if (c < n) { coff[c] = acc + x - v; s.cnt[c] = acc + x - v; }
       acc += __shfl(x, 63, 64);
     }
     if (threadIdx.x == 0) coff[n] = acc;
   }
+}
+
+// The lane's phases for the streaming sweep, by wavefront 0: at most 16 contacts
+// of one level for a wavefront's sweep, a contact per quad of the workgroup for
+// the workgroup's.  One wavefront takes about nl / 2 + K / 16 phases, the
+// workgroup nl / 2 + K / 64 of about 1.4 times the length (its barrier), but
+// only one lane at a time: worth it from levels of 8 contacts on when the group
+// has one lane, and 8 times as many as wavefronts it would leave idle.
+template <typename R>
+__device__ __forceinline__ void order_phases(const Dev<R>& d, int l, int nl, const int* coff) {
+  if (threadIdx.x >= 64) return;
+  const int p0 = d.l_start[l], K = d.l_end[l] - p0, lane = (int)threadIdx.x;
+  const int lanes = d.unit_split > 0 ? min(d.l_cnt[d.l_bs[l]], d.solve_quads / PHASE_Q) : 1;
+  const bool wg = K > 8 * lanes * nl;
+  const int per = wg ? d.solve_quads : PHASE_Q;
+  int ph = 0;
+  for (int c0 = 0; c0 < nl; c0 += 64) {
+    const int c = c0 + lane;
+    const int lo = c < nl ? coff[c] : 0, w = c < nl ? coff[c + 1] - lo : 0;
+    const int np = (w + per - 1) / per;
+    const int inc = wave_inclusive_sum(np);
+    unsigned* out = d.l_phase + p0 + ph + inc - np;
+    for (int i = 0; i < np; ++i) out[i] = (unsigned)(lo + i * per) << PHASE_BITS | (unsigned)min(per, w - i * per);
+    ph += __shfl(inc, 63, 64);
+  }
+  if (lane == 0) d.l_nph[l] = ph << 1 | (wg ? 1 : 0);
 }
 
 // One workgroup per sweep lane: its positions [l_start, l_end) in sweep order.
@@ -1317,6 +1373,9 @@ template <typename R> __device__ __forceinline__ void order_lane(const Dev<R>& d
   }
   if (!levels) {
     if (threadIdx.x == 0) { coff[nc] = K; d.l_ncol[l] = nc; }
+    __threadfence_block();
+    __syncthreads();
+    order_phases(d, l, nc, coff);
     return;
   }
   for (int i = threadIdx.x; i <= (int)ORD_FIXED; i += COLOR_BLOCK) s.last[i] = 0;
@@ -1357,7 +1416,9 @@ template <typename R> __device__ __forceinline__ void order_lane(const Dev<R>& d
   __syncthreads();
   order_scan(s, nl, coff);
   if (threadIdx.x == 0) d.l_ncol[l] = nl;
+  __threadfence_block();
   __syncthreads();
+  order_phases(d, l, nl, coff);
   // each contact's position, taken from LDS counters (the order inside a level
   // changes no result)
   for (int q = threadIdx.x; q < K; q += COLOR_BLOCK) d.l_pos[p0 + s.ord[q]] = atomicAdd(&s.cnt[s.lev[q] - 1], 1);
@@ -1386,19 +1447,22 @@ template <typename R> __device__ void gather_lane(const Dev<R>& d, int l) {
   // the items only where the global layout may read them: a group too large
   // for the velocity-only layout, or the post-stabilisation rows
   const int bs = d.l_bs[l];
+  const bool iso = d.sp[d.bs_slot[bs]].friction != 1;
   bool items = d.items_nb < 0 || d.sp[d.bs_slot[bs]].use_post_stab;
   if (!items) {
     const int u0 = d.u_base[bs];
     items = d.u_boff[u0 + d.u_cnt[bs]] - d.u_boff[u0] > d.items_nb;
   }
   for (int i = blockIdx.y * COLOR_BLOCK + threadIdx.x; i < p1 - p0; i += GATHER_SPLIT * COLOR_BLOCK) {
-    gather_contact(d, p0 + d.l_pos[p0 + i], d.uperm[p0 + i], items);
+    gather_contact(d, p0 + d.l_pos[p0 + i], d.uperm[p0 + i], items, iso);
   }
 }
 
 template <typename R> __global__ void __launch_bounds__(COLOR_BLOCK) k_lane_gather(Dev<R> d) {
   if (aborted(d.err)) return;
   const int nl = *d.n_lanes;
+  if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x < Rec<R>::BYTES / 16)   // the null contact's record
+    reinterpret_cast<int4*>(d.s_rec + (size_t)d.cap_contacts * Rec<R>::BYTES)[threadIdx.x] = make_int4(0, 0, 0, 0);
   for (int l = blockIdx.x; l < nl; l += gridDim.x) gather_lane(d, l);
 }
 
@@ -1408,26 +1472,16 @@ template <typename R> __global__ void __launch_bounds__(COLOR_BLOCK) k_lane_gath
 // scene-wide merit then meets in a grid barrier once per sweep).  A group's
 // bodies are the slot range [b_lo, b_hi) of u_blist.  Three layouts, chosen
 // per group:
-//  * resident: everything a sweep touches -- contact rows, both iterates,
-//    colour offsets, the bodies' velocity changes and inverse masses -- is
-//    staged in LDS once per solve; each wavefront sweeps its own lanes colour
-//    by colour with wavefront-level syncs, and a sweep issues no global
-//    memory access;
-//  * velocity-only: the bodies' velocity changes in LDS, contact rows read
-//    from global memory with the next colour's rows prefetched;
+//  * resident: everything a sweep touches -- contact records, the lanes'
+//    schedules, the bodies' velocity changes and inverse masses -- is staged
+//    in LDS once per solve; each wavefront sweeps its own lanes level by level
+//    with wavefront-level syncs, and a sweep issues no global memory access;
+//  * streaming: the bodies in LDS, contact records read from global memory two
+//    phases ahead; a lane with wide levels is swept by the whole workgroup;
 //  * global: everything in global memory, lanes swept by the whole workgroup.
-// Lanes larger than WAVE_LANE_MAX contacts are swept by the whole workgroup.
 // The sweep order inside an island is the same in every layout and schedule,
 // so all of them give bitwise the same iterates.
 constexpr int SOLVE_BLOCK = 256;
-constexpr int WAVE_LANE_MAX = 512;
-constexpr int SOLVE_LDS_BYTES = 65536 - 512;
-
-// bodies whose velocity changes fit the velocity-only layout
-template <typename R> __host__ __device__ constexpr int lds_body_cap() {
-  return SOLVE_LDS_BYTES / (4 * (int)sizeof(V4<R>));
-}
-
 // The scene parameters the friction projection reads, taken into registers
 // once per solve: a reference into the scene table would be read again from
 // memory after every colour phase's fence.
@@ -1622,12 +1676,9 @@ __device__ __forceinline__ bool grid_merit(unsigned long long* slots, int it, do
   return *s_ok != 0;
 }
 
-// Working (wl, wa) and accepted (sl, sa) velocity changes of a group's
-// bodies: LDS (slot - base) or the arena arrays (by body).
-template <typename R, bool LDS> struct VelStore {
+// Working (wl, wa) and accepted (sl, sa) velocity changes of the bodies (arena arrays).
+template <typename R> struct VelStore {
   V4<R>* wl; V4<R>* wa; V4<R>* sl; V4<R>* sa;
-  int base;
-  __device__ __forceinline__ int at(int slot, int body) const { return LDS ? slot - base : body; }
 };
 
 // the constant rows of one contact and its previous iterate
@@ -1653,15 +1704,15 @@ template <typename R> __device__ __forceinline__ void load_item(const Dev<R>& d,
 // working velocity changes; Jacobi (jacobi_solver.py:6-57) reads the
 // accepted ones and adds its change to the working ones.  Returns
 // max |x_new - x_old| in FP64.
-template <typename R, bool LDS>
-__device__ __forceinline__ double update_contact(const ProxParams& pp, const Item<R>& it, VelStore<R, LDS>& w,
+template <typename R>
+__device__ __forceinline__ double update_contact(const ProxParams& pp, const Item<R>& it, VelStore<R>& w,
                                                  V4<R>* xn, int kk, R rs, bool jacobi, bool hybrid) {
   ContactRow<R> J;
   contact_rows(it.n, it.rA, it.rB, J);
   const V4<R> rr = {it.r0.x * rs, it.r0.y * rs, it.r0.z * rs, it.r0.w * rs};
   const V4<R> mu = {it.n.w, it.rA.w, it.rB.w, R(0)};
   const bool fa = it.loc.x >= 0, fb = it.loc.y >= 0;
-  const int sa = w.at(it.loc.x, it.id.x), sb = w.at(it.loc.y, it.id.y);
+  const int sa = it.id.x, sb = it.id.y;
   const V4<R> z = {R(0), R(0), R(0), R(0)};
   const V4<R>* rl = jacobi ? w.sl : w.wl;
   const V4<R>* ra = jacobi ? w.sa : w.wa;
@@ -1700,8 +1751,8 @@ template <int STRIDE> __device__ __forceinline__ void phase_sync() {
 // lanes (a wavefront or the workgroup) take the contacts of a colour, in
 // passes of STRIDE; colours are separated by a sync.  coff: colour offsets
 // Returns this thread's max |dx|.
-template <typename R, bool LDS, int STRIDE>
-__device__ double sweep_lane(const Dev<R>& d, const ProxParams& pp, VelStore<R, LDS>& w, int p0, int nc,
+template <typename R, int STRIDE>
+__device__ double sweep_lane(const Dev<R>& d, const ProxParams& pp, VelStore<R>& w, int p0, int nc,
                              const int* coff, bool jacobi, bool hybrid, const V4<R>* xa, V4<R>* xn,
                              R rs, int lane) {
   double m = 0.0;
@@ -1748,28 +1799,15 @@ struct Group {
   bool lead;          // writes the scene's solver state
 };
 
-template <typename R, bool LDS, bool COOP, int NT>
-__device__ void solve_group(const Dev<R>& d, const int slot, const Group& gr, V4<R>* smem, double* sh_red,
-                            int* s_ok) {
+template <typename R, bool COOP, int NT>
+__device__ void solve_group(const Dev<R>& d, const int slot, const Group& gr, double* sh_red, int* s_ok) {
   const SceneParams& sp = d.sp[slot];
   SceneState& st = d.ss[slot];
   const int b0 = gr.b_lo, nbody = gr.b_hi - gr.b_lo;
-  constexpr int CAP = lds_body_cap<R>();
-  VelStore<R, LDS> w;
-  if (LDS) { w.wl = smem; w.wa = smem + CAP; w.sl = smem + 2 * CAP; w.sa = smem + 3 * CAP; }
-  else { w.wl = d.ww0; w.wa = d.ww1; w.sl = d.ws0; w.sa = d.ws1; }
-  w.base = b0;
-  if (LDS) {
-    for (int i = threadIdx.x; i < nbody; i += blockDim.x) {
-      const int b = d.u_blist[b0 + i];
-      w.wl[i] = d.ww0[b]; w.wa[i] = d.ww1[b]; w.sl[i] = d.ws0[b]; w.sa[i] = d.ws1[b];
-    }
-    __syncthreads();
-  }
+  VelStore<R> w{d.ww0, d.ww1, d.ws0, d.ws1};
   const bool jacobi = sp.scheme == SCHEME_JACOBI || sp.scheme == SCHEME_JACOBI_HYBRID;
   const bool hybrid = sp.scheme == SCHEME_JACOBI_HYBRID;
   const ProxParams pp(sp);
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, nwave = blockDim.x >> 6;
   double* res = residual_record(d, sp);
   SolveCtl ctl;
   ctl.iters = sp.max_iter;
@@ -1778,19 +1816,11 @@ __device__ void solve_group(const Dev<R>& d, const int slot, const Group& gr, V4
     V4<R>* xn = ctl.acc ? d.x0 : d.x1;
     const R rs = R(ctl.rscale);
     double m = 0.0;
-    if (LDS) {
-      for (int l = gr.l_lo + wave; l < gr.l_hi; l += nwave) {
-        const int p0 = d.l_start[l], K = d.l_end[l] - p0;
-        if (K <= 0 || K > WAVE_LANE_MAX) continue;
-        m = fmax(m, sweep_lane<R, LDS, 64>(d, pp, w, p0, d.l_ncol[l], lane_coff(d, l), jacobi,
-                                           hybrid, xa, xn, rs, lane));
-      }
-    }
     for (int l = gr.l_lo; l < gr.l_hi; ++l) {
       const int p0 = d.l_start[l], K = d.l_end[l] - p0;
-      if (K <= 0 || (LDS && K <= WAVE_LANE_MAX)) continue;
-      m = fmax(m, sweep_lane<R, LDS, NT>(d, pp, w, p0, d.l_ncol[l], lane_coff(d, l),
-                                                  jacobi, hybrid, xa, xn, rs, (int)threadIdx.x));
+      if (K <= 0) continue;
+      m = fmax(m, sweep_lane<R, NT>(d, pp, w, p0, d.l_ncol[l], lane_coff(d, l), jacobi, hybrid, xa, xn, rs,
+                                    (int)threadIdx.x));
     }
     double merit = block_max(m, sh_red);
     if (COOP && !grid_merit(d.merit, it, merit, d.err, s_ok, sh_red)) return;
@@ -1798,7 +1828,7 @@ __device__ void solve_group(const Dev<R>& d, const int slot, const Group& gr, V4
                                hinge_merit(d, sp, it));
     // accepted sweep: ws <- ww, else ww <- ws
     for (int i = threadIdx.x; i < nbody; i += blockDim.x) {
-      const int s = LDS ? i : d.u_blist[b0 + i];
+      const int s = d.u_blist[b0 + i];
       if (dec & 1) { w.sl[s] = w.wl[s]; w.sa[s] = w.wa[s]; }
       else { w.wl[s] = w.sl[s]; w.wa[s] = w.sa[s]; }
     }
@@ -1822,7 +1852,7 @@ __device__ void solve_group(const Dev<R>& d, const int slot, const Group& gr, V4
       contact_rows(c.n, c.rA, c.rB, J);
       const V4<R> mu = {c.n.w, c.rA.w, c.rB.w, R(0)};
       const bool fa = c.loc.x >= 0, fb = c.loc.y >= 0;
-      const int sa = w.at(c.loc.x, c.id.x), sb = w.at(c.loc.y, c.id.y);
+      const int sa = c.id.x, sb = c.id.y;
       const V4<R> lA = fa ? w.sl[sa] : z, aA = fa ? w.sa[sa] : z;
       const V4<R> lB = fb ? w.sl[sb] : z, aB = fb ? w.sa[sb] : z;
       const V4<R> y = contact_prox(pp, J, x, c.b, c.r0, mu, xyz(lA), xyz(aA), xyz(lB), xyz(aB), false);
@@ -1831,12 +1861,6 @@ __device__ void solve_group(const Dev<R>& d, const int slot, const Group& gr, V4
       xmax = fmax(xmax, absmax4(x.x, x.y, x.z, x.w));
     }
   }
-  if (LDS)
-    for (int i = threadIdx.x; i < nbody; i += blockDim.x) {
-      const int b = d.u_blist[b0 + i];
-      d.ws0[b] = w.sl[i];
-      d.ws1[b] = w.sa[i];
-    }
   const double rm = block_max(rloc, sh_red), xm = block_max(xmax, sh_red);
   if (threadIdx.x == 0) {
     if (d.post) {
@@ -1862,14 +1886,6 @@ template <int K> __device__ __forceinline__ double quad_bcast(double v) {
   return __hiloint2double(hi, lo);
 }
 
-// One lane's share of a contact for the quad update: row q of J (lin, angA,
-// angB with b, r0, mu in w), its iterate and the contact's two body slots.
-template <typename R> struct QuadRow {
-  V4<R> jl, ja, jb;
-  R xo;
-  int2 lc;
-};
-
 // One field of the bodies' LDS records: entry i of a record array with
 // BODY_REC vec4s per body.
 constexpr int BODY_REC = 6;
@@ -1881,110 +1897,20 @@ template <typename R> struct BodyCol {
 // bytes of one body record
 template <typename R> __host__ __device__ constexpr int rec_bytes() { return BODY_REC * (int)sizeof(V4<R>); }
 
-// Velocity changes and inverse masses of a group's bodies in LDS, one record
-// per slot: working (wl, wa) and accepted (sl, sa) velocity changes, W0, W1.
-// A contact's loads of one body then share one address.  Slot zs stays zero
-// and stands for every fixed body; slot ts = zs + 1 takes the discarded
-// velocity updates of fixed bodies, so no update branches on them.
+// Velocity changes and inverse masses of a group's bodies at the start of its
+// LDS, one record each: working (wl, wa) and accepted (sl, sa) velocity
+// changes, W0, W1.  A contact's loads of one body then share one address.  The
+// first record stays zero and stands for every fixed body, the second takes
+// the discarded velocity updates of fixed bodies (so no update branches on
+// them), the group's bodies follow.
+constexpr int BODY_SPARE = 2;
 template <typename R> struct BodyLds {
-  BodyCol<R> wl, wa, sl, sa, W0, W1;
-  unsigned char* base;
-  __device__ void at(V4<R>* b) {
-    base = reinterpret_cast<unsigned char*>(b);
+  BodyCol<R> wl, wa, sl, sa, W0, W1;   // (index -2: the zero record)
+  __device__ explicit BodyLds(unsigned char* smem) {
+    V4<R>* b = reinterpret_cast<V4<R>*>(smem) + BODY_REC * BODY_SPARE;
     wl.p = b; wa.p = b + 1; sl.p = b + 2; sa.p = b + 3; W0.p = b + 4; W1.p = b + 5;
   }
-  // field f of the record at byte offset off (a slot times rec_bytes)
-  __device__ __forceinline__ V4<R>& rec(int off, int f) const {
-    return *reinterpret_cast<V4<R>*>(base + off + f * (int)sizeof(V4<R>));
-  }
 };
-
-// One contact by one quad; lane q holds row q.  Every lane repeats the serial
-// update's operations (update_contact) on the same operands in the same
-// order, so the results are bitwise the same.  it.lc holds the byte offsets
-// of the two bodies' records (zsb: the zero record of fixed bodies, tsb: the
-// discard record).  Writes this lane's velocity block (to the discard record
-// for a fixed body); returns the new iterate in xq and |xq - xo| in FP64.
-// JAC: Jacobi reads the accepted velocity changes (jacobi_solver.py:6-57),
-// Gauss-Seidel the working ones.
-// JL/JA/JB + 4 i: the contact's rows (LDS or global); this lane's velocity
-// block is built from rows 0..3 of one of them, loaded first.
-template <typename R, bool JAC, typename F>
-__device__ __forceinline__ double quad_core(const ProxParams& pp, const QuadRow<R>& it, int q, R rs, bool hybrid,
-                                            const BodyLds<R>& B, int zsb, int tsb, const V4<R>* JL,
-                                            const V4<R>* JA, const V4<R>* JB, size_t i4, R& xq, F&& after_loads) {
-  constexpr int FL = JAC ? F_SL : F_WL, FA = JAC ? F_SA : F_WA;
-  const bool side_b = q >= 2, ang = q & 1;   // lane 0: linear A, 1: angular A, 2: linear B, 3: angular B
-  const int offA = it.lc.x, offB = it.lc.y;
-  const int off = side_b ? offB : offA;
-  const bool own = off != zsb;
-  // fixed bodies read the zero record (the serial update uses zeros for them)
-  const V4<R> lA = B.rec(offA, FL), aA = B.rec(offA, FA), lB = B.rec(offB, FL), aB = B.rec(offB, FA);
-  const V4<R> W0 = B.rec(off, F_W0), W1 = B.rec(off, F_W1);
-  // the working block this lane updates, read beside the four blocks above (in
-  // Gauss-Seidel it is one of them: no other quad of the phase writes it)
-  const int fo = ang ? (int)sizeof(V4<R>) : 0;
-  const V4<R> old = B.rec(off + fo, F_WL);
-  // the caller's loads (the next phase's contact), issued behind this phase's
-  after_loads();
-  const V4<R>* srcv = (q & 1) ? (q >= 2 ? JB : JA) : JL;
-  const V4<R> v0 = srcv[i4], v1 = srcv[i4 + 1], v2 = srcv[i4 + 2], v3 = srcv[i4 + 3];
-  const V4<R> jl = it.jl, ja = it.ja, jb = it.jb;
-  const R xo = it.xo;
-  // row q of z = x - r (J w + b)  (contacts.py:77-92)
-  const R Jw = row_jw(xyz(jl), xyz(ja), xyz(jb), xyz(lA), xyz(aA), xyz(lB), xyz(aB));
-  const R z = row_z(xo, ja.w * rs, Jw, jl.w);
-  const R z0 = quad_bcast<0>(z), z1 = quad_bcast<1>(z), z2 = quad_bcast<2>(z), z3 = quad_bcast<3>(z);
-  const R xo0 = quad_bcast<0>(xo);
-  const R mu0 = quad_bcast<1>(jb.w), mu1 = quad_bcast<2>(jb.w), mu2 = quad_bcast<3>(jb.w);
-  // projections (contacts.py:92-95), the same in every lane of the quad
-  const R xnrm = fmax(R(0), z0);
-  const R xr = (JAC && !hybrid) ? xo0 : xnrm;
-  R os, ot, orr;
-  if (pp.friction == 1) {
-    const V3<R> o = prox_ellipsoid_call<R>(z1, z2, z3, mu0, mu1, mu2, xr, pp.ell_tol, pp.ell_expansion, pp.ell_max_iter);
-    os = o.x; ot = o.y; orr = o.z;
-  } else {
-    prox_sphere<R>(z1, z2, z3, mu0, xr, os, ot, orr);
-  }
-  // row q's new value, by two selects on the bits of q
-  const R x01 = ang ? os : xnrm, x23 = ang ? orr : ot;
-  xq = side_b ? x23 : x01;
-  const R dq = xq - xo;
-  const R d0 = quad_bcast<0>(dq), d1 = quad_bcast<1>(dq), d2 = quad_bcast<2>(dq), d3 = quad_bcast<3>(dq);
-  // w += W J^T dx (contacts.py:107), this lane's block; a fixed body's
-  // (zero W, zero block) lands in the discard record
-  {
-    const R sign = side_b ? R(1) : R(-1);
-    const R s0 = sign * d0, s1 = sign * d1, s2 = sign * d2, s3 = sign * d3;
-    V3<R> acc = {sum_first(v0.x * s0), sum_first(v0.y * s0), sum_first(v0.z * s0)};
-    acc.x = madd(v1.x, s1, acc.x); acc.y = madd(v1.y, s1, acc.y); acc.z = madd(v1.z, s1, acc.z);
-    acc.x = madd(v2.x, s2, acc.x); acc.y = madd(v2.y, s2, acc.y); acc.z = madd(v2.z, s2, acc.z);
-    acc.x = madd(v3.x, s3, acc.x); acc.y = madd(v3.y, s3, acc.y); acc.z = madd(v3.z, s3, acc.z);
-    V4<R> nw;
-    if (ang) {
-      const R W[6] = {W0.x, W0.y, W0.z, W0.w, W1.x, W1.y};
-      const V3<R> t = sym_madd(W, acc);
-      nw = V4<R>{old.x + t.x, old.y + t.y, old.z + t.z, R(0)};
-    } else {
-      nw = V4<R>{madd(W1.z, acc.x, old.x), madd(W1.z, acc.y, old.y), madd(W1.z, acc.z, old.z), R(0)};
-    }
-    B.rec((own ? off : tsb) + fo, F_WL) = nw;
-  }
-  return fabs((double)xq - (double)xo);
-}
-
-// lane q's share of contact i from row arrays (LDS or global); body slots
-// made local and turned into record byte offsets
-template <typename R>
-__device__ __forceinline__ void load_quad(const V4<R>* JL, const V4<R>* JA, const V4<R>* JB, const R* xa,
-                                          const int2* loc, int i, int q, int b0, int zs, QuadRow<R>& it) {
-  const size_t row = 4 * (size_t)i + q;
-  it.jl = JL[row]; it.ja = JA[row]; it.jb = JB[row];
-  it.xo = xa[row];
-  const int2 lc = loc[i];
-  it.lc = make_int2((lc.x >= 0 ? lc.x - b0 : zs) * rec_bytes<R>(), (lc.y >= 0 ? lc.y - b0 : zs) * rec_bytes<R>());
-}
 
 // natural-map residual parts of a contact (FP64) from its rows (row r at JL[S r],
 // JA[S r], JB[S r]), its final values xs[0..3] and the accepted velocity changes
@@ -2010,32 +1936,22 @@ __device__ __forceinline__ void quad_finish_contact(const ProxParams& pp, const 
   xmax = fmax(xmax, absmax4(x.x, x.y, x.z, x.w));
 }
 
-// ---- resident layout
-// Everything a sweep touches lies in LDS, staged once per solve: the group's
-// bodies (one record each, slot nb the zero record of fixed bodies, slot nb + 1
-// the discard record), one record per contact, and a schedule.  A sweep issues
-// no global memory access.
-//
-// A contact's record: row r of J at r * ROW as (lin_r, b_r | angA_r, r0_r |
-// angB_r, mu_r), both iterates, and the LDS offsets of its bodies' records: A
-// and B to read, A and B to write (a fixed body is written to the discard
-// record).  Under the isotropic projection every row's mu_r is mu_1, the only
-// one it reads.  Record nc is the null contact (zero rows and iterates, both
-// bodies fixed), which changes nothing.
-//
-// The schedule lists, phase by phase, the record of each quad's contact (in
-// units of 16 bytes; the null contact where a quad has none).  A phase is at
-// most 16 contacts of one colour, so a wavefront needs no test of positions
-// against colour ends, no loop over a wide colour, and no branch.
-template <typename R> struct Rec {
-  static constexpr int ROW = 12 * (int)sizeof(R);
-  static constexpr int X0 = 4 * ROW, X1 = X0 + 4 * (int)sizeof(R), LOC = X1 + 4 * (int)sizeof(R);
-  static constexpr int BYTES = (LOC + 16 + 4 * (int)sizeof(R) - 1) / (4 * (int)sizeof(R)) * (4 * (int)sizeof(R));
-};
+// LDS as plain 32-bit addresses: an access costs no address arithmetic beyond
+// its own offset
+template <typename T> using LdsPtr = __attribute__((address_space(3))) T*;
+__device__ __forceinline__ int lds_addr(void* p) { return (int)(unsigned)(size_t)(LdsPtr<unsigned char>)p; }
+template <typename T> __device__ __forceinline__ T& lds_at(int addr) { return *(T*)(LdsPtr<T>)(size_t)(unsigned)addr; }
+
+// LDS addresses of a contact's bodies (A and B to read, A and B to write) from
+// their slots; body: the address of the group's first record, b0 its first slot
+template <typename R> __device__ __forceinline__ int4 contact_bodies(int2 loc, int body, int b0) {
+  const int a = body + (loc.x - b0 + BODY_SPARE) * rec_bytes<R>(), b = body + (loc.y - b0 + BODY_SPARE) * rec_bytes<R>();
+  const int z = body, t = body + rec_bytes<R>();
+  return make_int4(loc.x >= 0 ? a : z, loc.y >= 0 ? b : z, loc.x >= 0 ? a : t, loc.y >= 0 ? b : t);
+}
 
 constexpr int RES_LANES = 64;   // lanes of a resident group
-constexpr int PHASE_Q = 16;     // quads of a wavefront: contacts per phase
-constexpr int PHASE_B = 2 * PHASE_Q;   // bytes of one phase of the schedule
+constexpr int PHASE_B = 2 * PHASE_Q;   // bytes of one phase of a resident lane's schedule
 constexpr int PHASE_PAD = 4;    // phases read past a lane's last one
 
 // LDS of a solve workgroup and the most contacts and bodies a tuning may ask
@@ -2046,51 +1962,34 @@ template <typename R, int H = 0> struct ResCap {
   static constexpr int B = C;                                   // bodies: limit of rbh_tuning.resident_bodies
   static constexpr size_t LDS = (size_t)(H ? 80 : 160) * 1024 - 512;   // dynamic LDS of the launch
   static constexpr size_t BYTES = LDS - 128;                            // of it for the layouts (solve_scratch has the rest)
-  // the streaming layout keeps only bodies (and the zero and discard slots) in the same LDS
-  static constexpr int VB = (int)(BYTES / (6 * sizeof(V4<R>))) - 2;
+  // the streaming layout keeps only bodies in the same LDS
+  static constexpr int VB = (int)(BYTES / (6 * sizeof(V4<R>))) - BODY_SPARE;
 };
 
-// LDS addresses of a group of nb bodies, nc contacts, nl lanes (plain 32-bit
-// addresses: an access costs no address arithmetic beyond its own offset)
-template <typename T> using LdsPtr = __attribute__((address_space(3))) T*;
+// LDS addresses of a resident group of nb bodies, nc contacts, nl lanes: its
+// bodies, one record per contact (as in s_rec, the bodies as LDS addresses)
+// and the null contact's, the lane table and the lanes' schedules.  A schedule
+// lists, phase by phase, the record of each quad's contact (in units of 16
+// bytes; the null contact where a quad has none).  A phase is at most 16
+// contacts of one level, so a wavefront needs no test of positions against
+// level ends, no loop over a wide level, and no branch.
 template <typename R> struct ResLds {
   int body;            // first body record
-  int zsb, tsb;        // records of the zero and the discard slot
   int rec, nul;        // first contact record, the null contact's
   int lt, sched;       // lane table (int4: first record, contacts, first phase, phases), schedule
   __device__ ResLds(unsigned char* p, int nb, int nc, int nl) {
-    body = (int)(unsigned)(size_t)(LdsPtr<unsigned char>)p;
-    zsb = body + nb * rec_bytes<R>();
-    tsb = zsb + rec_bytes<R>();
-    rec = tsb + rec_bytes<R>();
+    body = lds_addr(p);
+    rec = body + (nb + BODY_SPARE) * rec_bytes<R>();
     nul = rec + nc * Rec<R>::BYTES;
     lt = nul + Rec<R>::BYTES;
     sched = lt + nl * (int)sizeof(int4);
   }
   static constexpr size_t bytes(int nb, int nc, int nl, int nph) {
-    return (size_t)(nb + 2) * rec_bytes<R>() + (size_t)(nc + 1) * Rec<R>::BYTES + (size_t)nl * sizeof(int4) +
+    return (size_t)(nb + BODY_SPARE) * rec_bytes<R>() + (size_t)(nc + 1) * Rec<R>::BYTES + (size_t)nl * sizeof(int4) +
            (size_t)(nph + PHASE_PAD) * PHASE_B;
   }
-  template <typename T> __device__ __forceinline__ T& at(int addr) const { return *(T*)(LdsPtr<T>)(size_t)(unsigned)addr; }
 };
 static_assert(ResCap<float>::BYTES / 16 < 65536, "a schedule entry addresses LDS in units of 16 bytes");
-
-// ---- streaming layout: bodies in LDS, contact rows and iterates in global memory
-template <typename R, int H = 0> struct StreamLds {
-  BodyLds<R> B;
-  static constexpr int zs = ResCap<R, H>::VB;
-  static constexpr int ts = ResCap<R, H>::VB + 1;
-  __device__ explicit StreamLds(unsigned char* p) {
-    V4<R>* v = reinterpret_cast<V4<R>*>(p);
-    B.at(v);
-  }
-};
-
-// most phases of a lane of K contacts in nc colours :
-// a colour of w > 0 contacts takes ceil(w / 16) <= 1 + (w - 1) / 16
-__device__ __forceinline__ int lane_phases(int K, int nc) {
-  return min(K, nc + K / PHASE_Q);
-}
 
 // sizes of a group's resident data (uniform over the workgroup)
 struct GroupSize { int p0, nc, nph, nl; };
@@ -2119,31 +2018,60 @@ __device__ __forceinline__ bool group_fits(const Dev<R>& d, const Group& gr, con
          ResLds<R>::bytes(nb, g.nc, g.nl, g.nph) <= ResCap<R, H>::BYTES;
 }
 
-// What a quad's lane needs of its next contact: row q of J, rows 0..3 of the
-// block it updates, that body's inverse mass, the old iterate, and LDS offsets.
-// None of it changes during a sweep, so it is read a phase ahead.
+// What a quad's lane needs of its contact: row q of J, rows 0..3 of the block
+// it updates, the old iterate, that block's inverse mass, LDS addresses.  None
+// of it changes during a sweep.
 template <typename R> struct PhaseIn {
   V4<R> jl, ja, jb, W0, W1;
   V3<R> v0, v1, v2, v3;
   R xo;
-  int oA, oB;      // the two bodies' records
-  int own, wr;     // the velocity block this lane updates: where it is read, where it is written
-  int xw;          // the new iterate
 };
 
-// One sweep of one resident lane by one wavefront: nph phases of up to 16
-// contacts, one per quad, lane q of a quad holding row q (the arithmetic and
-// its order are those of update_contact, so the iterates are bitwise the
-// same).  ISO: the isotropic projection.  JAC: Jacobi reads the accepted
-// velocity changes (jacobi_solver.py:6-57), Gauss-Seidel the working ones.
+// a lane's fixed part in the phases of a sweep
+template <typename R, bool JAC> struct PhaseLane {
+  int q;
+  bool side_b, ang;        // lane 0: linear A, 1: angular A, 2: linear B, 3: angular B
+  int row, blk, fo;        // offsets: row q in a record, the block's rows, the block in a body record
+  int xro, xwo;            // offsets of the old and the new iterate in a record
+  R sgn;
+  static constexpr int VB = (int)sizeof(V4<R>), FV = JAC ? F_SL * VB : F_WL * VB;
+  __device__ PhaseLane(int tid, int acc) {
+    using X = Rec<R>;
+    q = tid & 3;
+    side_b = q >= 2;
+    ang = q & 1;
+    row = q * X::ROW;
+    blk = ang ? (side_b ? 2 * VB : VB) : 0;
+    fo = ang ? VB : 0;
+    xro = (acc ? X::X1 : X::X0) + q * (int)sizeof(R);
+    xwo = (acc ? X::X0 : X::X1) + q * (int)sizeof(R);
+    sgn = side_b ? R(1) : R(-1);
+  }
+  __device__ __forceinline__ int own(const int4& lc) const { return side_b ? lc.y : lc.x; }
+  __device__ __forceinline__ int wr(const int4& lc) const { return (side_b ? lc.w : lc.z) + fo; }
+};
+
+// The four velocity blocks a phase starts from and the block it updates.
+template <typename R> struct PhaseVel { V4<R> lA, aA, lB, aB, old; };
+template <typename R, bool JAC>
+__device__ __forceinline__ PhaseVel<R> phase_velocities(const PhaseLane<R, JAC>& P, int oA, int oB, int own) {
+  constexpr int FV = PhaseLane<R, JAC>::FV, VB = PhaseLane<R, JAC>::VB;
+  return PhaseVel<R>{lds_at<V4<R>>(oA + FV), lds_at<V4<R>>(oA + FV + VB), lds_at<V4<R>>(oB + FV),
+                     lds_at<V4<R>>(oB + FV + VB), lds_at<V4<R>>(own + P.fo)};
+}
+
+// One contact by one quad; lane q holds row q.  The arithmetic and its order
+// are those of update_contact, so the iterates are bitwise the same.  Returns
+// the lane's new iterate; nw: its velocity block after the update.  ISO: the
+// isotropic projection.  JAC: Jacobi reads the accepted velocity changes
+// (jacobi_solver.py:6-57), Gauss-Seidel the working ones.
 //
 // A phase is a serial chain: velocities from LDS, the row products, the
 // projection, the velocity update, back to LDS.  With one wavefront per SIMD
 // nothing else hides its latency (measured here: 8 cycles per dependent
 // vector instruction against 4.5 per independent one, 100 per LDS round trip,
 // 33 per saveexec and branch), so:
-//  * everything but the velocities is read one phase ahead, the bodies'
-//    offsets two ahead and the schedule three ahead;
+//  * everything but the velocities is read ahead;
 //  * the projection and the choice between the linear and the angular block
 //    are selects, not branches;
 //  * a row keeps its own projected value: it needs the others' only through
@@ -2152,98 +2080,104 @@ template <typename R> struct PhaseIn {
 //    the end, and a linear update runs through the same multiply-add as an
 //    angular one (times 1/m instead of times one).
 // A phase is then ~118 instructions and ~570 cycles (0.24 us), bound by their
-// issue; with the branches, the position tests and a wait for the previous
-// phase's writes it took ~1,050.  4,096 spheres, 60 colours, 50 sweeps:
-// solve 1613 -> 875 us.
+// issue; with the branches, position tests and a wait for the previous phase's
+// writes it took ~1,050.  4,096 spheres, 60 colours, 50 sweeps: solve 1613 ->
+// 875 us.
+template <typename R, bool ISO, bool JAC>
+__device__ __forceinline__ R phase_update(const ProxParams& pp, const PhaseLane<R, JAC>& P, const PhaseIn<R>& c,
+                                          const PhaseVel<R>& v, R rs, bool hybrid, V4<R>& nw) {
+  // row q of z = x - r (J w + b)  (contacts.py:77-92)
+  const R Jw = row_jw(xyz(c.jl), xyz(c.ja), xyz(c.jb), xyz(v.lA), xyz(v.aA), xyz(v.lB), xyz(v.aB));
+  const R z = row_z(c.xo, c.ja.w * rs, Jw, c.jl.w);
+  // projections (contacts.py:92-95)
+  const R z0 = fmax(R(0), z);
+  const R xnrm = quad_bcast<0>(z0);
+  const R xr = (JAC && !hybrid) ? quad_bcast<0>(c.xo) : xnrm;
+  R val;
+  if constexpr (ISO) {
+    const R zz = z * z;
+    const R sq = (quad_bcast<1>(zz) + quad_bcast<2>(zz)) + quad_bcast<3>(zz);
+    val = prox_sphere_row<R>(z, sq, c.jb.w, xr);
+  } else {
+    const R z1 = quad_bcast<1>(z), z2 = quad_bcast<2>(z), z3 = quad_bcast<3>(z);
+    const R mu0 = quad_bcast<1>(c.jb.w), mu1 = quad_bcast<2>(c.jb.w), mu2 = quad_bcast<3>(c.jb.w);
+    const V3<R> o = prox_ellipsoid_call<R>(z1, z2, z3, mu0, mu1, mu2, xr, pp.ell_tol, pp.ell_expansion, pp.ell_max_iter);
+    val = P.side_b ? (P.ang ? o.z : o.y) : o.x;
+  }
+  const R xq = P.q == 0 ? z0 : val;
+  const R dq = xq - c.xo;
+  // w += W J^T dx (contacts.py:107), this lane's block
+  const R d0 = quad_bcast<0>(dq), d1 = quad_bcast<1>(dq), d2 = quad_bcast<2>(dq), d3 = quad_bcast<3>(dq);
+  V3<R> a = {sum_first(d0 * c.v0.x), sum_first(d0 * c.v0.y), sum_first(d0 * c.v0.z)};
+  a.x = madd(d1, c.v1.x, a.x); a.y = madd(d1, c.v1.y, a.y); a.z = madd(d1, c.v1.z, a.z);
+  a.x = madd(d2, c.v2.x, a.x); a.y = madd(d2, c.v2.y, a.y); a.z = madd(d2, c.v2.z, a.z);
+  a.x = madd(d3, c.v3.x, a.x); a.y = madd(d3, c.v3.y, a.y); a.z = madd(d3, c.v3.z, a.z);
+  const R W[6] = {c.W0.x, c.W0.y, c.W0.z, c.W0.w, c.W1.x, c.W1.y};
+  const V3<R> t = sym_madd(W, a);
+  const R s = P.ang ? P.sgn : P.sgn * c.W1.z;
+  const V3<R> u = {P.ang ? t.x : a.x, P.ang ? t.y : a.y, P.ang ? t.z : a.z};
+  nw = V4<R>{madd(s, u.x, v.old.x), madd(s, u.y, v.old.y), madd(s, u.z, v.old.z), R(0)};
+  return xq;
+}
+
+// ---- resident layout: everything a sweep touches in LDS
+
+// One sweep of one resident lane by one wavefront, one contact per quad and
+// phase.  Rows, inverse masses and iterates are read one phase ahead, the
+// bodies' addresses two ahead and the schedule three ahead.
 template <typename R, bool ISO, bool JAC>
 __device__ double res_sweep(const ProxParams& pp, const ResLds<R>& L, int4 lt, bool hybrid, int acc, R rs, int lane) {
   using X = Rec<R>;
-  constexpr int VB = (int)sizeof(V4<R>), FV = JAC ? F_SL * VB : F_WL * VB;
+  constexpr int VB = (int)sizeof(V4<R>);
+  struct In : PhaseIn<R> { int oA, oB, own, wr, xw; };
   const int rec0 = __builtin_amdgcn_readfirstlane(lt.x), K = __builtin_amdgcn_readfirstlane(lt.y);
   const int nph = __builtin_amdgcn_readfirstlane(lt.w);
-  const int q = lane & 3;
-  const bool side_b = q >= 2, ang = q & 1;   // lane 0: linear A, 1: angular A, 2: linear B, 3: angular B
-  const int row = q * X::ROW, blk = ang ? (side_b ? 2 * VB : VB) : 0, fo = ang ? VB : 0;
-  const int xa = (acc ? X::X1 : X::X0), xn = (acc ? X::X0 : X::X1);
-  const int xro = xa + q * (int)sizeof(R), xwo = xn + q * (int)sizeof(R);
-  const R sgn = side_b ? R(1) : R(-1);
   if (nph <= 0) return 0.0;
+  const PhaseLane<R, JAC> P(lane, acc);
   int sp = L.sched + __builtin_amdgcn_readfirstlane(lt.z) * PHASE_B + 2 * (lane >> 2);
-  auto entry = [&](int ahead) { return (int)L.template at<unsigned short>(sp + ahead * PHASE_B) * 16; };
-  auto load = [&](int r, const int4& lc, PhaseIn<R>& p) {
-    const int rr = r + row, rb = r + blk;
-    p.jl = L.template at<V4<R>>(rr);
-    p.ja = L.template at<V4<R>>(rr + VB);
-    p.jb = L.template at<V4<R>>(rr + 2 * VB);
-    p.xo = L.template at<R>(r + xro);
-    p.v0 = xyz(L.template at<V4<R>>(rb));
-    p.v1 = xyz(L.template at<V4<R>>(rb + X::ROW));
-    p.v2 = xyz(L.template at<V4<R>>(rb + 2 * X::ROW));
-    p.v3 = xyz(L.template at<V4<R>>(rb + 3 * X::ROW));
-    const int own = side_b ? lc.y : lc.x;
-    p.W0 = L.template at<V4<R>>(own + F_W0 * VB);
-    p.W1 = L.template at<V4<R>>(own + F_W1 * VB);
+  auto entry = [&](int ahead) { return (int)lds_at<unsigned short>(sp + ahead * PHASE_B) * 16; };
+  auto load = [&](int r, const int4& lc, In& p) {
+    const int rr = r + P.row, rb = r + P.blk;
+    p.jl = lds_at<V4<R>>(rr);
+    p.ja = lds_at<V4<R>>(rr + VB);
+    p.jb = lds_at<V4<R>>(rr + 2 * VB);
+    p.xo = lds_at<R>(r + P.xro);
+    p.v0 = xyz(lds_at<V4<R>>(rb));
+    p.v1 = xyz(lds_at<V4<R>>(rb + X::ROW));
+    p.v2 = xyz(lds_at<V4<R>>(rb + 2 * X::ROW));
+    p.v3 = xyz(lds_at<V4<R>>(rb + 3 * X::ROW));
+    p.own = P.own(lc);
+    p.W0 = lds_at<V4<R>>(p.own + F_W0 * VB);
+    p.W1 = lds_at<V4<R>>(p.own + F_W1 * VB);
     p.oA = lc.x;
     p.oB = lc.y;
-    p.own = own + fo;
-    p.wr = (side_b ? lc.w : lc.z) + fo;
-    p.xw = r + xwo;
+    p.wr = P.wr(lc);
+    p.xw = r + P.xwo;
   };
   int r1 = entry(1), e2 = entry(2);
-  PhaseIn<R> pa, pb;
+  In pa, pb;
   int4 lc1;
   {
     const int r0 = entry(0);
-    const int4 lc0 = L.template at<int4>(r0 + X::LOC);
-    lc1 = L.template at<int4>(r1 + X::LOC);
+    const int4 lc0 = lds_at<int4>(r0 + X::LOC);
+    lc1 = lds_at<int4>(r1 + X::LOC);
     load(r0, lc0, pa);
   }
   // the reads above are done when the loop starts: a wait inside it would
   // also wait for the previous phase's writes
   __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0)
-  auto phase = [&](const PhaseIn<R>& c, PhaseIn<R>& n) {
-    const V4<R> lA = L.template at<V4<R>>(c.oA + FV), aA = L.template at<V4<R>>(c.oA + FV + VB);
-    const V4<R> lB = L.template at<V4<R>>(c.oB + FV), aB = L.template at<V4<R>>(c.oB + FV + VB);
-    const V4<R> old = L.template at<V4<R>>(c.own + F_WL * VB);
+  auto phase = [&](const In& c, In& n) {
+    const PhaseVel<R> v = phase_velocities<R, JAC>(P, c.oA, c.oB, c.own);
     load(r1, lc1, n);
     const int r2 = e2;
-    lc1 = L.template at<int4>(r2 + X::LOC);
+    lc1 = lds_at<int4>(r2 + X::LOC);
     e2 = entry(3);
     r1 = r2;
     sp += PHASE_B;
-    // row q of z = x - r (J w + b)  (contacts.py:77-92)
-    const R Jw = row_jw(xyz(c.jl), xyz(c.ja), xyz(c.jb), xyz(lA), xyz(aA), xyz(lB), xyz(aB));
-    const R z = row_z(c.xo, c.ja.w * rs, Jw, c.jl.w);
-    // projections (contacts.py:92-95)
-    const R z0 = fmax(R(0), z);
-    const R xnrm = quad_bcast<0>(z0);
-    R val;
-    if constexpr (ISO) {
-      const R xr = (JAC && !hybrid) ? quad_bcast<0>(c.xo) : xnrm;
-      const R zz = z * z;
-      const R sq = (quad_bcast<1>(zz) + quad_bcast<2>(zz)) + quad_bcast<3>(zz);
-      val = prox_sphere_row<R>(z, sq, c.jb.w, xr);
-    } else {
-      const R xr = (JAC && !hybrid) ? quad_bcast<0>(c.xo) : xnrm;
-      const R z1 = quad_bcast<1>(z), z2 = quad_bcast<2>(z), z3 = quad_bcast<3>(z);
-      const R mu0 = quad_bcast<1>(c.jb.w), mu1 = quad_bcast<2>(c.jb.w), mu2 = quad_bcast<3>(c.jb.w);
-      const V3<R> o = prox_ellipsoid_call<R>(z1, z2, z3, mu0, mu1, mu2, xr, pp.ell_tol, pp.ell_expansion, pp.ell_max_iter);
-      val = side_b ? (ang ? o.z : o.y) : o.x;
-    }
-    const R xq = q == 0 ? z0 : val;
-    const R dq = xq - c.xo;
-    // w += W J^T dx (contacts.py:107), this lane's block
-    const R d0 = quad_bcast<0>(dq), d1 = quad_bcast<1>(dq), d2 = quad_bcast<2>(dq), d3 = quad_bcast<3>(dq);
-    V3<R> a = {sum_first(d0 * c.v0.x), sum_first(d0 * c.v0.y), sum_first(d0 * c.v0.z)};
-    a.x = madd(d1, c.v1.x, a.x); a.y = madd(d1, c.v1.y, a.y); a.z = madd(d1, c.v1.z, a.z);
-    a.x = madd(d2, c.v2.x, a.x); a.y = madd(d2, c.v2.y, a.y); a.z = madd(d2, c.v2.z, a.z);
-    a.x = madd(d3, c.v3.x, a.x); a.y = madd(d3, c.v3.y, a.y); a.z = madd(d3, c.v3.z, a.z);
-    const R W[6] = {c.W0.x, c.W0.y, c.W0.z, c.W0.w, c.W1.x, c.W1.y};
-    const V3<R> t = sym_madd(W, a);
-    const R s = ang ? sgn : sgn * c.W1.z;
-    const V3<R> u = {ang ? t.x : a.x, ang ? t.y : a.y, ang ? t.z : a.z};
-    L.template at<V4<R>>(c.wr + F_WL * VB) = V4<R>{madd(s, u.x, old.x), madd(s, u.y, old.y), madd(s, u.z, old.z), R(0)};
-    L.template at<R>(c.xw) = xq;
+    V4<R> nw;
+    const R xq = phase_update<R, ISO, JAC>(pp, P, c, v, rs, hybrid, nw);
+    lds_at<V4<R>>(c.wr) = nw;
+    lds_at<R>(c.xw) = xq;
     phase_sync<64>();
   };
   for (int p = 0;;) {
@@ -2256,7 +2190,7 @@ __device__ double res_sweep(const ProxParams& pp, const ResLds<R>& L, int4 lt, b
   double m = 0.0;
   for (int i = lane >> 2; i < K; i += PHASE_Q) {
     const int r = rec0 + i * X::BYTES;
-    m = fmax(m, fabs((double)L.template at<R>(r + xwo) - (double)L.template at<R>(r + xro)));
+    m = fmax(m, fabs((double)lds_at<R>(r + P.xwo) - (double)lds_at<R>(r + P.xro)));
   }
   return m;
 }
@@ -2279,15 +2213,16 @@ __device__ __forceinline__ int sweep_decide(const Dev<R>& d, const SceneParams& 
   return dec;
 }
 
-template <typename R> __device__ void stage_bodies(const Dev<R>& d, const BodyLds<R>& B, int b0, int nb, int zs) {
+template <typename R> __device__ void stage_bodies(const Dev<R>& d, const BodyLds<R>& B, int b0, int nb) {
   for (int i = threadIdx.x; i < nb; i += blockDim.x) {
     const int b = d.u_blist[b0 + i];
     B.wl[i] = d.ww0[b]; B.wa[i] = d.ww1[b]; B.sl[i] = d.ws0[b]; B.sa[i] = d.ws1[b];
     B.W0[i] = d.b_W0[b]; B.W1[i] = d.b_W1[b];
   }
-  if (threadIdx.x == 0) {
+  if (threadIdx.x < BODY_SPARE) {
     const V4<R> z = {R(0), R(0), R(0), R(0)};
-    B.wl[zs] = z; B.wa[zs] = z; B.sl[zs] = z; B.sa[zs] = z; B.W0[zs] = z; B.W1[zs] = z;
+    const int i = (int)threadIdx.x - BODY_SPARE;
+    B.wl[i] = z; B.wa[i] = z; B.sl[i] = z; B.sa[i] = z; B.W0[i] = z; B.W1[i] = z;
   }
 }
 
@@ -2327,8 +2262,7 @@ __device__ void solve_group_resident(const Dev<R>& d, const int slot, const Grou
   const bool iso = pp.friction != 1;
   const int b0 = gr.b_lo, nb = gr.b_hi - gr.b_lo;
   const ResLds<R> L(smem, nb, gs.nc, gs.nl);
-  BodyLds<R> B;
-  B.at(reinterpret_cast<V4<R>*>(smem));
+  const BodyLds<R> B(smem);
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, nwave = blockDim.x >> 6;
   // stage: lane table (fourth entry: the sweep lane, until its schedule is written), an empty schedule,
   // contact records, bodies
@@ -2337,65 +2271,40 @@ __device__ void solve_group_resident(const Dev<R>& d, const int slot, const Grou
     for (int l = gr.l_lo; l < gr.l_hi; ++l) {
       const int a = d.l_start[l], e = d.l_end[l];
       if (e <= a) continue;
-      L.template at<int4>(L.lt + 16 * t++) = make_int4(L.rec + (a - gs.p0) * X::BYTES, e - a, o, l);
+      lds_at<int4>(L.lt + 16 * t++) = make_int4(L.rec + (a - gs.p0) * X::BYTES, e - a, o, l);
       o += lane_phases(e - a, d.l_ncol[l]);
     }
   }
   for (int i = threadIdx.x; i < (gs.nph + PHASE_PAD) * PHASE_Q; i += blockDim.x)
-    L.template at<unsigned short>(L.sched + 2 * i) = (unsigned short)(L.nul / 16);
-  const V4<R> zero = {R(0), R(0), R(0), R(0)};
-  for (int r = threadIdx.x; r < 4 * (gs.nc + 1); r += blockDim.x) {
-    const int i = r >> 2, q = r & 3;
-    const int rec = L.rec + i * X::BYTES;
-    V4<R> jl = zero, ja = zero, jb = zero;
-    R x0 = R(0), x1 = R(0);
-    int2 lc = make_int2(-1, -1);
-    if (i < gs.nc) {
-      const size_t g = 4 * (size_t)gs.p0 + r;
-      jl = d.s_JL[g]; ja = d.s_JA[g]; jb = d.s_JB[g];
-      if (iso) jb.w = d.s_JB[4 * ((size_t)gs.p0 + i) + 1].w;
-      x0 = d.xr0[g]; x1 = d.xr1[g];
-      lc = d.s_loc[gs.p0 + i];
-    }
-    L.template at<V4<R>>(rec + q * X::ROW) = jl;
-    L.template at<V4<R>>(rec + q * X::ROW + VB) = ja;
-    L.template at<V4<R>>(rec + q * X::ROW + 2 * VB) = jb;
-    L.template at<R>(rec + X::X0 + q * (int)sizeof(R)) = x0;
-    L.template at<R>(rec + X::X1 + q * (int)sizeof(R)) = x1;
-    if (q == 0) {
-      const int a = L.body + (lc.x - b0) * rec_bytes<R>(), b = L.body + (lc.y - b0) * rec_bytes<R>();
-      L.template at<int4>(rec + X::LOC) = make_int4(lc.x >= 0 ? a : L.zsb, lc.y >= 0 ? b : L.zsb,
-                                                    lc.x >= 0 ? a : L.tsb, lc.y >= 0 ? b : L.tsb);
-    }
-  }
-  stage_bodies(d, B, b0, nb, nb);
+    lds_at<unsigned short>(L.sched + 2 * i) = (unsigned short)(L.nul / 16);
+  constexpr int WORDS = X::BYTES / 16, LOCW = X::LOC / 16;
+  const int4* src = reinterpret_cast<const int4*>(d.s_rec + (size_t)gs.p0 * X::BYTES);
+  for (int i = threadIdx.x; i < gs.nc * WORDS; i += blockDim.x)
+    if (i % WORDS != LOCW) lds_at<int4>(L.rec + 16 * i) = src[i];
+  for (int i = threadIdx.x; i < WORDS; i += blockDim.x)
+    if (i != LOCW) lds_at<int4>(L.nul + 16 * i) = make_int4(0, 0, 0, 0);
+  for (int i = threadIdx.x; i <= gs.nc; i += blockDim.x)
+    lds_at<int4>(L.rec + i * X::BYTES + X::LOC) =
+        contact_bodies<R>(i < gs.nc ? d.s_loc[gs.p0 + i] : make_int2(-1, -1), L.body, b0);
+  stage_bodies(d, B, b0, nb);
   __syncthreads();
-  // schedules: a wavefront per lane, its colours 64 at a time
+  // schedules: a wavefront per lane, its levels 64 at a time
   for (int t = wave; t < gs.nl; t += nwave) {
-    const int4 lt = L.template at<int4>(L.lt + 16 * t);
+    const int4 lt = lds_at<int4>(L.lt + 16 * t);
     const int nc = d.l_ncol[lt.w];
     const int* co = lane_coff(d, lt.w);
     int ph = lt.z;
     for (int c0 = 0; c0 < nc; c0 += 64) {
       const int c = c0 + lane;
-      int lo = 0, w = 0;
-      if (c < nc) {
-        lo = co[c];
-        w = co[c + 1] - lo;
-      }
+      const int lo = c < nc ? co[c] : 0, w = c < nc ? co[c + 1] - lo : 0;
       const int np = (w + PHASE_Q - 1) / PHASE_Q;
-      int inc = np;
-#pragma unroll
-      for (int o = 1; o < 64; o <<= 1) {
-        const int v = __shfl_up(inc, o, 64);
-        if (lane >= o) inc += v;
-      }
+      const int inc = wave_inclusive_sum(np);
       const int s0 = L.sched + (ph + inc - np) * PHASE_B;
       for (int i = 0; i < w; ++i)   // (slots of one phase are consecutive, and so are its phases)
-        L.template at<unsigned short>(s0 + 2 * i) = (unsigned short)((lt.x + (lo + i) * X::BYTES) / 16);
+        lds_at<unsigned short>(s0 + 2 * i) = (unsigned short)((lt.x + (lo + i) * X::BYTES) / 16);
       ph += __shfl(inc, 63, 64);
     }
-    if (lane == 0) L.template at<int>(L.lt + 16 * t + 12) = ph - lt.z;
+    if (lane == 0) lds_at<int>(L.lt + 16 * t + 12) = ph - lt.z;
   }
   __syncthreads();
   SolveCtl ctl;
@@ -2405,7 +2314,7 @@ __device__ void solve_group_resident(const Dev<R>& d, const int slot, const Grou
     const R rs = R(ctl.rscale);
     double m = 0.0;
     for (int t = wave; t < gs.nl; t += nwave) {
-      const int4 lt = L.template at<int4>(L.lt + 16 * t);
+      const int4 lt = lds_at<int4>(L.lt + 16 * t);
       double ml;
       if (jacobi)
         ml = iso ? res_sweep<R, true, true>(pp, L, lt, hybrid, ctl.acc, rs, lane)
@@ -2423,124 +2332,163 @@ __device__ void solve_group_resident(const Dev<R>& d, const int slot, const Grou
   double rloc = 0.0, xmax = 0.0;
   for (int i = threadIdx.x; i < gs.nc; i += blockDim.x) {
     const int rec = L.rec + i * X::BYTES;
-    const int4 lc = L.template at<int4>(rec + X::LOC);
-    const R* xs = &L.template at<R>(rec + (ctl.acc ? X::X1 : X::X0));
-    const V4<R>* rows = &L.template at<V4<R>>(rec);
+    const int4 lc = lds_at<int4>(rec + X::LOC);
+    const R* xs = &lds_at<R>(rec + (ctl.acc ? X::X1 : X::X0));
+    const V4<R>* rows = &lds_at<V4<R>>(rec);
     V4<R> x;
-    quad_finish_contact<R, 3>(pp, rows, rows + 1, rows + 2, xs, L.template at<V4<R>>(lc.x + F_SL * VB),
-                              L.template at<V4<R>>(lc.x + F_SA * VB), L.template at<V4<R>>(lc.y + F_SL * VB),
-                              L.template at<V4<R>>(lc.y + F_SA * VB), x, rloc, xmax);
+    quad_finish_contact<R, 3>(pp, rows, rows + 1, rows + 2, xs, lds_at<V4<R>>(lc.x + F_SL * VB),
+                              lds_at<V4<R>>(lc.x + F_SA * VB), lds_at<V4<R>>(lc.y + F_SL * VB),
+                              lds_at<V4<R>>(lc.y + F_SA * VB), x, rloc, xmax);
     if (!d.post) d.c_imp[d.perm[gs.p0 + i]] = x;
   }
   finish_group<R, COOP>(d, st, ctl, gr.lead, B, b0, nb, rloc, xmax, sh_red);
 }
 
-// One sweep of one lane in the streaming layout: rows and iterates from
-// global memory, the next pass prefetched into the other of two buffers
-// while the current one is updated.
-template <typename R, int STRIDE, bool JAC>
-__device__ double stream_sweep(const Dev<R>& d, const ProxParams& pp, const BodyLds<R>& B, int zs, int b0, int p0,
-                               int nc, const int* coff, bool hybrid, const R* xa, R* xn, R rs, int tid) {
-  constexpr int PER = STRIDE / 4;
-  const int q = tid & 3, j = tid >> 2;
-  double m = 0.0;
-  if (nc <= 0) return m;
-  int c = 0;
-  int pb = coff[0];                        // first position of the current pass
-  int hi = coff[1];                        // end of the current colour
-  int hn = nc > 1 ? coff[2] : hi;        // end of the next colour
-  QuadRow<R> ia, ib;
-  bool ha = pb + j < hi;
-  if (ha) load_quad(d.s_JL, d.s_JA, d.s_JB, xa, d.s_loc, p0 + pb + j, q, b0, zs, ia);
-  auto step = [&](QuadRow<R>& use, bool have, QuadRow<R>& fill, bool& fhave) {
-    const bool same = pb + PER < hi;
-    int c1, pb1, hi1, hn1;
-    if (same) {
-      c1 = c; pb1 = pb + PER; hi1 = hi; hn1 = hn;
-    } else {
-      c1 = c + 1; pb1 = hi; hi1 = hn;
-      hn1 = c1 + 1 < nc ? coff[c1 + 2] : hi1;
-    }
-    fhave = c1 < nc && pb1 + j < hi1;
-    if (fhave) load_quad(d.s_JL, d.s_JA, d.s_JB, xa, d.s_loc, p0 + pb1 + j, q, b0, zs, fill);
-    if (have) {
-      R xq;
-      m = fmax(m, quad_core<R, JAC>(pp, use, q, rs, hybrid, B, zs * rec_bytes<R>(), (zs + 1) * rec_bytes<R>(),
-                                    d.s_JL, d.s_JA, d.s_JB,
-                            4 * (size_t)(p0 + pb + j), xq, [] {}));
-      xn[4 * (size_t)(p0 + pb + j) + q] = xq;
-    }
-    if (!same) phase_sync<STRIDE>();
-    c = c1; pb = pb1; hi = hi1; hn = hn1;
+// ---- streaming layout: bodies in LDS, contact records in global memory
+
+// One sweep of one lane: its phases from k_order_lanes' list, one contact per
+// quad.  WG: by the whole workgroup (up to NT / 4 contacts of a level per
+// phase, a workgroup barrier between phases), else by one wavefront.  The
+// records of a phase are read from global memory two phases ahead, each lane
+// its own row and block, in three register buffers used in turn; a quad
+// without a contact reads the null record after the last one.  Bound by the
+// phase's chain (phase_update) as long as the records come from L2.  With rows
+// loaded one phase ahead, the block's rows in the phase itself and lanes of
+// more than 512 contacts always swept by the workgroup, the solve took: 24
+// scenes of ~2,100 contacts 6859 us (now 1406), 320 of ~330 1960 (977),
+// 1,500-sphere pile 5278 (2158), 48 meshes 8920 (4300).
+template <typename R, bool ISO, bool JAC, bool WG>
+__device__ double stream_sweep(const Dev<R>& d, const ProxParams& pp, int l, bool hybrid, int acc, R rs, int tid) {
+  using X = Rec<R>;
+  constexpr int VB = (int)sizeof(V4<R>);
+  struct In : PhaseIn<R> { int4 lc; unsigned off; };
+  const int p0 = __builtin_amdgcn_readfirstlane(d.l_start[l]);
+  const int nph = __builtin_amdgcn_readfirstlane(d.l_nph[l]) >> 1;
+  if (nph <= 0) return 0.0;
+  const int j = tid >> 2, lane = tid & 63;
+  const PhaseLane<R, JAC> P(tid, acc);
+  unsigned char* const rec = d.s_rec;
+  const unsigned nul = (unsigned)d.cap_contacts * (unsigned)X::BYTES;
+  // the list, 64 phases at a time (lane i holds phase i of the run), the next run read ahead
+  const unsigned* list = d.l_phase + p0;
+  unsigned run = list[min(lane, nph - 1)], ahead = list[min(64 + lane, nph - 1)];
+  int base = 0;
+  auto fetch = [&](int p, In& n) {
+    if (p - base >= 64) { run = ahead; base += 64; ahead = list[min(base + 64 + lane, nph - 1)]; }
+    const unsigned e = p < nph ? (unsigned)__builtin_amdgcn_readlane((int)run, p & 63) : 0u;
+    const unsigned pos = e >> PHASE_BITS, cnt = e & ((1u << PHASE_BITS) - 1u);
+    n.off = (unsigned)j < cnt ? ((unsigned)p0 + pos + (unsigned)j) * (unsigned)X::BYTES : nul;
+    n.lc = *reinterpret_cast<const int4*>(rec + n.off + X::LOC);
+    const unsigned rr = n.off + P.row, rb = n.off + P.blk;
+    n.jl = *reinterpret_cast<const V4<R>*>(rec + rr);
+    n.ja = *reinterpret_cast<const V4<R>*>(rec + rr + VB);
+    n.jb = *reinterpret_cast<const V4<R>*>(rec + rr + 2 * VB);
+    n.xo = *reinterpret_cast<const R*>(rec + n.off + P.xro);
+    n.v0 = xyz(*reinterpret_cast<const V4<R>*>(rec + rb));
+    n.v1 = xyz(*reinterpret_cast<const V4<R>*>(rec + rb + X::ROW));
+    n.v2 = xyz(*reinterpret_cast<const V4<R>*>(rec + rb + 2 * X::ROW));
+    n.v3 = xyz(*reinterpret_cast<const V4<R>*>(rec + rb + 3 * X::ROW));
   };
-  bool hb = false;
+  auto masses = [&](In& n) {
+    const int own = P.own(n.lc);
+    n.W0 = lds_at<V4<R>>(own + F_W0 * VB);
+    n.W1 = lds_at<V4<R>>(own + F_W1 * VB);
+  };
+  double m = 0.0;
+  In a, b, c;
+  fetch(0, a);
+  fetch(1, b);
+  masses(a);
+  int p = 0;
+  auto phase = [&](In& cur, In& nxt, In& fill) {
+    const PhaseVel<R> v = phase_velocities<R, JAC>(P, cur.lc.x, cur.lc.y, P.own(cur.lc));
+    masses(nxt);
+    fetch(p + 2, fill);
+    V4<R> nw;
+    const R xq = phase_update<R, ISO, JAC>(pp, P, cur, v, rs, hybrid, nw);
+    lds_at<V4<R>>(P.wr(cur.lc)) = nw;
+    if (cur.off != nul) *reinterpret_cast<R*>(rec + cur.off + P.xwo) = xq;
+    m = fmax(m, fabs((double)xq - (double)cur.xo));
+    if (WG) __syncthreads();
+    else phase_sync<64>();
+    ++p;
+  };
   while (true) {
-    step(ia, ha, ib, hb);
-    if (c >= nc) break;
-    step(ib, hb, ia, ha);
-    if (c >= nc) break;
+    phase(a, b, c);
+    if (p >= nph) break;
+    phase(b, c, a);
+    if (p >= nph) break;
+    phase(c, a, b);
+    if (p >= nph) break;
+  }
+  return m;
+}
+
+template <typename R, bool ISO, bool JAC>
+__device__ double stream_lanes(const Dev<R>& d, const ProxParams& pp, const Group& gr, bool hybrid, int acc, R rs) {
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, nwave = blockDim.x >> 6;
+  double m = 0.0;
+  int t = 0;
+  for (int l = gr.l_lo; l < gr.l_hi; ++l) {
+    if (d.l_end[l] <= d.l_start[l] || (d.l_nph[l] & 1)) continue;
+    if (t++ % nwave == wave) m = fmax(m, stream_sweep<R, ISO, JAC, false>(d, pp, l, hybrid, acc, rs, lane));
+  }
+  for (int l = gr.l_lo; l < gr.l_hi; ++l) {   // lanes swept by the workgroup
+    if (d.l_end[l] <= d.l_start[l] || !(d.l_nph[l] & 1)) continue;
+    m = fmax(m, stream_sweep<R, ISO, JAC, true>(d, pp, l, hybrid, acc, rs, (int)threadIdx.x));
   }
   return m;
 }
 
 template <typename R, bool COOP, int NT, int H>
-__device__ void solve_group_stream(const Dev<R>& d, const int slot, const Group& gr, unsigned char* smem,
-                                   double* sh_red, int* s_ok) {
+__device__ void solve_group_stream(const Dev<R>& d, const int slot, const Group& gr, const GroupSize& gs,
+                                   unsigned char* smem, double* sh_red, int* s_ok) {
+  using X = Rec<R>;
   const SceneParams& sp = d.sp[slot];
   SceneState& st = d.ss[slot];
   const bool jacobi = sp.scheme == SCHEME_JACOBI || sp.scheme == SCHEME_JACOBI_HYBRID;
   const bool hybrid = sp.scheme == SCHEME_JACOBI_HYBRID;
   const ProxParams pp(sp);
-  StreamLds<R, H> L(smem);
-  const int b0 = gr.b_lo, nb = gr.b_hi - gr.b_lo;
-  stage_bodies(d, L.B, b0, nb, L.zs);
+  const bool iso = pp.friction != 1;
+  const BodyLds<R> B(smem);
+  const int body = lds_addr(smem), b0 = gr.b_lo, nb = gr.b_hi - gr.b_lo;
+  stage_bodies(d, B, b0, nb);
+  // the contacts' bodies as LDS addresses of this group (the null contact's are the same in every group)
+  for (int i = threadIdx.x; i < gs.nc; i += blockDim.x)
+    *reinterpret_cast<int4*>(d.s_rec + (size_t)(gs.p0 + i) * X::BYTES + X::LOC) =
+        contact_bodies<R>(d.s_loc[gs.p0 + i], body, b0);
+  if (threadIdx.x == 0)
+    *reinterpret_cast<int4*>(d.s_rec + (size_t)d.cap_contacts * X::BYTES + X::LOC) =
+        contact_bodies<R>(make_int2(-1, -1), body, b0);
   __syncthreads();
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, nwave = blockDim.x >> 6;
   SolveCtl ctl;
   ctl.iters = sp.max_iter;
   bool abort = false;
   for (int it = 0; it < sp.max_iter; ++it) {
-    const R* xa = ctl.acc ? d.xr1 : d.xr0;
-    R* xn = ctl.acc ? d.xr0 : d.xr1;
     const R rs = R(ctl.rscale);
-    double m = 0.0;
-    for (int l = gr.l_lo + wave; l < gr.l_hi; l += nwave) {
-      const int p0 = d.l_start[l], K = d.l_end[l] - p0;
-      if (K <= 0 || K > WAVE_LANE_MAX) continue;
-      const int nc = d.l_ncol[l];
-      m = fmax(m, jacobi ? stream_sweep<R, 64, true>(d, pp, L.B, L.zs, b0, p0, nc, lane_coff(d, l), hybrid,
-                                                     xa, xn, rs, lane)
-                         : stream_sweep<R, 64, false>(d, pp, L.B, L.zs, b0, p0, nc, lane_coff(d, l), hybrid,
-                                                      xa, xn, rs, lane));
-    }
-    for (int l = gr.l_lo; l < gr.l_hi; ++l) {
-      const int p0 = d.l_start[l], K = d.l_end[l] - p0;
-      if (K <= WAVE_LANE_MAX) continue;
-      m = fmax(m, jacobi ? stream_sweep<R, NT, true>(d, pp, L.B, L.zs, b0, p0, d.l_ncol[l], lane_coff(d, l),
-                                                     hybrid, xa, xn, rs, (int)threadIdx.x)
-                         : stream_sweep<R, NT, false>(d, pp, L.B, L.zs, b0, p0, d.l_ncol[l], lane_coff(d, l),
-                                                      hybrid, xa, xn, rs, (int)threadIdx.x));
-    }
-    const int dec = sweep_decide<R, COOP>(d, sp, ctl, m, it, gr.lead, sh_red, s_ok, L.B, nb, abort);
+    double m;
+    if (jacobi)
+      m = iso ? stream_lanes<R, true, true>(d, pp, gr, hybrid, ctl.acc, rs)
+              : stream_lanes<R, false, true>(d, pp, gr, hybrid, ctl.acc, rs);
+    else
+      m = iso ? stream_lanes<R, true, false>(d, pp, gr, hybrid, ctl.acc, rs)
+              : stream_lanes<R, false, false>(d, pp, gr, hybrid, ctl.acc, rs);
+    const int dec = sweep_decide<R, COOP>(d, sp, ctl, m, it, gr.lead, sh_red, s_ok, B, nb, abort);
     if (abort) return;
     if (dec & 2) { ctl.iters = it; break; }
   }
-  const R* xs = ctl.acc ? d.xr1 : d.xr0;
   double rloc = 0.0, xmax = 0.0;
-  for (int l = gr.l_lo; l < gr.l_hi; ++l) {
-    const int p0 = d.l_start[l], K = d.l_end[l] - p0;
-    for (int pos = threadIdx.x; pos < K; pos += blockDim.x) {
-      const int i = p0 + pos;
-      const int2 lc = d.s_loc[i];
-      const int sa = lc.x >= 0 ? lc.x - b0 : L.zs, sb = lc.y >= 0 ? lc.y - b0 : L.zs;
-      V4<R> x;
-      const size_t r = 4 * (size_t)i;
-      quad_finish_contact<R, 1>(pp, d.s_JL + r, d.s_JA + r, d.s_JB + r, xs + r, L.B.sl[sa], L.B.sa[sa], L.B.sl[sb],
-                                L.B.sa[sb], x, rloc, xmax);
-      if (!d.post) d.c_imp[d.perm[i]] = x;
-    }
+  for (int i = threadIdx.x; i < gs.nc; i += blockDim.x) {
+    const unsigned char* rec = d.s_rec + (size_t)(gs.p0 + i) * X::BYTES;
+    const int2 lc = d.s_loc[gs.p0 + i];
+    const int sa = lc.x >= 0 ? lc.x - b0 : -BODY_SPARE, sb = lc.y >= 0 ? lc.y - b0 : -BODY_SPARE;
+    const V4<R>* rows = reinterpret_cast<const V4<R>*>(rec);
+    V4<R> x;
+    quad_finish_contact<R, 3>(pp, rows, rows + 1, rows + 2, reinterpret_cast<const R*>(rec + (ctl.acc ? X::X1 : X::X0)),
+                              B.sl[sa], B.sa[sa], B.sl[sb], B.sa[sb], x, rloc, xmax);
+    if (!d.post) d.c_imp[d.perm[gs.p0 + i]] = x;
   }
-  finish_group<R, COOP>(d, st, ctl, gr.lead, L.B, b0, nb, rloc, xmax, sh_red);
+  finish_group<R, COOP>(d, st, ctl, gr.lead, B, b0, nb, rloc, xmax, sh_red);
 }
 
 template <typename R> __device__ __forceinline__ void no_contacts(SceneState& st) {
@@ -2551,10 +2499,10 @@ template <typename R, bool COOP, int NT, int H>
 __device__ __forceinline__ void solve_dispatch(const Dev<R>& d, int slot, const Group& gr, unsigned char* smem,
                                                double* sh_red, int* s_ok) {
   const GroupSize gs = group_size(d, gr);
-  V4<R>* vs = reinterpret_cast<V4<R>*>(smem);
   if (group_fits<R, H>(d, gr, gs)) solve_group_resident<R, COOP, NT, H>(d, slot, gr, gs, smem, sh_red, s_ok);
-  else if (gr.b_hi - gr.b_lo <= ResCap<R, H>::VB) solve_group_stream<R, COOP, NT, H>(d, slot, gr, smem, sh_red, s_ok);
-  else solve_group<R, false, COOP, NT>(d, slot, gr, vs, sh_red, s_ok);
+  else if (gr.b_hi - gr.b_lo <= ResCap<R, H>::VB && rec_addressable<R>(d.cap_contacts))
+    solve_group_stream<R, COOP, NT, H>(d, slot, gr, gs, smem, sh_red, s_ok);
+  else solve_group<R, COOP, NT>(d, slot, gr, sh_red, s_ok);
 }
 
 // The solve kernels' reduction scratch (at most 8 doubles) and flag, at the end
