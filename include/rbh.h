@@ -155,7 +155,8 @@ int rbh_memory_usage(rbh_ctx* ctx, unsigned long long* bytes);
 /* Signed distance of the res I x J x K node grid spanning [min_coord, max_coord]
  * to the closed mesh (V, T): replaces igl.signed_distance inside
  * GRID.create_signed_distance (grid3.py:320-339).  values: I*J*K, index
- * i + I*(j + J*k). */
+ * i + I*(j + J*k).  The context keeps a buffer of up to 64 MiB for the next
+ * call (outside the HBM budget and rbh_memory_usage). */
 int rbh_sdf_build(rbh_ctx* ctx, const double* V, int nv, const int* T, int nt, const double* min_coord,
                   const double* max_coord, int I, int J, int K, double* values);
 
