@@ -131,13 +131,6 @@ __device__ __forceinline__ void hinge_body_w(const Dev<R>& d, const SceneParams&
   }
 }
 
-__device__ __forceinline__ double wave_max_d(double v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
-  return v;
-}
-
-
 // Per-hinge constants a lane needs for one Gauss-Seidel update: lanes 0-4
 // hold row `lane` (J, b, r0), lanes 0-11 the W J^T entries of body entry
 // `lane` for rows 0-4.  Loaded HINGE_AHEAD hinges ahead of their use.
@@ -230,6 +223,7 @@ template <typename R> __global__ void __launch_bounds__(64) k_hinge_solve(Dev<R>
   if (own)
     for (int i = lane; i < sp.max_iter; i += 64) res[i] = INFINITY;
   __syncthreads();
+  const CtlParams cp(sp);
   SolveCtl ctl;
   ctl.iters = sp.max_iter;
   for (int it = 0; it < n_it; ++it) {
@@ -252,12 +246,12 @@ template <typename R> __global__ void __launch_bounds__(64) k_hinge_solve(Dev<R>
     }
     double m = 0.0;
     for (int i = lane; i < nrow; i += 64) m = fmax(m, fabs((double)(x[i] - sol[i])));
-    m = wave_max_d(m);
+    m = wave_max(m);
     int dec;
     if (own) {
-      dec = ctl.decide(sp, m, lane == 0 ? res : nullptr, it);
+      dec = ctl.decide(cp, m, lane == 0 ? res : nullptr, it);
     } else {
-      dec = ctl.accept_or_reject(sp, m);
+      dec = ctl.accept_or_reject(cp, m);
       if (pass == 0 && lane == 0) hm[it] = ctl.gm;
     }
     for (int i = lane; i < nrow; i += 64) {

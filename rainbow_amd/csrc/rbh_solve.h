@@ -1561,10 +1561,32 @@ __device__ __forceinline__ double absmax4(double a, double b, double c, double e
   return fmax(fmax(fabs(a), fabs(b)), fmax(fabs(c), fabs(e)));
 }
 
+// one step of a maximum over a wavefront: v against the lane DPP control CTRL names
+template <int CTRL, int ROWS = 0xf> __device__ __forceinline__ double dpp_max(double v) {
+  const int lo = __double2loint(v), hi = __double2hiint(v);
+  const int l = __builtin_amdgcn_update_dpp(lo, lo, CTRL, ROWS, 0xf, false);
+  const int h = __builtin_amdgcn_update_dpp(hi, hi, CTRL, ROWS, 0xf, false);
+  return fmax(v, __hiloint2double(h, l));
+}
+
+// largest v of a wavefront, in every lane.  By DPP: within the rows of 16
+// lanes by xor 1, xor 2, half-row and row mirror, then row 0 into 1 and 2
+// into 3, then the lower half into the upper (through LDS, as __shfl_xor
+// does it, the six steps cost ~900 cycles, three times as much).
+__device__ __forceinline__ double wave_max(double v) {
+  v = dpp_max<0xb1>(v);          // quad_perm 1, 0, 3, 2
+  v = dpp_max<0x4e>(v);          // quad_perm 2, 3, 0, 1
+  v = dpp_max<0x141>(v);         // row_half_mirror
+  v = dpp_max<0x140>(v);         // row_mirror
+  v = dpp_max<0x142, 0xa>(v);    // row_bcast 15 into rows 1 and 3
+  v = dpp_max<0x143, 0xc>(v);    // row_bcast 31 into rows 2 and 3
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), 63),
+                          __builtin_amdgcn_readlane(__double2loint(v), 63));
+}
+
 __device__ __forceinline__ double block_max(double v, double* sh) {
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
+  v = wave_max(v);
   if (lane == 0) sh[wid] = v;
   __syncthreads();
   double m = 0.0;
@@ -1573,13 +1595,22 @@ __device__ __forceinline__ double block_max(double v, double* sh) {
   return m;
 }
 
+// the scene parameters of the accept/reject driver, taken into registers once
+// per solve
+struct CtlParams {
+  double nu_reduce, nu_increase, too_small, abs_tol, rel_tol;
+  __device__ explicit CtlParams(const SceneParams& sp)
+      : nu_reduce(sp.nu_reduce), nu_increase(sp.nu_increase), too_small(sp.too_small), abs_tol(sp.abs_tol),
+        rel_tol(sp.rel_tol) {}
+};
+
 // gauss_seidel_solver.py:56-97: accept/reject, r-factor, stopping tests.
 struct SolveCtl {
   double last_merit = INFINITY, glast = INFINITY, rscale = 1.0, gm = 0.0;
   int acc = 0, rejects = 0, exitcode = 0, iters = 0, sweeps = 0;
   // accept (bit0) or reject, r-factor update; gm = this problem's contribution
   // to the global merit (its merit, or its last accepted merit on a reject)
-  __device__ int accept_or_reject(const SceneParams& sp, double merit) {
+  __device__ int accept_or_reject(const CtlParams& sp, double merit) {
     int dec = 0;
     if (merit > last_merit) {
       rscale *= sp.nu_reduce;
@@ -1595,7 +1626,7 @@ struct SolveCtl {
   }
   // returns bit0 accept, bit1 stop; `other` is the contribution of the
   // scene's other problem (the hinges) to the global merit of this sweep
-  __device__ int decide(const SceneParams& sp, double merit, double* res, int it, double other = 0.0) {
+  __device__ int decide(const CtlParams& sp, double merit, double* res, int it, double other = 0.0) {
     int dec = accept_or_reject(sp, merit);
     gm = fmax(gm, other);
     if (res) res[it] = gm;
@@ -1608,10 +1639,11 @@ struct SolveCtl {
   }
 };
 
-// the hinge problem's contribution to sweep `it` (recorded before the contact
-// solve; gauss_seidel_solver.py:47-73 takes the largest over the problems)
-template <typename R> __device__ __forceinline__ double hinge_merit(const Dev<R>& d, const SceneParams& sp, int it) {
-  return (sp.h_cnt > 0 && !d.post) ? d.h_mer[sp.res_off + it] : 0.0;
+// the hinge problem's contributions to the sweeps (recorded before the contact
+// solve; gauss_seidel_solver.py:47-73 takes the largest over the problems), or
+// null
+template <typename R> __device__ __forceinline__ const double* hinge_merits(const Dev<R>& d, const SceneParams& sp) {
+  return (sp.h_cnt > 0 && !d.post) ? d.h_mer + sp.res_off : nullptr;
 }
 
 // the scene's per-sweep merit record: the contact solve's 'residuals', then
@@ -1643,37 +1675,62 @@ template <typename R> __device__ void write_solve_state(const Dev<R>& d, SceneSt
 // sweep's G slots are all published and takes their maximum.  Workgroups
 // share no other data during the solve, so the slots need no fences.  The
 // wait is bounded: it flags ERR_SOLVER and returns false instead of hanging.
-__device__ __forceinline__ bool grid_merit(unsigned long long* slots, int it, double& merit, int* err, int* s_ok,
-                                           double* s_m) {
+// (called by wavefront 0 alone, merit the same in all its lanes)
+__device__ __forceinline__ bool grid_merit(unsigned long long* slots, int it, double& merit, int* err) {
   const unsigned G = gridDim.x;
+  if (G == 1) return true;
   unsigned long long* row = slots + (size_t)it * G;
   if (threadIdx.x == 0)
     __hip_atomic_store(&row[blockIdx.x], merit > 0.0 ? (unsigned long long)__double_as_longlong(merit) : 0ull,
                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  if (threadIdx.x < 64) {
-    unsigned long long m = 0;
-    bool ok = true;
-    for (unsigned j = threadIdx.x; j < G && ok; j += 64) {
-      unsigned long long v = __hip_atomic_load(&row[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      for (unsigned spins = 0; v == ~0ull;) {
-        __builtin_amdgcn_s_sleep(1);
-        if (++spins > (1u << 26)) { ok = false; break; }
-        v = __hip_atomic_load(&row[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      }
-      if (ok) m = max(m, v);
+  double m = 0.0;
+  bool ok = true;
+  for (unsigned j = threadIdx.x; j < G && ok; j += 64) {
+    unsigned long long v = __hip_atomic_load(&row[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (unsigned spins = 0; v == ~0ull;) {
+      __builtin_amdgcn_s_sleep(1);
+      if (++spins > (1u << 26)) { ok = false; break; }
+      v = __hip_atomic_load(&row[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) m = max(m, (unsigned long long)__shfl_xor(m, o, 64));
-    const bool all_ok = __ballot(!ok) == 0;
-    if (threadIdx.x == 0) {
-      if (!all_ok) atomicOr(err, ERR_SOLVER);
-      *s_ok = all_ok ? 1 : 0;
-      *s_m = __longlong_as_double((long long)m);
-    }
+    if (ok) m = fmax(m, __longlong_as_double((long long)v));
   }
-  __syncthreads();
-  merit = *s_m;
-  return *s_ok != 0;
+  merit = wave_max(m);
+  const bool all_ok = __ballot(!ok) == 0;
+  if (threadIdx.x == 0 && !all_ok) atomicOr(err, ERR_SOLVER);
+  return all_ok;
+}
+
+// The merit of sweep `it` over the workgroup's threads (v each) and, in a
+// cooperative launch, over the grid; false if the grid's wait failed.  lone:
+// only wavefront 0 swept, so it publishes without waiting for the others.
+// The scratch entries alternate between sweeps (sh: 2 x 8 doubles), so one
+// barrier per exchange is enough: a workgroup meets another one before an
+// entry is written again.
+template <typename R, bool COOP>
+__device__ __forceinline__ bool sweep_merit(const Dev<R>& d, double v, int it, bool lone, double* sh, int* s_ok,
+                                            double& merit) {
+  double* s = sh + 8 * (it & 1);
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  double m = wave_max(v);
+  if (!(COOP && lone)) {
+    if (lane == 0) s[wid] = m;
+    __syncthreads();
+    m = 0.0;
+    for (int i = 0; i < (int)(blockDim.x >> 6); ++i) m = fmax(m, s[i]);
+  }
+  if (COOP) {
+    if (!lone) __syncthreads();     // s is read before it is written again
+    if (wid == 0) {
+      const bool ok = grid_merit(d.merit, it, m, d.err);
+      if (lane == 0) { s[0] = m; *s_ok = ok ? 1 : 0; }
+    }
+    __syncthreads();
+    m = s[0];
+    merit = m;
+    return *s_ok != 0;
+  }
+  merit = m;
+  return true;
 }
 
 // Working (wl, wa) and accepted (sl, sa) velocity changes of the bodies (arena arrays).
@@ -1808,6 +1865,8 @@ __device__ void solve_group(const Dev<R>& d, const int slot, const Group& gr, do
   const bool jacobi = sp.scheme == SCHEME_JACOBI || sp.scheme == SCHEME_JACOBI_HYBRID;
   const bool hybrid = sp.scheme == SCHEME_JACOBI_HYBRID;
   const ProxParams pp(sp);
+  const CtlParams cp(sp);
+  const double* hm = hinge_merits(d, sp);
   double* res = residual_record(d, sp);
   SolveCtl ctl;
   ctl.iters = sp.max_iter;
@@ -1822,10 +1881,9 @@ __device__ void solve_group(const Dev<R>& d, const int slot, const Group& gr, do
       m = fmax(m, sweep_lane<R, NT>(d, pp, w, p0, d.l_ncol[l], lane_coff(d, l), jacobi, hybrid, xa, xn, rs,
                                     (int)threadIdx.x));
     }
-    double merit = block_max(m, sh_red);
-    if (COOP && !grid_merit(d.merit, it, merit, d.err, s_ok, sh_red)) return;
-    const int dec = ctl.decide(sp, merit, (gr.lead && threadIdx.x == 0) ? res : nullptr, it,
-                               hinge_merit(d, sp, it));
+    double merit;
+    if (!sweep_merit<R, COOP>(d, m, it, false, sh_red, s_ok, merit)) return;
+    const int dec = ctl.decide(cp, merit, (gr.lead && threadIdx.x == 0) ? res : nullptr, it, hm ? hm[it] : 0.0);
     // accepted sweep: ws <- ww, else ww <- ws
     for (int i = threadIdx.x; i < nbody; i += blockDim.x) {
       const int s = d.u_blist[b0 + i];
@@ -1961,7 +2019,7 @@ template <typename R, int H = 0> struct ResCap {
   static constexpr int C = (sizeof(R) == 4 ? 384 : 192) >> H;   // contacts: limit of rbh_tuning.resident_contacts
   static constexpr int B = C;                                   // bodies: limit of rbh_tuning.resident_bodies
   static constexpr size_t LDS = (size_t)(H ? 80 : 160) * 1024 - 512;   // dynamic LDS of the launch
-  static constexpr size_t BYTES = LDS - 128;                            // of it for the layouts (solve_scratch has the rest)
+  static constexpr size_t BYTES = LDS - 256;                            // of it for the layouts (solve_scratch has the rest)
   // the streaming layout keeps only bodies in the same LDS
   static constexpr int VB = (int)(BYTES / (6 * sizeof(V4<R>))) - BODY_SPARE;
 };
@@ -1992,10 +2050,10 @@ template <typename R> struct ResLds {
 static_assert(ResCap<float>::BYTES / 16 < 65536, "a schedule entry addresses LDS in units of 16 bytes");
 
 // sizes of a group's resident data (uniform over the workgroup)
-struct GroupSize { int p0, nc, nph, nl; };
+struct GroupSize { int p0, nc, nph, nl; bool wg; };   // wg: a lane is for the whole workgroup (streaming)
 
 template <typename R> __device__ GroupSize group_size(const Dev<R>& d, const Group& gr) {
-  GroupSize g{0x7fffffff, 0, 0, 0};
+  GroupSize g{0x7fffffff, 0, 0, 0, false};
   int p1 = 0;
   for (int l = gr.l_lo; l < gr.l_hi; ++l) {
     const int a = d.l_start[l], e = d.l_end[l];
@@ -2003,6 +2061,7 @@ template <typename R> __device__ GroupSize group_size(const Dev<R>& d, const Gro
     g.p0 = min(g.p0, a);
     p1 = max(p1, e);
     g.nph += lane_phases(e - a, d.l_ncol[l]);
+    g.wg = g.wg || (d.l_nph[l] & 1);
     ++g.nl;
   }
   g.nc = g.nl ? p1 - g.p0 : 0;
@@ -2187,24 +2246,41 @@ __device__ double res_sweep(const ProxParams& pp, const ResLds<R>& L, int4 lt, b
     if (++p >= nph) break;
   }
   // the merit, max |x_new - x_old| in FP64 (a sweep updates each contact once)
+  // 64 contacts per pass, their reads in flight together (past the last
+  // contact the last one again)
   double m = 0.0;
-  for (int i = lane >> 2; i < K; i += PHASE_Q) {
-    const int r = rec0 + i * X::BYTES;
-    m = fmax(m, fabs((double)lds_at<R>(r + P.xwo) - (double)lds_at<R>(r + P.xro)));
+  for (int i = lane >> 2; i - (lane >> 2) < K; i += 4 * PHASE_Q) {
+    R xn[4], xo[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int r = rec0 + min(i + u * PHASE_Q, K - 1) * X::BYTES;
+      xn[u] = lds_at<R>(r + P.xwo);
+      xo[u] = lds_at<R>(r + P.xro);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) m = fmax(m, fabs((double)xn[u] - (double)xo[u]));
   }
   return m;
 }
 
+// what a group's sweeps are decided with, the same for every sweep
+template <typename R> struct Decide {
+  CtlParams cp;
+  const double* hm;    // the hinges' merits, or null
+  double* res;         // the scene's merit record, or null where another thread writes it
+  bool lone;           // only wavefront 0 sweeps
+  __device__ Decide(const Dev<R>& d, const SceneParams& sp, bool lead, bool lone_)
+      : cp(sp), hm(hinge_merits(d, sp)), res(lead && threadIdx.x == 0 ? residual_record(d, sp) : nullptr), lone(lone_) {}
+};
+
 // merit meets, accept/reject decided, velocity changes settled (all groups of the scene)
 template <typename R, bool COOP>
-__device__ __forceinline__ int sweep_decide(const Dev<R>& d, const SceneParams& sp, SolveCtl& ctl, double m,
-                                            int it, bool lead, double* sh_red, int* s_ok, const BodyLds<R>& B, int nb,
-                                            bool& abort) {
-  double merit = block_max(m, sh_red);
-  if (COOP && !grid_merit(d.merit, it, merit, d.err, s_ok, sh_red)) { abort = true; return 0; }
-  double* res = residual_record(d, sp);
-  const int dec = ctl.decide(sp, merit, (lead && threadIdx.x == 0) ? res : nullptr, it,
-                             hinge_merit(d, sp, it));
+__device__ __forceinline__ int sweep_decide(const Dev<R>& d, const Decide<R>& by, SolveCtl& ctl, double m, int it,
+                                            double* sh_red, int* s_ok, const BodyLds<R>& B, int nb, bool& abort) {
+  double merit;
+  const double other = by.hm ? by.hm[it] : 0.0;
+  if (!sweep_merit<R, COOP>(d, m, it, by.lone, sh_red, s_ok, merit)) { abort = true; return 0; }
+  const int dec = ctl.decide(by.cp, merit, by.res, it, other);
   for (int i = threadIdx.x; i < nb; i += blockDim.x) {
     if (dec & 1) { B.sl[i] = B.wl[i]; B.sa[i] = B.wa[i]; }
     else { B.wl[i] = B.sl[i]; B.wa[i] = B.sa[i]; }
@@ -2307,6 +2383,7 @@ __device__ void solve_group_resident(const Dev<R>& d, const int slot, const Grou
     if (lane == 0) lds_at<int>(L.lt + 16 * t + 12) = ph - lt.z;
   }
   __syncthreads();
+  const Decide<R> by(d, sp, gr.lead, gs.nl <= 1);
   SolveCtl ctl;
   ctl.iters = sp.max_iter;
   bool abort = false;
@@ -2324,7 +2401,7 @@ __device__ void solve_group_resident(const Dev<R>& d, const int slot, const Grou
                  : res_sweep<R, false, false>(pp, L, lt, hybrid, ctl.acc, rs, lane);
       m = fmax(m, ml);
     }
-    const int dec = sweep_decide<R, COOP>(d, sp, ctl, m, it, gr.lead, sh_red, s_ok, B, nb, abort);
+    const int dec = sweep_decide<R, COOP>(d, by, ctl, m, it, sh_red, s_ok, B, nb, abort);
     if (abort) return;
     if (dec & 2) { ctl.iters = it; break; }
   }
@@ -2461,6 +2538,7 @@ __device__ void solve_group_stream(const Dev<R>& d, const int slot, const Group&
     *reinterpret_cast<int4*>(d.s_rec + (size_t)d.cap_contacts * X::BYTES + X::LOC) =
         contact_bodies<R>(make_int2(-1, -1), body, b0);
   __syncthreads();
+  const Decide<R> by(d, sp, gr.lead, gs.nl <= 1 && !gs.wg);
   SolveCtl ctl;
   ctl.iters = sp.max_iter;
   bool abort = false;
@@ -2473,7 +2551,7 @@ __device__ void solve_group_stream(const Dev<R>& d, const int slot, const Group&
     else
       m = iso ? stream_lanes<R, true, false>(d, pp, gr, hybrid, ctl.acc, rs)
               : stream_lanes<R, false, false>(d, pp, gr, hybrid, ctl.acc, rs);
-    const int dec = sweep_decide<R, COOP>(d, sp, ctl, m, it, gr.lead, sh_red, s_ok, B, nb, abort);
+    const int dec = sweep_decide<R, COOP>(d, by, ctl, m, it, sh_red, s_ok, B, nb, abort);
     if (abort) return;
     if (dec & 2) { ctl.iters = it; break; }
   }
@@ -2505,13 +2583,13 @@ __device__ __forceinline__ void solve_dispatch(const Dev<R>& d, int slot, const 
   else solve_group<R, COOP, NT>(d, slot, gr, sh_red, s_ok);
 }
 
-// The solve kernels' reduction scratch (at most 8 doubles) and flag, at the end
+// The solve kernels' reduction scratch (2 x 8 doubles) and flag, at the end
 // of the dynamic LDS: with no static LDS the layouts start at LDS address 0,
 // so their offsets fold into the LDS instructions.
 template <typename R, int H>
 __device__ __forceinline__ void solve_scratch(unsigned char* smem, double*& red, int*& ok) {
   red = reinterpret_cast<double*>(smem + ResCap<R, H>::BYTES);
-  ok = reinterpret_cast<int*>(red + 8);
+  ok = reinterpret_cast<int*>(red + 16);
 }
 
 // One workgroup of NT threads (NT / 64 wavefronts, one per sweep lane) per
