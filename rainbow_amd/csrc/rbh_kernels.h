@@ -139,8 +139,8 @@ template <typename R> struct Dev {
   int res_cap_c, res_cap_b;            // most contacts and bodies of a resident solve group (rbh_tuning)
   V4<R>* s_W;                          // 4 per position: W0, W1 of body A, then of body B (zero if fixed)
   unsigned char* s_rec;                // per position its record (Rec<R>), then the null contact's (at cap_contacts)
-  unsigned* l_phase; int* l_nph;       // per lane, from l_start: its phases (first position, contacts); 2 * their
-                                       // number + 1 if the workgroup sweeps it together
+  unsigned* l_phase; int* l_nph;       // per lane, from l_start: its phases (first position, contacts); their number
+                                       // above LANE_BITS flags
   int solve_quads;                     // quads of a solve workgroup
   // hinges (constraints/hinges.py): static per hinge, then per-step rows and iterates
   const int4* h_ids;                   // (parent, child) arena bodies, (parent, child) hinge-body slots

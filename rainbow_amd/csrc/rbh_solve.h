@@ -1121,6 +1121,8 @@ template <typename R> __host__ __device__ constexpr bool rec_addressable(int c) 
 }
 
 constexpr int PHASE_Q = 16;      // quads of a wavefront: contacts per phase of a wavefront's sweep
+constexpr int PHASE_R = 4;       // rows of 16 lanes of a wavefront: contacts per phase of a narrow lane's sweep
+constexpr int LANE_WG = 1, LANE_NARROW = 2, LANE_BITS = 2;   // low bits of l_nph: streamed by the workgroup; narrow if resident
 constexpr int PHASE_BITS = 8;    // low bits of an entry of l_phase: contacts of the phase (at most 128); the rest: its first position
 // most phases of a lane of K contacts in nc levels: a level of w > 0 contacts
 // takes ceil(w / 16) <= 1 + (w - 1) / 16
@@ -1282,6 +1284,21 @@ __device__ __forceinline__ void order_scan(OrderLds& s, int n, int* coff) {
   }
 }
 
+// sum over the levels of ceil(width / per), in every lane of the wavefront
+__device__ __forceinline__ int count_phases(int nl, const int* coff, int per) {
+  const int lane = (int)threadIdx.x & 63;
+  int n = 0;
+  for (int c = lane; c < nl; c += 64) n += (coff[c + 1] - coff[c] + per - 1) / per;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o, 64);
+  return n;
+}
+
+// Whether a resident lane is swept with 16 lanes a contact instead of 4, a
+// quarter of the contacts per phase: a row's phase takes about 0.8 of a quad's
+// (440 cycles against 550), so it may take up to 5/4 as many.
+__device__ __forceinline__ bool narrow_phases(int wide, int narrow) { return 4 * narrow <= 5 * wide; }
+
 // The lane's phases for the streaming sweep, by wavefront 0: at most 16 contacts
 // of one level for a wavefront's sweep, a contact per quad of the workgroup for
 // the workgroup's.  One wavefront takes about nl / 2 + K / 16 phases, the
@@ -1295,6 +1312,7 @@ __device__ __forceinline__ void order_phases(const Dev<R>& d, int l, int nl, con
   const int lanes = d.unit_split > 0 ? min(d.l_cnt[d.l_bs[l]], d.solve_quads / PHASE_Q) : 1;
   const bool wg = K > 8 * lanes * nl;
   const int per = wg ? d.solve_quads : PHASE_Q;
+  const bool narrow = narrow_phases(count_phases(nl, coff, PHASE_Q), count_phases(nl, coff, PHASE_R));
   int ph = 0;
   for (int c0 = 0; c0 < nl; c0 += 64) {
     const int c = c0 + lane;
@@ -1305,7 +1323,8 @@ __device__ __forceinline__ void order_phases(const Dev<R>& d, int l, int nl, con
     for (int i = 0; i < np; ++i) out[i] = (unsigned)(lo + i * per) << PHASE_BITS | (unsigned)min(per, w - i * per);
     ph += __shfl(inc, 63, 64);
   }
-  if (lane == 0) d.l_nph[l] = ph << 1 | (wg ? 1 : 0);
+  if (lane == 0)
+    d.l_nph[l] = ph << LANE_BITS | (narrow ? LANE_NARROW : 0) | (wg ? LANE_WG : 0);
 }
 
 // One workgroup per sweep lane: its positions [l_start, l_end) in sweep order.
@@ -1944,6 +1963,25 @@ template <int K> __device__ __forceinline__ double quad_bcast(double v) {
   return __hiloint2double(hi, lo);
 }
 
+// value of lane K of each row of 16 lanes (DPP row_newbcast)
+template <int K> __device__ __forceinline__ float row_bcast(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x150 + K, 0xf, 0xf, true));
+}
+template <int K> __device__ __forceinline__ double row_bcast(double v) {
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), 0x150 + K, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), 0x150 + K, 0xf, 0xf, true);
+  return __hiloint2double(hi, lo);
+}
+// value of the lane 8 further round its row (DPP row_ror:8)
+__device__ __forceinline__ float row_other_half(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x128, 0xf, 0xf, true));
+}
+__device__ __forceinline__ double row_other_half(double v) {
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), 0x128, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), 0x128, 0xf, 0xf, true);
+  return __hiloint2double(hi, lo);
+}
+
 // One field of the bodies' LDS records: entry i of a record array with
 // BODY_REC vec4s per body.
 constexpr int BODY_REC = 6;
@@ -1957,7 +1995,9 @@ template <typename R> __host__ __device__ constexpr int rec_bytes() { return BOD
 
 // Velocity changes and inverse masses of a group's bodies at the start of its
 // LDS, one record each: working (wl, wa) and accepted (sl, sa) velocity
-// changes, W0, W1.  A contact's loads of one body then share one address.  The
+// changes, inverse masses W0 = (I^-1 xx, xy, xz, 1/m), W1 = (I^-1 yy, yz, zz,
+// 0) -- so that each row of I^-1 is one value and a pair of neighbours.  A
+// contact's loads of one body then share one address.  The
 // first record stays zero and stands for every fixed body, the second takes
 // the discarded velocity updates of fixed bodies (so no update branches on
 // them), the group's bodies follow.
@@ -2027,14 +2067,15 @@ template <typename R, int H = 0> struct ResCap {
 // LDS addresses of a resident group of nb bodies, nc contacts, nl lanes: its
 // bodies, one record per contact (as in s_rec, the bodies as LDS addresses)
 // and the null contact's, the lane table and the lanes' schedules.  A schedule
-// lists, phase by phase, the record of each quad's contact (in units of 16
-// bytes; the null contact where a quad has none).  A phase is at most 16
+// lists, phase by phase, the record of each quad's or row's contact (in units
+// of 16 bytes; the null contact where it has none).  A phase is at most 16 (4)
 // contacts of one level, so a wavefront needs no test of positions against
-// level ends, no loop over a wide level, and no branch.
+// level ends, no loop over a wide level, and no branch.  (A narrow lane's
+// phases, at most nc + K / 4 of 8 bytes, fit in the nc + K / 16 of 32.)
 template <typename R> struct ResLds {
   int body;            // first body record
   int rec, nul;        // first contact record, the null contact's
-  int lt, sched;       // lane table (int4: first record, contacts, first phase, phases), schedule
+  int lt, sched;       // lane table (int4: first record, contacts, first phase's place, 2 * phases + 1 if narrow), schedule
   __device__ ResLds(unsigned char* p, int nb, int nc, int nl) {
     body = lds_addr(p);
     rec = body + (nb + BODY_SPARE) * rec_bytes<R>();
@@ -2061,7 +2102,7 @@ template <typename R> __device__ GroupSize group_size(const Dev<R>& d, const Gro
     g.p0 = min(g.p0, a);
     p1 = max(p1, e);
     g.nph += lane_phases(e - a, d.l_ncol[l]);
-    g.wg = g.wg || (d.l_nph[l] & 1);
+    g.wg = g.wg || (d.l_nph[l] & LANE_WG);
     ++g.nl;
   }
   g.nc = g.nl ? p1 - g.p0 : 0;
@@ -2077,53 +2118,24 @@ __device__ __forceinline__ bool group_fits(const Dev<R>& d, const Group& gr, con
          ResLds<R>::bytes(nb, g.nc, g.nl, g.nph) <= ResCap<R, H>::BYTES;
 }
 
-// What a quad's lane needs of its contact: row q of J, rows 0..3 of the block
-// it updates, the old iterate, that block's inverse mass, LDS addresses.  None
-// of it changes during a sweep.
-template <typename R> struct PhaseIn {
-  V4<R> jl, ja, jb, W0, W1;
-  V3<R> v0, v1, v2, v3;
-  R xo;
+// where a contact's record is read from: LDS (resident) or global memory
+// (streaming); off: the lane's offset, k: a constant that folds into the load
+struct LdsRec {
+  int r;
+  template <typename T> __device__ __forceinline__ T get(int off, int k = 0) const { return lds_at<T>(r + off + k); }
 };
-
-// a lane's fixed part in the phases of a sweep
-template <typename R, bool JAC> struct PhaseLane {
-  int q;
-  bool side_b, ang;        // lane 0: linear A, 1: angular A, 2: linear B, 3: angular B
-  int row, blk, fo;        // offsets: row q in a record, the block's rows, the block in a body record
-  int xro, xwo;            // offsets of the old and the new iterate in a record
-  R sgn;
-  static constexpr int VB = (int)sizeof(V4<R>), FV = JAC ? F_SL * VB : F_WL * VB;
-  __device__ PhaseLane(int tid, int acc) {
-    using X = Rec<R>;
-    q = tid & 3;
-    side_b = q >= 2;
-    ang = q & 1;
-    row = q * X::ROW;
-    blk = ang ? (side_b ? 2 * VB : VB) : 0;
-    fo = ang ? VB : 0;
-    xro = (acc ? X::X1 : X::X0) + q * (int)sizeof(R);
-    xwo = (acc ? X::X0 : X::X1) + q * (int)sizeof(R);
-    sgn = side_b ? R(1) : R(-1);
+struct GlbRec {
+  const unsigned char* base;
+  unsigned r;
+  template <typename T> __device__ __forceinline__ T get(int off, int k = 0) const {
+    return *reinterpret_cast<const T*>(base + (r + (unsigned)off) + k);
   }
-  __device__ __forceinline__ int own(const int4& lc) const { return side_b ? lc.y : lc.x; }
-  __device__ __forceinline__ int wr(const int4& lc) const { return (side_b ? lc.w : lc.z) + fo; }
 };
 
-// The four velocity blocks a phase starts from and the block it updates.
-template <typename R> struct PhaseVel { V4<R> lA, aA, lB, aB, old; };
-template <typename R, bool JAC>
-__device__ __forceinline__ PhaseVel<R> phase_velocities(const PhaseLane<R, JAC>& P, int oA, int oB, int own) {
-  constexpr int FV = PhaseLane<R, JAC>::FV, VB = PhaseLane<R, JAC>::VB;
-  return PhaseVel<R>{lds_at<V4<R>>(oA + FV), lds_at<V4<R>>(oA + FV + VB), lds_at<V4<R>>(oB + FV),
-                     lds_at<V4<R>>(oB + FV + VB), lds_at<V4<R>>(own + P.fo)};
-}
-
-// One contact by one quad; lane q holds row q.  The arithmetic and its order
-// are those of update_contact, so the iterates are bitwise the same.  Returns
-// the lane's new iterate; nw: its velocity block after the update.  ISO: the
-// isotropic projection.  JAC: Jacobi reads the accepted velocity changes
-// (jacobi_solver.py:6-57), Gauss-Seidel the working ones.
+// A phase of a sweep is one contact by one quad, 16 contacts a wavefront
+// (QuadPhase), or one contact by a row of 16 lanes, 4 contacts a wavefront
+// (RowPhase); a lane of the problem is swept by one or the other throughout
+// (narrow_phases).  Both give the iterates of update_contact bit for bit.
 //
 // A phase is a serial chain: velocities from LDS, the row products, the
 // projection, the velocity update, back to LDS.  With one wavefront per SIMD
@@ -2138,104 +2150,282 @@ __device__ __forceinline__ PhaseVel<R> phase_velocities(const PhaseLane<R, JAC>&
 //  * the sign of the update (body A minus, body B plus) is applied once, at
 //    the end, and a linear update runs through the same multiply-add as an
 //    angular one (times 1/m instead of times one).
-// A phase is then ~118 instructions and ~570 cycles (0.24 us), bound by their
-// issue; with the branches, position tests and a wait for the previous phase's
-// writes it took ~1,050.  4,096 spheres, 60 colours, 50 sweeps: solve 1613 ->
-// 875 us.
-template <typename R, bool ISO, bool JAC>
-__device__ __forceinline__ R phase_update(const ProxParams& pp, const PhaseLane<R, JAC>& P, const PhaseIn<R>& c,
-                                          const PhaseVel<R>& v, R rs, bool hybrid, V4<R>& nw) {
-  // row q of z = x - r (J w + b)  (contacts.py:77-92)
-  const R Jw = row_jw(xyz(c.jl), xyz(c.ja), xyz(c.jb), xyz(v.lA), xyz(v.aA), xyz(v.lB), xyz(v.aB));
-  const R z = row_z(c.xo, c.ja.w * rs, Jw, c.jl.w);
-  // projections (contacts.py:92-95)
-  const R z0 = fmax(R(0), z);
-  const R xnrm = quad_bcast<0>(z0);
-  const R xr = (JAC && !hybrid) ? quad_bcast<0>(c.xo) : xnrm;
-  R val;
-  if constexpr (ISO) {
-    const R zz = z * z;
-    const R sq = (quad_bcast<1>(zz) + quad_bcast<2>(zz)) + quad_bcast<3>(zz);
-    val = prox_sphere_row<R>(z, sq, c.jb.w, xr);
-  } else {
-    const R z1 = quad_bcast<1>(z), z2 = quad_bcast<2>(z), z3 = quad_bcast<3>(z);
-    const R mu0 = quad_bcast<1>(c.jb.w), mu1 = quad_bcast<2>(c.jb.w), mu2 = quad_bcast<3>(c.jb.w);
-    const V3<R> o = prox_ellipsoid_call<R>(z1, z2, z3, mu0, mu1, mu2, xr, pp.ell_tol, pp.ell_expansion, pp.ell_max_iter);
-    val = P.side_b ? (P.ang ? o.z : o.y) : o.x;
+// A quad's phase is then ~118 instructions and ~570 cycles (0.24 us), bound by
+// their issue; with the branches, position tests and a wait for the previous
+// phase's writes it took ~1,050.  4,096 spheres, 60 colours, 50 sweeps: solve
+// 1613 -> 875 us.
+//
+// Most levels hold 2 to 4 contacts, so most quads idle, while a lane of a busy
+// one computes a whole block.  A row of 16 splits the same sums: a half of J w
+// per lane instead of both, one component of a block instead of three, 12
+// instead of 17 LDS reads.  A row's phase is ~80 instructions and ~440 cycles,
+// now bound by its dependent chain.  4,096 spheres, 59 phases: solve 800 -> 662
+// us; 333-sphere Jacobi pile 1761 -> 1672.  (Streamed records stay with quads:
+// a row's ten loads cover a quarter of the contacts but cost as much to issue,
+// and a shorter phase leaves less time for them; 320 scenes 966 -> 1066 us.)
+//
+// Interface: LANES per contact; In, what a lane needs of its contact and none
+// of which changes during a sweep; Loc, LDS addresses of its bodies; rows,
+// loc, bodies and masses fill In; velocities reads what a phase starts from;
+// update returns the lane's new iterate and sets nw, its part of the
+// velocities after the update, for store.  JAC: Jacobi reads the accepted
+// velocity changes (jacobi_solver.py:6-57), Gauss-Seidel the working ones.
+template <typename R, bool ISO, bool JAC> struct QuadPhase {
+  using X = Rec<R>;
+  static constexpr int LANES = 4;
+  static constexpr int VB = (int)sizeof(V4<R>), FV = JAC ? F_SL * VB : F_WL * VB;
+  using Loc = int4;
+  using Out = V4<R>;
+  struct In {
+    V4<R> jl, ja, jb, W0, W1;   // row q of J, the inverse mass of the block this lane updates
+    V3<R> v0, v1, v2, v3;       // rows 0..3 of that block
+    R xo;                       // the old iterate
+    int oA, oB, own, wr;        // LDS addresses of the bodies read, the one updated, its block's new value
+  };
+  struct Vel { V4<R> lA, aA, lB, aB, old; };
+  int q;
+  bool side_b, ang;        // lane 0: linear A, 1: angular A, 2: linear B, 3: angular B
+  int row, blk, fo;        // offsets: row q in a record, the block's rows, the block in a body record
+  int xro, xwo;            // offsets of the old and the new iterate in a record
+  R sgn;
+  __device__ QuadPhase(int tid, int acc, int) {
+    q = tid & 3;
+    side_b = q >= 2;
+    ang = q & 1;
+    row = q * X::ROW;
+    blk = ang ? (side_b ? 2 * VB : VB) : 0;
+    fo = ang ? VB : 0;
+    xro = (acc ? X::X1 : X::X0) + q * (int)sizeof(R);
+    xwo = (acc ? X::X0 : X::X1) + q * (int)sizeof(R);
+    sgn = side_b ? R(1) : R(-1);
   }
-  const R xq = P.q == 0 ? z0 : val;
-  const R dq = xq - c.xo;
-  // w += W J^T dx (contacts.py:107), this lane's block
-  const R d0 = quad_bcast<0>(dq), d1 = quad_bcast<1>(dq), d2 = quad_bcast<2>(dq), d3 = quad_bcast<3>(dq);
-  V3<R> a = {sum_first(d0 * c.v0.x), sum_first(d0 * c.v0.y), sum_first(d0 * c.v0.z)};
-  a.x = madd(d1, c.v1.x, a.x); a.y = madd(d1, c.v1.y, a.y); a.z = madd(d1, c.v1.z, a.z);
-  a.x = madd(d2, c.v2.x, a.x); a.y = madd(d2, c.v2.y, a.y); a.z = madd(d2, c.v2.z, a.z);
-  a.x = madd(d3, c.v3.x, a.x); a.y = madd(d3, c.v3.y, a.y); a.z = madd(d3, c.v3.z, a.z);
-  const R W[6] = {c.W0.x, c.W0.y, c.W0.z, c.W0.w, c.W1.x, c.W1.y};
-  const V3<R> t = sym_madd(W, a);
-  const R s = P.ang ? P.sgn : P.sgn * c.W1.z;
-  const V3<R> u = {P.ang ? t.x : a.x, P.ang ? t.y : a.y, P.ang ? t.z : a.z};
-  nw = V4<R>{madd(s, u.x, v.old.x), madd(s, u.y, v.old.y), madd(s, u.z, v.old.z), R(0)};
-  return xq;
-}
+  template <typename A> __device__ __forceinline__ Loc loc(const A& at) const { return at.template get<int4>(0, X::LOC); }
+  __device__ __forceinline__ void bodies(In& n, const Loc& lc) const {
+    n.oA = lc.x;
+    n.oB = lc.y;
+    n.own = side_b ? lc.y : lc.x;
+    n.wr = (side_b ? lc.w : lc.z) + fo;
+  }
+  template <typename A> __device__ __forceinline__ void rows(In& n, const A& at) const {
+    n.jl = at.template get<V4<R>>(row);
+    n.ja = at.template get<V4<R>>(row, VB);
+    n.jb = at.template get<V4<R>>(row, 2 * VB);
+    n.xo = at.template get<R>(xro);
+    n.v0 = xyz(at.template get<V4<R>>(blk));
+    n.v1 = xyz(at.template get<V4<R>>(blk, X::ROW));
+    n.v2 = xyz(at.template get<V4<R>>(blk, 2 * X::ROW));
+    n.v3 = xyz(at.template get<V4<R>>(blk, 3 * X::ROW));
+  }
+  __device__ __forceinline__ void masses(In& n) const {
+    n.W0 = lds_at<V4<R>>(n.own + F_W0 * VB);
+    n.W1 = lds_at<V4<R>>(n.own + F_W1 * VB);
+  }
+  __device__ __forceinline__ Vel velocities(const In& c) const {
+    return Vel{lds_at<V4<R>>(c.oA + FV), lds_at<V4<R>>(c.oA + FV + VB), lds_at<V4<R>>(c.oB + FV),
+               lds_at<V4<R>>(c.oB + FV + VB), lds_at<V4<R>>(c.own + fo)};
+  }
+  __device__ __forceinline__ R update(const ProxParams& pp, const In& c, const Vel& v, R rs, bool hybrid, Out& nw) const {
+    // row q of z = x - r (J w + b)  (contacts.py:77-92)
+    const R Jw = row_jw(xyz(c.jl), xyz(c.ja), xyz(c.jb), xyz(v.lA), xyz(v.aA), xyz(v.lB), xyz(v.aB));
+    const R z = row_z(c.xo, c.ja.w * rs, Jw, c.jl.w);
+    // projections (contacts.py:92-95)
+    const R z0 = fmax(R(0), z);
+    const R xnrm = quad_bcast<0>(z0);
+    const R xr = (JAC && !hybrid) ? quad_bcast<0>(c.xo) : xnrm;
+    R val;
+    if constexpr (ISO) {
+      const R zz = z * z;
+      const R sq = (quad_bcast<1>(zz) + quad_bcast<2>(zz)) + quad_bcast<3>(zz);
+      val = prox_sphere_row<R>(z, sq, c.jb.w, xr);
+    } else {
+      const R z1 = quad_bcast<1>(z), z2 = quad_bcast<2>(z), z3 = quad_bcast<3>(z);
+      const R mu0 = quad_bcast<1>(c.jb.w), mu1 = quad_bcast<2>(c.jb.w), mu2 = quad_bcast<3>(c.jb.w);
+      const V3<R> o = prox_ellipsoid_call<R>(z1, z2, z3, mu0, mu1, mu2, xr, pp.ell_tol, pp.ell_expansion, pp.ell_max_iter);
+      val = side_b ? (ang ? o.z : o.y) : o.x;
+    }
+    const R xq = q == 0 ? z0 : val;
+    const R dq = xq - c.xo;
+    // w += W J^T dx (contacts.py:107), this lane's block
+    const R d0 = quad_bcast<0>(dq), d1 = quad_bcast<1>(dq), d2 = quad_bcast<2>(dq), d3 = quad_bcast<3>(dq);
+    V3<R> a = {sum_first(d0 * c.v0.x), sum_first(d0 * c.v0.y), sum_first(d0 * c.v0.z)};
+    a.x = madd(d1, c.v1.x, a.x); a.y = madd(d1, c.v1.y, a.y); a.z = madd(d1, c.v1.z, a.z);
+    a.x = madd(d2, c.v2.x, a.x); a.y = madd(d2, c.v2.y, a.y); a.z = madd(d2, c.v2.z, a.z);
+    a.x = madd(d3, c.v3.x, a.x); a.y = madd(d3, c.v3.y, a.y); a.z = madd(d3, c.v3.z, a.z);
+    const R W[6] = {c.W0.x, c.W1.x, c.W1.z, c.W0.y, c.W0.z, c.W1.y};   // (xx, yy, zz, xy, xz, yz)
+    const V3<R> t = sym_madd(W, a);
+    const R s = ang ? sgn : sgn * c.W0.w;
+    const V3<R> u = {ang ? t.x : a.x, ang ? t.y : a.y, ang ? t.z : a.z};
+    nw = V4<R>{madd(s, u.x, v.old.x), madd(s, u.y, v.old.y), madd(s, u.z, v.old.z), R(0)};
+    return xq;
+  }
+  __device__ __forceinline__ void store(const In& c, const Out& nw) const { lds_at<V4<R>>(c.wr) = nw; }
+  // where the lane's new iterate goes in LDS
+  __device__ __forceinline__ int x_addr(int r) const { return r + xwo; }
+};
+
+// Quad b of a row of 16 lanes updates block b (linear A, angular A, linear B,
+// angular B), its lane c component c.  Before that the lanes of the two side-A
+// quads sum side A's half of row c's J w, those of the side-B quads side B's,
+// which take the others' sums and go on to row c's projection; the side-A
+// quads compute along on values that nothing uses, and their iterates and the
+// fourth lanes' velocities are stored in the spare body record.
+template <typename R, bool ISO, bool JAC> struct RowPhase {
+  using X = Rec<R>;
+  static constexpr int LANES = 16;
+  static constexpr int SR = (int)sizeof(R), VB = (int)sizeof(V4<R>), FV = JAC ? F_SL * VB : F_WL * VB;
+  using Loc = int2;        // the lane's side: body to read, body to write
+  using Out = R;
+  struct In {
+    V4<R> jl, js;          // row c of J: linear part and this side's angular one
+    R r, xo;               // of row c: r0, the old iterate
+    R v0, v1, v2, v3;      // component c of rows 0..3 of the block
+    R w0, w1, w2;          // row c of I^-1 (linear blocks: w0 = 1/m)
+    int own, wr;           // LDS addresses of the body, of the component's new value
+  };
+  struct Vel { V4<R> l, a; R old; };
+  int c;
+  bool ang;
+  int row, jso, blk, loc_o, fo, wf, wp;   // offsets
+  int xro, xadd;
+  unsigned wmul, xmul;     // 1: store, 0: store in the spare record
+  int wadd;
+  R sgn;
+  __device__ RowPhase(int tid, int acc, int body) {
+    c = tid & 3;
+    const int b = (tid >> 2) & 3;
+    const bool side_b = b >= 2;
+    ang = b & 1;
+    row = c * X::ROW;
+    jso = row + (side_b ? 2 * VB : VB);
+    blk = (ang ? (side_b ? 2 * VB : VB) : 0) + c * SR;
+    loc_o = X::LOC + (side_b ? 4 : 0);
+    fo = (ang ? VB : 0) + c * SR;
+    wf = F_W0 * VB + (ang ? (c < 3 ? c : 0) : 3) * SR;
+    wp = F_W0 * VB + (c == 1 ? 4 : c == 2 ? 5 : 1) * SR;
+    const int spare = body + rec_bytes<R>();
+    wmul = c < 3 ? 1u : 0u;
+    wadd = c < 3 ? fo : spare;
+    xro = (acc ? X::X1 : X::X0) + c * SR;
+    xmul = b == 2 ? 1u : 0u;
+    xadd = b == 2 ? (acc ? X::X0 : X::X1) + c * SR : spare;
+    sgn = side_b ? R(1) : R(-1);
+    // (factors the compiler does not see through: one multiply-add an address, not a mask, a select and an add)
+    asm("" : "+v"(wmul), "+v"(xmul));
+  }
+  template <typename A> __device__ __forceinline__ Loc loc(const A& at) const {
+    return make_int2(at.template get<int>(loc_o), at.template get<int>(loc_o, 8));
+  }
+  __device__ __forceinline__ void bodies(In& n, const Loc& lc) const {
+    n.own = lc.x;
+    n.wr = (int)(__umul24((unsigned)lc.y, wmul) + (unsigned)wadd);
+  }
+  template <typename A> __device__ __forceinline__ void rows(In& n, const A& at) const {
+    n.jl = at.template get<V4<R>>(row);
+    n.js = at.template get<V4<R>>(jso);
+    n.r = at.template get<R>(row, VB + 3 * SR);
+    n.xo = at.template get<R>(xro);
+    n.v0 = at.template get<R>(blk);
+    n.v1 = at.template get<R>(blk, X::ROW);
+    n.v2 = at.template get<R>(blk, 2 * X::ROW);
+    n.v3 = at.template get<R>(blk, 3 * X::ROW);
+  }
+  __device__ __forceinline__ void masses(In& n) const {
+    n.w0 = lds_at<R>(n.own + wf);
+    n.w1 = lds_at<R>(n.own + wp);
+    n.w2 = lds_at<R>(n.own + wp + SR);
+  }
+  __device__ __forceinline__ Vel velocities(const In& k) const {
+    return Vel{lds_at<V4<R>>(k.own + FV), lds_at<V4<R>>(k.own + FV + VB), lds_at<R>(k.own + fo)};
+  }
+  __device__ __forceinline__ R update(const ProxParams& pp, const In& k, const Vel& v, R rs, bool hybrid, Out& nw) const {
+    // this side's half of row c of J w, then the row on the side-B quads (row_jw's sums in its order)
+    R Jw;
+    if constexpr (sizeof(R) == 8) {
+      const R lw = dot(xyz(k.jl), xyz(v.l)), aw = dot(xyz(k.js), xyz(v.a));
+      Jw = row_other_half(-lw - aw) + lw + aw;
+    } else {
+      R h = k.jl.x * v.l.x;
+      h = madd(k.jl.y, v.l.y, h); h = madd(k.jl.z, v.l.z, h);
+      h = madd(k.js.x, v.a.x, h); h = madd(k.js.y, v.a.y, h); h = madd(k.js.z, v.a.z, h);
+      Jw = h - row_other_half(h);
+    }
+    const R z = row_z(k.xo, k.r * rs, Jw, k.jl.w);
+    const R z0 = fmax(R(0), z);
+    const R xnrm = quad_bcast<0>(z0);
+    const R xr = (JAC && !hybrid) ? quad_bcast<0>(k.xo) : xnrm;
+    R val;
+    if constexpr (ISO) {
+      const R zz = z * z;
+      const R sq = (quad_bcast<1>(zz) + quad_bcast<2>(zz)) + quad_bcast<3>(zz);
+      val = prox_sphere_row<R>(z, sq, k.js.w, xr);
+    } else {
+      const R z1 = row_bcast<9>(z), z2 = row_bcast<10>(z), z3 = row_bcast<11>(z);
+      const R mu0 = row_bcast<9>(k.js.w), mu1 = row_bcast<10>(k.js.w), mu2 = row_bcast<11>(k.js.w);
+      const V3<R> o = prox_ellipsoid_call<R>(z1, z2, z3, mu0, mu1, mu2, row_bcast<8>(xr), pp.ell_tol, pp.ell_expansion,
+                                             pp.ell_max_iter);
+      val = c == 3 ? o.z : c == 2 ? o.y : o.x;
+    }
+    const R xq = c == 0 ? z0 : val;
+    const R dq = xq - k.xo;
+    // component c of the block's update
+    R a = sum_first(row_bcast<8>(dq) * k.v0);
+    a = madd(row_bcast<9>(dq), k.v1, a);
+    a = madd(row_bcast<10>(dq), k.v2, a);
+    a = madd(row_bcast<11>(dq), k.v3, a);
+    const R t = madd(k.w2, quad_bcast<2>(a), madd(k.w1, quad_bcast<1>(a), k.w0 * quad_bcast<0>(a)));
+    nw = madd(ang ? sgn : sgn * k.w0, ang ? t : a, v.old);
+    return xq;
+  }
+  __device__ __forceinline__ void store(const In& k, const Out& nw) const { lds_at<R>(k.wr) = nw; }
+  __device__ __forceinline__ int x_addr(int r) const { return (int)(__umul24((unsigned)r, xmul) + (unsigned)xadd); }
+};
 
 // ---- resident layout: everything a sweep touches in LDS
 
-// One sweep of one resident lane by one wavefront, one contact per quad and
-// phase.  Rows, inverse masses and iterates are read one phase ahead, the
-// bodies' addresses two ahead and the schedule three ahead.
-template <typename R, bool ISO, bool JAC>
+// One sweep of one resident lane by one wavefront.  Rows, inverse masses and
+// iterates are read one phase ahead, the bodies' addresses two ahead and the
+// schedule three ahead.
+template <typename R, typename P>
 __device__ double res_sweep(const ProxParams& pp, const ResLds<R>& L, int4 lt, bool hybrid, int acc, R rs, int lane) {
   using X = Rec<R>;
-  constexpr int VB = (int)sizeof(V4<R>);
-  struct In : PhaseIn<R> { int oA, oB, own, wr, xw; };
+  constexpr int STEP = 2 * (64 / P::LANES);   // bytes of a phase of the schedule
+  struct In : P::In { int xw; };
   const int rec0 = __builtin_amdgcn_readfirstlane(lt.x), K = __builtin_amdgcn_readfirstlane(lt.y);
-  const int nph = __builtin_amdgcn_readfirstlane(lt.w);
+  const int nph = __builtin_amdgcn_readfirstlane(lt.w) >> 1;
   if (nph <= 0) return 0.0;
-  const PhaseLane<R, JAC> P(lane, acc);
-  int sp = L.sched + __builtin_amdgcn_readfirstlane(lt.z) * PHASE_B + 2 * (lane >> 2);
-  auto entry = [&](int ahead) { return (int)lds_at<unsigned short>(sp + ahead * PHASE_B) * 16; };
-  auto load = [&](int r, const int4& lc, In& p) {
-    const int rr = r + P.row, rb = r + P.blk;
-    p.jl = lds_at<V4<R>>(rr);
-    p.ja = lds_at<V4<R>>(rr + VB);
-    p.jb = lds_at<V4<R>>(rr + 2 * VB);
-    p.xo = lds_at<R>(r + P.xro);
-    p.v0 = xyz(lds_at<V4<R>>(rb));
-    p.v1 = xyz(lds_at<V4<R>>(rb + X::ROW));
-    p.v2 = xyz(lds_at<V4<R>>(rb + 2 * X::ROW));
-    p.v3 = xyz(lds_at<V4<R>>(rb + 3 * X::ROW));
-    p.own = P.own(lc);
-    p.W0 = lds_at<V4<R>>(p.own + F_W0 * VB);
-    p.W1 = lds_at<V4<R>>(p.own + F_W1 * VB);
-    p.oA = lc.x;
-    p.oB = lc.y;
-    p.wr = P.wr(lc);
-    p.xw = r + P.xwo;
+  const P ph(lane, acc, L.body);
+  int sp = L.sched + __builtin_amdgcn_readfirstlane(lt.z) * PHASE_B + 2 * (lane / P::LANES);
+  auto entry = [&](int ahead) { return (int)lds_at<unsigned short>(sp + ahead * STEP) * 16; };
+  auto load = [&](int r, const typename P::Loc& lc, In& p) {
+    const LdsRec at{r};
+    ph.bodies(p, lc);
+    ph.rows(p, at);
+    ph.masses(p);
+    p.xw = ph.x_addr(r);
   };
   int r1 = entry(1), e2 = entry(2);
   In pa, pb;
-  int4 lc1;
+  typename P::Loc lc1;
   {
     const int r0 = entry(0);
-    const int4 lc0 = lds_at<int4>(r0 + X::LOC);
-    lc1 = lds_at<int4>(r1 + X::LOC);
+    const typename P::Loc lc0 = ph.loc(LdsRec{r0});
+    lc1 = ph.loc(LdsRec{r1});
     load(r0, lc0, pa);
   }
   // the reads above are done when the loop starts: a wait inside it would
   // also wait for the previous phase's writes
   __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0)
   auto phase = [&](const In& c, In& n) {
-    const PhaseVel<R> v = phase_velocities<R, JAC>(P, c.oA, c.oB, c.own);
+    const typename P::Vel v = ph.velocities(c);
     load(r1, lc1, n);
     const int r2 = e2;
-    lc1 = lds_at<int4>(r2 + X::LOC);
+    lc1 = ph.loc(LdsRec{r2});
     e2 = entry(3);
     r1 = r2;
-    sp += PHASE_B;
-    V4<R> nw;
-    const R xq = phase_update<R, ISO, JAC>(pp, P, c, v, rs, hybrid, nw);
-    lds_at<V4<R>>(c.wr) = nw;
+    sp += STEP;
+    typename P::Out nw;
+    const R xq = ph.update(pp, c, v, rs, hybrid, nw);
+    ph.store(c, nw);
     lds_at<R>(c.xw) = xq;
     phase_sync<64>();
   };
@@ -2248,19 +2438,27 @@ __device__ double res_sweep(const ProxParams& pp, const ResLds<R>& L, int4 lt, b
   // the merit, max |x_new - x_old| in FP64 (a sweep updates each contact once)
   // 64 contacts per pass, their reads in flight together (past the last
   // contact the last one again)
+  const int xr = (acc ? X::X1 : X::X0) + (lane & 3) * (int)sizeof(R), xw = X::X0 + X::X1 + 2 * (lane & 3) * (int)sizeof(R) - xr;
   double m = 0.0;
   for (int i = lane >> 2; i - (lane >> 2) < K; i += 4 * PHASE_Q) {
     R xn[4], xo[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const int r = rec0 + min(i + u * PHASE_Q, K - 1) * X::BYTES;
-      xn[u] = lds_at<R>(r + P.xwo);
-      xo[u] = lds_at<R>(r + P.xro);
+      xn[u] = lds_at<R>(r + xw);
+      xo[u] = lds_at<R>(r + xr);
     }
 #pragma unroll
     for (int u = 0; u < 4; ++u) m = fmax(m, fabs((double)xn[u] - (double)xo[u]));
   }
   return m;
+}
+
+template <typename R, bool ISO, bool JAC>
+__device__ __forceinline__ double res_sweep_lane(const ProxParams& pp, const ResLds<R>& L, int4 lt, bool hybrid, int acc,
+                                                 R rs, int lane) {
+  return lt.w & 1 ? res_sweep<R, RowPhase<R, ISO, JAC>>(pp, L, lt, hybrid, acc, rs, lane)
+                  : res_sweep<R, QuadPhase<R, ISO, JAC>>(pp, L, lt, hybrid, acc, rs, lane);
 }
 
 // what a group's sweeps are decided with, the same for every sweep
@@ -2293,7 +2491,9 @@ template <typename R> __device__ void stage_bodies(const Dev<R>& d, const BodyLd
   for (int i = threadIdx.x; i < nb; i += blockDim.x) {
     const int b = d.u_blist[b0 + i];
     B.wl[i] = d.ww0[b]; B.wa[i] = d.ww1[b]; B.sl[i] = d.ws0[b]; B.sa[i] = d.ws1[b];
-    B.W0[i] = d.b_W0[b]; B.W1[i] = d.b_W1[b];
+    const V4<R> w0 = d.b_W0[b], w1 = d.b_W1[b];   // (xx, yy, zz, xy), (xz, yz, 1/m, 0)
+    B.W0[i] = V4<R>{w0.x, w0.w, w1.x, w1.z};
+    B.W1[i] = V4<R>{w0.y, w1.y, w0.z, R(0)};
   }
   if (threadIdx.x < BODY_SPARE) {
     const V4<R> z = {R(0), R(0), R(0), R(0)};
@@ -2369,18 +2569,20 @@ __device__ void solve_group_resident(const Dev<R>& d, const int slot, const Grou
     const int4 lt = lds_at<int4>(L.lt + 16 * t);
     const int nc = d.l_ncol[lt.w];
     const int* co = lane_coff(d, lt.w);
-    int ph = lt.z;
+    const bool rows16 = d.l_nph[lt.w] & LANE_NARROW;
+    const int per = rows16 ? PHASE_R : PHASE_Q;
+    int ph = 0;
     for (int c0 = 0; c0 < nc; c0 += 64) {
       const int c = c0 + lane;
       const int lo = c < nc ? co[c] : 0, w = c < nc ? co[c + 1] - lo : 0;
-      const int np = (w + PHASE_Q - 1) / PHASE_Q;
+      const int np = (w + per - 1) / per;
       const int inc = wave_inclusive_sum(np);
-      const int s0 = L.sched + (ph + inc - np) * PHASE_B;
+      const int s0 = L.sched + lt.z * PHASE_B + (ph + inc - np) * 2 * per;
       for (int i = 0; i < w; ++i)   // (slots of one phase are consecutive, and so are its phases)
         lds_at<unsigned short>(s0 + 2 * i) = (unsigned short)((lt.x + (lo + i) * X::BYTES) / 16);
       ph += __shfl(inc, 63, 64);
     }
-    if (lane == 0) lds_at<int>(L.lt + 16 * t + 12) = ph - lt.z;
+    if (lane == 0) lds_at<int>(L.lt + 16 * t + 12) = ph << 1 | (rows16 ? 1 : 0);
   }
   __syncthreads();
   const Decide<R> by(d, sp, gr.lead, gs.nl <= 1);
@@ -2394,11 +2596,11 @@ __device__ void solve_group_resident(const Dev<R>& d, const int slot, const Grou
       const int4 lt = lds_at<int4>(L.lt + 16 * t);
       double ml;
       if (jacobi)
-        ml = iso ? res_sweep<R, true, true>(pp, L, lt, hybrid, ctl.acc, rs, lane)
-                 : res_sweep<R, false, true>(pp, L, lt, hybrid, ctl.acc, rs, lane);
+        ml = iso ? res_sweep_lane<R, true, true>(pp, L, lt, hybrid, ctl.acc, rs, lane)
+                 : res_sweep_lane<R, false, true>(pp, L, lt, hybrid, ctl.acc, rs, lane);
       else
-        ml = iso ? res_sweep<R, true, false>(pp, L, lt, hybrid, ctl.acc, rs, lane)
-                 : res_sweep<R, false, false>(pp, L, lt, hybrid, ctl.acc, rs, lane);
+        ml = iso ? res_sweep_lane<R, true, false>(pp, L, lt, hybrid, ctl.acc, rs, lane)
+                 : res_sweep_lane<R, false, false>(pp, L, lt, hybrid, ctl.acc, rs, lane);
       m = fmax(m, ml);
     }
     const int dec = sweep_decide<R, COOP>(d, by, ctl, m, it, sh_red, s_ok, B, nb, abort);
@@ -2437,13 +2639,13 @@ __device__ void solve_group_resident(const Dev<R>& d, const int slot, const Grou
 template <typename R, bool ISO, bool JAC, bool WG>
 __device__ double stream_sweep(const Dev<R>& d, const ProxParams& pp, int l, bool hybrid, int acc, R rs, int tid) {
   using X = Rec<R>;
-  constexpr int VB = (int)sizeof(V4<R>);
-  struct In : PhaseIn<R> { int4 lc; unsigned off; };
+  using P = QuadPhase<R, ISO, JAC>;
+  struct In : P::In { typename P::Loc lc; unsigned off; };
   const int p0 = __builtin_amdgcn_readfirstlane(d.l_start[l]);
-  const int nph = __builtin_amdgcn_readfirstlane(d.l_nph[l]) >> 1;
+  const int nph = __builtin_amdgcn_readfirstlane(d.l_nph[l]) >> LANE_BITS;
   if (nph <= 0) return 0.0;
-  const int j = tid >> 2, lane = tid & 63;
-  const PhaseLane<R, JAC> P(tid, acc);
+  const int j = tid / P::LANES, lane = tid & 63;
+  const P ph(tid, acc, 0);
   unsigned char* const rec = d.s_rec;
   const unsigned nul = (unsigned)d.cap_contacts * (unsigned)X::BYTES;
   // the list, 64 phases at a time (lane i holds phase i of the run), the next run read ahead
@@ -2455,21 +2657,13 @@ __device__ double stream_sweep(const Dev<R>& d, const ProxParams& pp, int l, boo
     const unsigned e = p < nph ? (unsigned)__builtin_amdgcn_readlane((int)run, p & 63) : 0u;
     const unsigned pos = e >> PHASE_BITS, cnt = e & ((1u << PHASE_BITS) - 1u);
     n.off = (unsigned)j < cnt ? ((unsigned)p0 + pos + (unsigned)j) * (unsigned)X::BYTES : nul;
-    n.lc = *reinterpret_cast<const int4*>(rec + n.off + X::LOC);
-    const unsigned rr = n.off + P.row, rb = n.off + P.blk;
-    n.jl = *reinterpret_cast<const V4<R>*>(rec + rr);
-    n.ja = *reinterpret_cast<const V4<R>*>(rec + rr + VB);
-    n.jb = *reinterpret_cast<const V4<R>*>(rec + rr + 2 * VB);
-    n.xo = *reinterpret_cast<const R*>(rec + n.off + P.xro);
-    n.v0 = xyz(*reinterpret_cast<const V4<R>*>(rec + rb));
-    n.v1 = xyz(*reinterpret_cast<const V4<R>*>(rec + rb + X::ROW));
-    n.v2 = xyz(*reinterpret_cast<const V4<R>*>(rec + rb + 2 * X::ROW));
-    n.v3 = xyz(*reinterpret_cast<const V4<R>*>(rec + rb + 3 * X::ROW));
+    const GlbRec at{rec, n.off};
+    n.lc = ph.loc(at);
+    ph.rows(n, at);
   };
   auto masses = [&](In& n) {
-    const int own = P.own(n.lc);
-    n.W0 = lds_at<V4<R>>(own + F_W0 * VB);
-    n.W1 = lds_at<V4<R>>(own + F_W1 * VB);
+    ph.bodies(n, n.lc);
+    ph.masses(n);
   };
   double m = 0.0;
   In a, b, c;
@@ -2478,13 +2672,13 @@ __device__ double stream_sweep(const Dev<R>& d, const ProxParams& pp, int l, boo
   masses(a);
   int p = 0;
   auto phase = [&](In& cur, In& nxt, In& fill) {
-    const PhaseVel<R> v = phase_velocities<R, JAC>(P, cur.lc.x, cur.lc.y, P.own(cur.lc));
+    const typename P::Vel v = ph.velocities(cur);
     masses(nxt);
     fetch(p + 2, fill);
-    V4<R> nw;
-    const R xq = phase_update<R, ISO, JAC>(pp, P, cur, v, rs, hybrid, nw);
-    lds_at<V4<R>>(P.wr(cur.lc)) = nw;
-    if (cur.off != nul) *reinterpret_cast<R*>(rec + cur.off + P.xwo) = xq;
+    typename P::Out nw;
+    const R xq = ph.update(pp, cur, v, rs, hybrid, nw);
+    ph.store(cur, nw);
+    if (cur.off != nul) *reinterpret_cast<R*>(rec + cur.off + ph.xwo) = xq;
     m = fmax(m, fabs((double)xq - (double)cur.xo));
     if (WG) __syncthreads();
     else phase_sync<64>();
@@ -2507,11 +2701,11 @@ __device__ double stream_lanes(const Dev<R>& d, const ProxParams& pp, const Grou
   double m = 0.0;
   int t = 0;
   for (int l = gr.l_lo; l < gr.l_hi; ++l) {
-    if (d.l_end[l] <= d.l_start[l] || (d.l_nph[l] & 1)) continue;
+    if (d.l_end[l] <= d.l_start[l] || (d.l_nph[l] & LANE_WG)) continue;
     if (t++ % nwave == wave) m = fmax(m, stream_sweep<R, ISO, JAC, false>(d, pp, l, hybrid, acc, rs, lane));
   }
   for (int l = gr.l_lo; l < gr.l_hi; ++l) {   // lanes swept by the workgroup
-    if (d.l_end[l] <= d.l_start[l] || !(d.l_nph[l] & 1)) continue;
+    if (d.l_end[l] <= d.l_start[l] || !(d.l_nph[l] & LANE_WG)) continue;
     m = fmax(m, stream_sweep<R, ISO, JAC, true>(d, pp, l, hybrid, acc, rs, (int)threadIdx.x));
   }
   return m;

@@ -108,3 +108,35 @@ def test_sweep_order_bitwise_fp32(bank, n, scheme):
             for a, b in zip(got, ref):
                 assert np.array_equal(a, b), (tuning, flags)
     assert len(c["ia"]) > 30 * n
+
+
+@pytest.mark.parametrize("n", [3, 4, 5, 8, 9])
+@pytest.mark.parametrize("friction", ["isotropic", "anisotropic"])
+@pytest.mark.parametrize("scheme", ["parallel_gauss_seidel", "parallel_jacobi_hybrid"])
+def test_row_phases(bank, n, friction, scheme):
+    """Levels of 4 contacts are swept with 16 lanes a contact, of 5 with 4: FP64 against the oracle, FP32 resident
+    against streamed records (always 4 lanes) bit for bit.  (A sphere gives about 58 contacts, a box 4 to 8.)"""
+    params = dict(max_iterations=12, proximal_solver=scheme, friction_model=friction)
+    eng = row_of_boxes(bank, n, dict(params, precision="fp64"))
+    if friction == "anisotropic":
+        eng.surfaces_interactions.storage[("default", "default")].mu = np.array([0.5, 0.3, 0.05])
+    sc = OS.from_engine(eng)
+    out = OST.step(sc, 0.01)
+    c, state, lg = step_with(eng, dict(unit_size=1024, lanes_per_scene=1), native.STEP_FORCE_SINGLE, "fp64")
+    assert assert_fp64_parity(c, state, lg, out, sc)
+    eng = row_of_boxes(bank, n, dict(params, precision="fp32"))
+    sphere = bank.get("sphere_shape", lambda: MESH.create_sphere(0.5, 16, 16))
+    for i in range(3):
+        scenes.add_body(eng, "s%d" % i, sphere, np.array([4.0 * i, 0.45, 9.0]), q=Q.identity(), v=np.array([0.3, -0.2, 0.1]))
+    if friction == "anisotropic":
+        eng.surfaces_interactions.storage[("default", "default")].mu = np.array([0.5, 0.3, 0.05])
+    ref = None
+    for tuning in (dict(), dict(resident_contacts=64)):
+        for lanes in (1, 2):
+            for flags in (native.STEP_FORCE_SINGLE, native.STEP_FORCE_MULTI):
+                t = dict(tuning, unit_size=1024, lanes_per_scene=lanes)
+                c, state, lg = step_with(eng, t, flags, "fp32", steps=2)
+                got = [c["impulse"], lg["residuals"], np.float64(lg["natural_residual"])] + list(state)
+                ref = ref or got
+                for a, b in zip(got, ref):
+                    assert np.array_equal(a, b), (t, flags)
