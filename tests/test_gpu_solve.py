@@ -140,3 +140,17 @@ def test_row_phases(bank, n, friction, scheme):
                 ref = ref or got
                 for a, b in zip(got, ref):
                     assert np.array_equal(a, b), (t, flags)
+
+
+@pytest.mark.parametrize("mu", [(0.5, 0.3, 0.05), (0.0, 0.4, 0.1), (0.6, 0.0, 0.0), (0.3, 0.3, 0.3), (0.0, 0.0, 0.0)])
+def test_ellipsoid_fp64(bank, mu):
+    """The ellipsoid's bisection, with axes of length zero among them, in boxes pressed sideways and spinning."""
+    eng = row_of_boxes(bank, 6, dict(precision="fp64", max_iterations=25, friction_model="anisotropic"))
+    eng.surfaces_interactions.storage[("default", "default")].mu = np.array(mu)
+    for i, b in enumerate(eng.bodies.values()):
+        if not b.is_fixed:
+            b.v, b.w = np.array([2.0 - i, -1.0, 0.3 * i]), np.array([0.2, 3.0 - i, 0.1])
+    sc = OS.from_engine(eng)
+    out = OST.step(sc, 0.01)
+    c, state, lg = step_with(eng, dict(), native.STEP_FORCE_SINGLE, "fp64")
+    assert assert_fp64_parity(c, state, lg, out, sc)
