@@ -1230,13 +1230,16 @@ template <typename R> int scene_statics(rbh_ctx* c, const rbh_scene_desc* d, con
                       {&c->b_damp, dp.data(), sizeof(V4<R>)}, {&c->b_broad, bb.data(), sizeof(int4)},
                       {&c->r, z.data(), sizeof(V4<R>)}, {&c->q, qid.data(), sizeof(V4<R>)},
                       {&c->v, z.data(), sizeof(V4<R>)}, {&c->w, z.data(), sizeof(V4<R>)}};
-  static_assert(sizeof(puts) / sizeof(puts[0]) <= MOVE_MAX, "one transfer");
+  static_assert(sizeof(puts) / sizeof(puts[0]) < MOVE_MAX, "one transfer");
   Transfer t(c);
   for (const Put& p : puts) t.add((char*)p.b->p + p.el * s.body_off, p.el * n);
+  t.add(reinterpret_cast<SceneState*>(c->d_ss.p) + slot, sizeof(SceneState));
   int rc = t.reserve();
   if (rc) return rc;
   int j = 0;
   for (const Put& p : puts) std::memcpy(t.host<unsigned char>(j++), p.src, p.el * n);
+  const SceneState st{};
+  std::memcpy(t.host<unsigned char>(j), &st, sizeof(st));
   return t.up();
 }
 
@@ -1502,7 +1505,6 @@ int rbh_sdf_build(rbh_ctx* c, const double* V, int nv, const int* T, int nt, con
   const SdfLayout lay(nv, nt, n, sdf_pruned(V, nv, nt, mn, mx, n));
   if (lay.total > c->sdf_buf_bytes) {
     if (c->sdf_buf) (void)hipFree(c->sdf_buf);
-  if (c->pin) (void)hipHostFree(c->pin);
     c->sdf_buf = nullptr;
     c->sdf_buf_bytes = 0;
     HIPCHK(c, hipMalloc(reinterpret_cast<void**>(&c->sdf_buf), lay.total));
@@ -1694,9 +1696,6 @@ int rbh_scene_create(rbh_ctx* c, const rbh_scene_desc* d, int* scene_id) {
   c->scenes_dirty = true;
   c->hinges_dirty = true;
   if ((rc = sync_scenes(c))) return rc;
-  SceneState z{};
-  HIPCHK(c, hipMemcpyAsync(reinterpret_cast<SceneState*>(c->d_ss.p) + slot, &z, sizeof(z), hipMemcpyHostToDevice,
-                           c->stream));
   rc = c->prec == 4 ? scene_statics<float>(c, d, s, slot) : scene_statics<double>(c, d, s, slot);
   if (rc) return rc;
   c->arena_gen++;

@@ -40,3 +40,23 @@ def test_state_round_trip(precision, count, n):
             assert ctx.get_log(sid, 4)["step_index"] == 7 + i
     finally:
         ctx.close()
+
+
+def test_scene_after_larger_sdf_build():
+    """A signed-distance build whose buffer grows between two scenes of one context leaves the transfers alone."""
+    bank = scenes.ShapeBank(resolution=16)
+    eng = scenes.new_engine(bank, dict(precision="fp64"))
+    scenes.add_ground(eng, bank)
+    ctx = native.Context(0, "fp64")
+    try:
+        V, T = MESH.create_sphere(0.5, 16, 16)
+        for resolution in (8, 24, 48):
+            ctx.sdf_build(V, T, V.min(0) - 0.2, V.max(0) + 0.2, resolution, resolution, resolution)
+            desc, keep = engine_desc(eng, ctx)
+            sid = ctx.scene_create(desc)
+            st = [np.full((1, d), float(resolution)) for d in (3, 4, 3, 3)]
+            ctx.set_state(sid, *st)
+            for a, b in zip(ctx.get_state(sid, 1), st):
+                assert np.array_equal(a, b)
+    finally:
+        ctx.close()
