@@ -459,6 +459,76 @@ __device__ __forceinline__ void wave_sync_lds() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// An integer carried in the unused w of a staged box
+__device__ __forceinline__ float box_tag(float, int i) { return __int_as_float(i); }
+__device__ __forceinline__ int box_tag_of(float w) { return __float_as_int(w); }
+__device__ __forceinline__ double box_tag(double, int i) { return (double)i; }
+__device__ __forceinline__ int box_tag_of(double w) { return (int)w; }
+
+constexpr int CAND_XQ = CAND_BLK / 64;   // positions of a block per lane
+
+// The lane's NQ positions still to test against the staged run, all of them
+// per staged box: one loop over the staged clusters and their triangles,
+// uniform over the wavefront (every lane reads the same LDS entry, a
+// broadcast).  A cluster is skipped when no position of the wavefront meets
+// its box.  (A loop per position, each walking the clusters its own box meets,
+// diverged across the lanes and repeated the staged reads for each of the
+// positions.)
+template <int NQ, typename R>
+__device__ __forceinline__ void cand_test_run(const V3<R>* xl, const V3<R>* xh, unsigned live, unsigned& flg,
+                                              unsigned long long& cnt, bool count_all, int ncl, const V4<R>* lo_s,
+                                              const V4<R>* hi_s, const V4<R>* clo_s, const V4<R>* chi_s,
+                                              const int2* crange_s) {
+  for (int k = 0; k < ncl; ++k) {
+    const unsigned want = count_all ? live : (live & ~flg);
+    if (!__ballot(want != 0u)) break;                 // every position decided
+    const V4<R> cl = clo_s[k], ch = chi_s[k];
+    unsigned mk = 0;                                  // positions that meet the cluster box
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+      const V4<R> lo{xl[q].x, xl[q].y, xl[q].z, R(0)}, hi{xh[q].x, xh[q].y, xh[q].z, R(0)};
+      if (((want >> q) & 1u) && box_overlap(lo, hi, cl, ch)) mk |= 1u << q;
+    }
+    if (!__ballot(mk != 0u)) continue;
+    const int2 rg = crange_s[k];
+    const int end = rg.x + rg.y;
+    // four staged boxes per pass, loaded together (indexes clamped into
+    // the cluster's run; a clamped repeat is not tested)
+    for (int e = rg.x; e < end; e += 4) {
+      V4<R> sl[4], sh[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int ej = min(e + j, end - 1);
+        sl[j] = lo_s[ej]; sh[j] = hi_s[ej];
+      }
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) {
+        if (!((mk >> q) & 1u)) continue;
+        const V4<R> lo{xl[q].x, xl[q].y, xl[q].z, R(0)}, hi{xh[q].x, xh[q].y, xh[q].z, R(0)};
+        unsigned hit = 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) hit |= (box_overlap(lo, hi, sl[j], sh[j]) & (e + j < end)) ? 1u << j : 0u;
+        if (hit) {
+          flg |= 1u << q;
+          if (count_all) cnt += __popc(hit);
+          else mk &= ~(1u << q);                      // decided: no further test
+        }
+      }
+      if (!count_all && !__ballot(mk != 0u)) break;
+    }
+  }
+}
+
+template <typename R>
+__device__ __forceinline__ void cand_test(int nq, const V3<R>* xl, const V3<R>* xh, unsigned live, unsigned& flg,
+                                          unsigned long long& cnt, bool count_all, int ncl, const V4<R>* lo_s,
+                                          const V4<R>* hi_s, const V4<R>* clo_s, const V4<R>* chi_s,
+                                          const int2* crange_s) {
+  if (nq == 1) cand_test_run<1>(xl, xh, live, flg, cnt, count_all, ncl, lo_s, hi_s, clo_s, chi_s, crange_s);
+  else if (nq == 2) cand_test_run<2>(xl, xh, live, flg, cnt, count_all, ncl, lo_s, hi_s, clo_s, chi_s, crange_s);
+  else cand_test_run<CAND_XQ>(xl, xh, live, flg, cnt, count_all, ncl, lo_s, hi_s, clo_s, chi_s, crange_s);
+}
+
 // Flags of X's positions [x0, x1) (one block) w.r.t. Y: a position is a
 // candidate iff its triangle box meets one of Y's triangle boxes.  The
 // block's positions stay in registers (CAND_BLK / 64 per lane) while Y's
@@ -471,7 +541,7 @@ template <typename R>
 __device__ int cand_block(const Dev<R>& d, int X, int Y, int4 gX, int4 gY, int slot_base, int x0, int x1,
                           bool count_all, bool exact, V4<R>* lo_s, V4<R>* hi_s, V4<R>* clo_s, V4<R>* chi_s,
                           int2* crange_s, unsigned long long& overlaps) {
-  constexpr int XQ = CAND_BLK / 64;
+  constexpr int XQ = CAND_XQ;
   const int cap = CandLds<R>::CAP;
   const int lane = threadIdx.x & 63;
   // gX, gY: the bodies' b_broad records (first triangle box, shape nt and t_off, scene slot)
@@ -514,6 +584,46 @@ __device__ int cand_block(const Dev<R>& d, int X, int Y, int4 gX, int4 gY, int s
     if (!box_overlap(lo, hi, rYlo, rYhi) || beyond(lo, hi)) continue;
     xl[q] = xyz(lo); xh[q] = xyz(hi);
     live |= 1u << q;
+  }
+  // Few of a block's positions can meet Y (a quarter on falling spheres), and a
+  // test of a staged box costs the wavefront the same for one as for 64: where
+  // they fit the staging space, the live ones move together, through it, into
+  // one or two positions a lane, each with its triangle (4,096 spheres 293 -> 273
+  // us a step, 1,500-sphere pile 530 -> 490, 24 scenes 553 -> 529).
+  int nq = XQ;
+  if (__ballot(live != 0)) {
+    int rank[XQ], nlive = 0;
+#pragma unroll
+    for (int q = 0; q < XQ; ++q) {
+      const unsigned long long m = __ballot((live >> q) & 1u);
+      rank[q] = nlive + lanes_below(m);
+      nlive += __popcll(m);
+    }
+    if (nlive <= min(cap, 128)) {
+#pragma unroll
+      for (int q = 0; q < XQ; ++q) {
+        if ((live >> q) & 1u) {
+          lo_s[rank[q]] = V4<R>{xl[q].x, xl[q].y, xl[q].z, box_tag(R(0), xt[q])};
+          hi_s[rank[q]] = V4<R>{xh[q].x, xh[q].y, xh[q].z, R(0)};
+        } else if (xt[q] >= 0) {
+          d.slot_flag[slot_base + xt[q]] = 0;
+        }
+        xt[q] = -1;
+      }
+      wave_sync_lds();
+      live = 0;
+      nq = nlive <= 64 ? 1 : 2;
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        if (lane + 64 * q < nlive) {
+          const V4<R> lo = lo_s[lane + 64 * q], hi = hi_s[lane + 64 * q];
+          xl[q] = xyz(lo); xh[q] = xyz(hi);
+          xt[q] = box_tag_of(lo.w);
+          live |= 1u << q;
+        }
+      }
+      wave_sync_lds();
+    }
   }
   unsigned long long cnt = 0;
   if (__ballot(live != 0)) {
@@ -574,51 +684,7 @@ __device__ int cand_block(const Dev<R>& d, int X, int Y, int4 gX, int4 gY, int s
         ybase += 64;
       }
       wave_sync_lds();
-      // The lane's positions still to test against the staged run, all of
-      // them per staged box: one loop over the staged clusters and their
-      // triangles, uniform over the wavefront (every lane reads the same LDS
-      // entry, a broadcast).  A cluster is skipped when no position of the
-      // wavefront meets its box.  (A loop per position, each walking the
-      // clusters its own box meets, diverged across the lanes and repeated
-      // the staged reads for each of the four positions.)
-      for (int k = 0; k < ncl; ++k) {
-        const unsigned want = count_all ? live : (live & ~flg);
-        if (!__ballot(want != 0u)) break;                 // every position decided
-        const V4<R> cl = clo_s[k], ch = chi_s[k];
-        unsigned mk = 0;                                  // positions that meet the cluster box
-#pragma unroll
-        for (int q = 0; q < XQ; ++q) {
-          const V4<R> lo{xl[q].x, xl[q].y, xl[q].z, R(0)}, hi{xh[q].x, xh[q].y, xh[q].z, R(0)};
-          if (((want >> q) & 1u) && box_overlap(lo, hi, cl, ch)) mk |= 1u << q;
-        }
-        if (!__ballot(mk != 0u)) continue;
-        const int2 rg = crange_s[k];
-        const int end = rg.x + rg.y;
-        // four staged boxes per pass, loaded together (indexes clamped into
-        // the cluster's run; a clamped repeat is not tested)
-        for (int e = rg.x; e < end; e += 4) {
-          V4<R> sl[4], sh[4];
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const int ej = min(e + j, end - 1);
-            sl[j] = lo_s[ej]; sh[j] = hi_s[ej];
-          }
-#pragma unroll
-          for (int q = 0; q < XQ; ++q) {
-            if (!((mk >> q) & 1u)) continue;
-            const V4<R> lo{xl[q].x, xl[q].y, xl[q].z, R(0)}, hi{xh[q].x, xh[q].y, xh[q].z, R(0)};
-            unsigned hit = 0;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) hit |= (box_overlap(lo, hi, sl[j], sh[j]) & (e + j < end)) ? 1u << j : 0u;
-            if (hit) {
-              flg |= 1u << q;
-              if (count_all) cnt += __popc(hit);
-              else mk &= ~(1u << q);                      // decided: no further test
-            }
-          }
-          if (!count_all && !__ballot(mk != 0u)) break;
-        }
-      }
+      cand_test(nq, xl, xh, live, flg, cnt, count_all, ncl, lo_s, hi_s, clo_s, chi_s, crange_s);
       wave_sync_lds();
       if (ybase >= ntY) break;
       // every position that can meet Y is already a candidate: the rest of Y changes no flag
