@@ -1019,7 +1019,9 @@ template <typename R> int run_steps(rbh_ctx* c, int n_steps, double dt, int flag
     const SceneParams& sp = c->sp_host[slot];
     c->any_post = c->any_post || c->scenes[slot].params.use_post_stabilization != 0;
     c->any_hinge = c->any_hinge || sp.h_cnt > 0;
-    c->hinge_lds = std::max(c->hinge_lds, hinge_lds_bytes<R>(sp.hb_cnt, sp.h_cnt));
+    if (sp.h_cnt > 0)
+      c->hinge_lds = std::max(c->hinge_lds, hinge_staged<R>(sp.hb_cnt, sp.h_cnt) ? HingeLds<R>::bytes(sp.hb_cnt, sp.h_cnt)
+                                                                                : hinge_lds_bytes<R>(sp.hb_cnt, sp.h_cnt));
   }
   const bool timing = (flags & RBH_STEP_TIMING) != 0;
   const bool use_graph = (flags & RBH_STEP_GRAPH) != 0;

@@ -18,9 +18,9 @@
 // A hinge sweep is serial over the hinges (Gauss-Seidel); inside one hinge
 // the five rows update from the same w (hinges.py:88), one lane per row, and
 // the twelve body entries of W J^T delta one lane each.  w, the iterate and
-// the accepted solution stay in LDS; the rows of the next HINGE_AHEAD hinges
-// are loaded while one updates, so a hinge costs two wave syncs and LDS
-// traffic.
+// the accepted solution stay in LDS, and so do the rows of all hinges where
+// they fit HINGE_STAGE; else the rows of the next HINGE_AHEAD hinges are loaded
+// from memory while one updates.
 // (included inside namespace rbh by rbh_kernels.h)
 #pragma once
 
@@ -195,6 +195,151 @@ template <typename R> __host__ __device__ constexpr size_t hinge_lds_bytes(int h
   return (2 * (size_t)hb * sizeof(V4<R>) + 10 * (size_t)nh * sizeof(R) + 15) & ~(size_t)15;
 }
 
+// ---- rows staged in LDS
+//
+// A sweep is one wavefront's chain of instructions: ~700 cycles an update from
+// LDS (12 products summed in order, the five deltas by DPP, 5 more products,
+// and reading the next hinge's rows), ~1,000 for w from x, ~1,000 for the merit
+// and the decision; from memory every read of a row waited for the cache.
+// Chains of 5, 16 and 48 cubes, 100 sweeps, four steps: 1.93, 3.71 and 9.30 ms
+// from memory, 1.83, 3.09 and 6.77 staged.
+// Up to 64 KB, so that at least two scenes of a batch share a CU: a chain of 83
+// hinges in FP32, 42 in FP64.
+constexpr size_t HINGE_STAGE = 64 * 1024;
+
+template <typename R> struct HingeLds {
+  static constexpr int VB = (int)sizeof(V4<R>), SR = (int)sizeof(R);
+  int wl, wa, x;             // as in the kernel's layout
+  int J, WJ, ids, br, off, inc;   // rows of J (body of lower index first), of W J^T, int4 (parent, child, first, second
+                                  // slot), b and r0, the bodies' hinge lists
+  __host__ __device__ static constexpr size_t bytes(int hb, int nh) {
+    return hinge_lds_bytes<R>(hb, nh) + (size_t)nh * (40 * VB + 16 + 10 * SR + 8) + 4 * ((size_t)hb + 1);
+  }
+  __device__ HingeLds(unsigned char* smem, int hb, int nh) {
+    wl = lds_addr(smem);
+    wa = wl + hb * VB;
+    x = wa + hb * VB;
+    J = wl + (int)hinge_lds_bytes<R>(hb, nh);
+    WJ = J + 20 * nh * VB;
+    ids = WJ + 20 * nh * VB;
+    br = ids + 16 * nh;
+    off = br + 10 * nh * SR;
+    inc = off + 4 * (hb + 1);
+  }
+};
+
+// dynamic LDS of a scene's hinge solve, staged or not
+template <typename R> __host__ __device__ constexpr bool hinge_staged(int hb, int nh) {
+  return HingeLds<R>::bytes(hb, nh) <= HINGE_STAGE;
+}
+
+template <typename R> __device__ void hinge_stage(const Dev<R>& d, const SceneParams& sp, const HingeLds<R>& L) {
+  constexpr int VB = HingeLds<R>::VB, SR = HingeLds<R>::SR;
+  const int lane = threadIdx.x, nh = sp.h_cnt, h0 = sp.h_off;
+  for (int i = lane; i < 20 * nh; i += 64) {
+    const int h = i / 20, k = i - 20 * h;
+    const int4 id = d.h_ids[h0 + h];
+    const int to = id.x < id.y ? i : 20 * h + (k ^ 2);   // parent first or child first
+    lds_at<V4<R>>(L.J + to * VB) = d.h_J[20 * h0 + i];
+    lds_at<V4<R>>(L.WJ + i * VB) = d.h_WJ[20 * h0 + i];
+  }
+  for (int i = lane; i < 5 * nh; i += 64) {
+    lds_at<R>(L.br + i * SR) = d.h_b[5 * h0 + i];
+    lds_at<R>(L.br + (5 * nh + i) * SR) = d.h_r0[5 * h0 + i];
+  }
+  for (int h = lane; h < nh; h += 64) {
+    const int4 id = d.h_ids[h0 + h];
+    const bool pfirst = id.x < id.y;
+    lds_at<int4>(L.ids + 16 * h) = make_int4(id.z, id.w, pfirst ? id.z : id.w, pfirst ? id.w : id.z);
+  }
+  const int e0 = d.hb_inc_off[sp.hb_off];
+  for (int j = lane; j <= sp.hb_cnt; j += 64) lds_at<int>(L.off + 4 * j) = d.hb_inc_off[sp.hb_off + j] - e0;
+  for (int e = lane; e < 2 * nh; e += 64) lds_at<int>(L.inc + 4 * e) = d.hb_inc[e0 + e] - 2 * h0;
+  for (int i = lane; i < 2 * sp.hb_cnt; i += 64) lds_at<V4<R>>(L.wl + i * VB) = V4<R>{R(0), R(0), R(0), R(0)};
+}
+
+// hinge_body_w, one component of a body per lane; x: LDS address of the rows
+template <typename R> __device__ __forceinline__ void hinge_body_w_lds(const HingeLds<R>& L, int hb, int x) {
+  constexpr int VB = HingeLds<R>::VB, SR = HingeLds<R>::SR;
+  for (int t = threadIdx.x; t < 6 * hb; t += 64) {
+    const int j = t / 6, k = t - 6 * j, ang = k >= 3, c = ang ? k - 3 : k;
+    const int end = lds_at<int>(L.off + 4 * j + 4);
+    int e = lds_at<int>(L.off + 4 * j), ahead = lds_at<int>(L.inc + 4 * e);   // (every body has a hinge)
+    R s = R(0);
+    for (; e < end; ++e) {
+      const int inc = ahead, h = inc >> 1, side = inc & 1;
+      ahead = lds_at<int>(L.inc + 4 * min(e + 1, end - 1));
+      const int w = L.WJ + (20 * h + 2 * side + ang) * VB + c * SR;
+#pragma unroll
+      for (int i = 0; i < 5; ++i) s += lds_at<R>(w + 4 * i * VB) * lds_at<R>(x + (5 * h + i) * SR);
+    }
+    lds_at<R>((ang ? L.wa : L.wl) + j * VB + c * SR) = s;
+  }
+}
+
+// what a lane of the first row needs of a hinge
+template <typename R> struct HingeRow {
+  V4<R> J[4];
+  R b, r0, wj[5];
+  int first, second, dst;   // LDS: slots of the bodies in row order, this lane's entry of w
+};
+
+template <typename R>
+__device__ __forceinline__ void hinge_row(const HingeLds<R>& L, int nh, int h, int lane, HingeRow<R>& g) {
+  constexpr int VB = HingeLds<R>::VB, SR = HingeLds<R>::SR;
+  const int row = min(lane, 4), part = min(lane / 3, 3), c = lane % 3;
+  const int4 id = lds_at<int4>(L.ids + 16 * h);
+  for (int k = 0; k < 4; ++k) g.J[k] = lds_at<V4<R>>(L.J + (20 * h + 4 * row + k) * VB);
+  g.b = lds_at<R>(L.br + (5 * h + row) * SR);
+  g.r0 = lds_at<R>(L.br + (5 * (nh + h) + row) * SR);
+  for (int i = 0; i < 5; ++i) g.wj[i] = lds_at<R>(L.WJ + (20 * h + 4 * i + part) * VB + c * SR);
+  g.first = id.z * VB;
+  g.second = id.w * VB;
+  g.dst = ((part & 1) ? L.wa : L.wl) + (part < 2 ? id.x : id.y) * VB + c * SR;
+}
+
+// hinge_update from LDS; the five deltas go to the other lanes by DPP.  The
+// rows of hinge `next` are read behind this one's w: LDS answers in order, and
+// w is what the chain waits for.
+template <typename R>
+__device__ __forceinline__ void hinge_update_lds(const HingeLds<R>& L, int nh, int h, int next, R rs,
+                                                 const HingeRow<R>& g, HingeRow<R>& n, int lane) {
+  constexpr int SR = HingeLds<R>::SR;
+  const int xa = L.x + (5 * h + min(lane, 4)) * SR;
+  const V3<R> b0 = xyz(lds_at<V4<R>>(L.wl + g.first)), b1 = xyz(lds_at<V4<R>>(L.wa + g.first));
+  const V3<R> b2 = xyz(lds_at<V4<R>>(L.wl + g.second)), b3 = xyz(lds_at<V4<R>>(L.wa + g.second));
+  const R old = lds_at<R>(g.dst), xo = lds_at<R>(xa);
+  __builtin_amdgcn_sched_barrier(0);
+  hinge_row(L, nh, next, lane, n);
+  R s = R(0);
+  s += g.J[0].x * b0.x; s += g.J[0].y * b0.y; s += g.J[0].z * b0.z;
+  s += g.J[1].x * b1.x; s += g.J[1].y * b1.y; s += g.J[1].z * b1.z;
+  s += g.J[2].x * b2.x; s += g.J[2].y * b2.y; s += g.J[2].z * b2.z;
+  s += g.J[3].x * b3.x; s += g.J[3].y * b3.y; s += g.J[3].z * b3.z;
+  const R xn = xo - (g.r0 * rs) * (s + g.b);
+  const R delta = xn - xo;
+  R t = R(0);
+  t += g.wj[0] * row_bcast<0>(delta);
+  t += g.wj[1] * row_bcast<1>(delta);
+  t += g.wj[2] * row_bcast<2>(delta);
+  t += g.wj[3] * row_bcast<3>(delta);
+  t += g.wj[4] * row_bcast<4>(delta);
+  if (lane < 5) lds_at<R>(xa) = xn;
+  if (lane < 12) lds_at<R>(g.dst) = old + t;
+  wave_sync_lds();
+}
+
+template <typename R> __device__ __forceinline__ void hinge_sweep_lds(const HingeLds<R>& L, int nh, R rs) {
+  const int lane = threadIdx.x;
+  HingeRow<R> a, b;
+  hinge_row(L, nh, 0, lane, a);
+  for (int h = 0; h < nh; h += 2) {
+    hinge_update_lds(L, nh, h, min(h + 1, nh - 1), rs, a, b, lane);
+    if (h + 1 >= nh) break;
+    hinge_update_lds(L, nh, h + 1, min(h + 2, nh - 1), rs, b, a, lane);
+  }
+}
+
 // One wavefront per batch scene.  pass 0 records the hinge merit
 // contributions for the contact solve; pass 1 runs to the joint stop and
 // writes hd0/hd1 (see the top of this file).  w, x and the accepted
@@ -219,6 +364,9 @@ template <typename R> __global__ void __launch_bounds__(64) k_hinge_solve(Dev<R>
   R* sol = x + nrow;
   double* res = d.residuals + sp.res_off;
   double* hm = d.h_mer + sp.res_off;
+  const bool staged = hinge_staged<R>(sp.hb_cnt, sp.h_cnt);   // uniform; the launch has room for it
+  const HingeLds<R> L(hinge_smem, sp.hb_cnt, sp.h_cnt);
+  if (staged) hinge_stage(d, sp, L);
   for (int i = lane; i < nrow; i += 64) { x[i] = R(0); sol[i] = R(0); }
   if (own)
     for (int i = lane; i < sp.max_iter; i += 64) res[i] = INFINITY;
@@ -228,20 +376,27 @@ template <typename R> __global__ void __launch_bounds__(64) k_hinge_solve(Dev<R>
   ctl.iters = sp.max_iter;
   for (int it = 0; it < n_it; ++it) {
     const R rs = R(ctl.rscale);
-    hinge_body_w(d, sp, x, wl, wa);
-    // rows of the next HINGE_AHEAD hinges in flight while one updates
-    HingeRegs<R> ring[HINGE_AHEAD];
+    if (staged) {
+      hinge_body_w_lds(L, sp.hb_cnt, L.x);
+      __syncthreads();
+      hinge_sweep_lds(L, sp.h_cnt, rs);
+      __syncthreads();
+    } else {
+      hinge_body_w(d, sp, x, wl, wa);
+      // rows of the next HINGE_AHEAD hinges in flight while one updates
+      HingeRegs<R> ring[HINGE_AHEAD];
 #pragma unroll
-    for (int k = 0; k < HINGE_AHEAD; ++k)
-      if (h0 + k < h1) hinge_load(d, h0 + k, lane, ring[k]);
-    __syncthreads();
-    for (int hh = h0; hh < h1; hh += HINGE_AHEAD) {
+      for (int k = 0; k < HINGE_AHEAD; ++k)
+        if (h0 + k < h1) hinge_load(d, h0 + k, lane, ring[k]);
+      __syncthreads();
+      for (int hh = h0; hh < h1; hh += HINGE_AHEAD) {
 #pragma unroll
-      for (int k = 0; k < HINGE_AHEAD; ++k) {
-        const int h = hh + k;
-        if (h >= h1) break;
-        hinge_update(wl, wa, x, s_delta, 5 * (h - h0), rs, ring[k], lane);
-        if (h + HINGE_AHEAD < h1) hinge_load(d, h + HINGE_AHEAD, lane, ring[k]);
+        for (int k = 0; k < HINGE_AHEAD; ++k) {
+          const int h = hh + k;
+          if (h >= h1) break;
+          hinge_update(wl, wa, x, s_delta, 5 * (h - h0), rs, ring[k], lane);
+          if (h + HINGE_AHEAD < h1) hinge_load(d, h + HINGE_AHEAD, lane, ring[k]);
+        }
       }
     }
     double m = 0.0;
@@ -270,7 +425,8 @@ template <typename R> __global__ void __launch_bounds__(64) k_hinge_solve(Dev<R>
     st.final_merit = ctl.last_merit;
   }
   // finalize_solution (hinges.py:50-57): W J^T sol per body
-  hinge_body_w(d, sp, sol, wl, wa);
+  if (staged) hinge_body_w_lds(L, sp.hb_cnt, L.x + nrow * (int)sizeof(R));
+  else hinge_body_w(d, sp, sol, wl, wa);
   __syncthreads();
   for (int j = lane; j < sp.hb_cnt; j += 64) {
     const int b = d.hb_body[sp.hb_off + j];
