@@ -1337,22 +1337,31 @@ struct SdfLayout {
   }
 };
 
-// the grid's values through the buffer buf (lay.total bytes), by either build
+// the grid's values through the buffer buf (lay.total bytes), by either build;
+// tri: the triangles' corners for the plain one (9 nt values), or null to have
+// them gathered on the device.  A small build is launches and copies: corners
+// gathered by the caller are one copy instead of two and a launch (12 triangles
+// on 12^3: 52.5 us gathered on the device, 48.9 by the caller).
 hipError_t sdf_run(hipStream_t s, const SdfLayout& lay, unsigned char* buf, const double* V, int nv, const int* T,
-                   int nt, const double* mn, const double* mx, int I, int J, int K, double* values) {
+                   int nt, const double* mn, const double* mx, int I, int J, int K, double* values, const double* tri) {
   const long n = (long)I * J * K;
   double* dV = reinterpret_cast<double*>(buf + lay.V);
   int* dT = reinterpret_cast<int*>(buf + lay.T);
   double* dtri = reinterpret_cast<double*>(buf + lay.tri);
   double* dout = reinterpret_cast<double*>(buf + lay.out);
-  hipError_t e = hipMemcpyAsync(dV, V, 24 * (size_t)nv, hipMemcpyHostToDevice, s);
-  if (e == hipSuccess) e = hipMemcpyAsync(dT, T, 12 * (size_t)nt, hipMemcpyHostToDevice, s);
+  hipError_t e = hipSuccess;
+  if (tri) {
+    e = hipMemcpyAsync(dtri, tri, 72 * (size_t)nt, hipMemcpyHostToDevice, s);
+  } else {
+    e = hipMemcpyAsync(dV, V, 24 * (size_t)nv, hipMemcpyHostToDevice, s);
+    if (e == hipSuccess) e = hipMemcpyAsync(dT, T, 12 * (size_t)nt, hipMemcpyHostToDevice, s);
+  }
   if (e != hipSuccess) return e;
   SdfGrid g{I, J, K, {mn[0], mn[1], mn[2]}, {}, {mx[0], mx[1], mx[2]}};
   const int dim[3] = {I, J, K};
   for (int a = 0; a < 3; ++a) g.h[a] = (mx[a] - mn[a]) / (dim[a] - 1);
   if (!lay.pruned) {
-    hipLaunchKernelGGL(k_sdf_gather, dim3(grid_for(9L * nt, 256)), dim3(256), 0, s, dV, dT, nt, dtri);
+    if (!tri) hipLaunchKernelGGL(k_sdf_gather, dim3(grid_for(9L * nt, 256)), dim3(256), 0, s, dV, dT, nt, dtri);
     hipLaunchKernelGGL(k_sdf, dim3((unsigned)((n + SDF_BLOCK - 1) / SDF_BLOCK)), dim3(SDF_BLOCK), 0, s, dtri, nt, I, J, K,
                        mn[0], mn[1], mn[2], g.h[0], g.h[1], g.h[2], dout);
   } else {
@@ -1512,7 +1521,10 @@ int rbh_sdf_build(rbh_ctx* c, const double* V, int nv, const int* T, int nt, con
     HIPCHK(c, hipMalloc(reinterpret_cast<void**>(&c->sdf_buf), lay.total));
     c->sdf_buf_bytes = lay.total;
   }
-  const hipError_t e = sdf_run(c->stream, lay, c->sdf_buf, V, nv, T, nt, mn, mx, I, J, K, values);
+  std::vector<double> tri(lay.pruned ? 0 : (size_t)nt * 9);
+  for (size_t i = 0; i < tri.size(); ++i) tri[i] = V[3 * (size_t)T[i / 3] + i % 3];
+  const hipError_t e = sdf_run(c->stream, lay, c->sdf_buf, V, nv, T, nt, mn, mx, I, J, K, values,
+                               lay.pruned ? nullptr : tri.data());
   if (c->sdf_buf_bytes > SDF_KEEP_BYTES) {
     (void)hipFree(c->sdf_buf);
     c->sdf_buf = nullptr;
@@ -1543,7 +1555,7 @@ int rbh_sdf_build_noalloc(rbh_ctx* c, const double* V, int nv, const int* T, int
   // the pruned build where its workspace fits the array too (the values are the same either way)
   SdfLayout lay(nv, nt, (long)n, sdf_pruned(V, nv, nt, mn, mx, (long)n));
   if (lay.total > NOALLOC_SCRATCH_BYTES) lay = SdfLayout(nv, nt, (long)n, false);
-  const hipError_t e = sdf_run(c->stream, lay, c->scratch, V, nv, T, nt, mn, mx, I, J, K, values);
+  const hipError_t e = sdf_run(c->stream, lay, c->scratch, V, nv, T, nt, mn, mx, I, J, K, values, nullptr);
   if (e != hipSuccess) return fail(c, RBH_E_HIP, std::string("SDF kernel: ") + hipGetErrorString(e));
   return 0;
 }
