@@ -277,6 +277,7 @@ class Transfer {
   }
   // room in the pinned buffer for the ranges added
   int reserve() {
+    HIPCHK(c, hipSetDevice(c->device));   // for the launch: some callers only read, with another device current
     if (c->pin_used + total > c->pin_bytes) {
       HIPCHK(c, hipStreamSynchronize(c->stream));
       c->pin_used = 0;
