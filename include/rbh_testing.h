@@ -23,6 +23,13 @@ extern "C" {
  * look-back scan (a wait for a predecessor that times out returns RBH_E_HIP). */
 int rbh_prefix_sum(rbh_ctx* ctx, const void* in, int elem_bytes, int n, int cap, int* out, int* total);
 
+/* The ellipsoid projection of the contact sweeps (anisotropic friction) in
+ * FP64, on n independent inputs: z (3n) projected onto the ellipsoid of axes
+ * mu (3n) times xn (n), with rbh_params' ellipsoid_tolerance,
+ * ellipsoid_expansion and ellipsoid_max_iterations; out (3n). */
+int rbh_prox_ellipsoid(rbh_ctx* ctx, int n, const double* z, const double* mu, const double* xn, double tolerance,
+                       double expansion, int max_iterations, double* out);
+
 #ifdef __cplusplus
 }
 #endif

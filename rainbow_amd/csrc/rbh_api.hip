@@ -780,6 +780,14 @@ __global__ void k_fill(int* p, int n, int v) {
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = v;
 }
 
+// rbh_prox_ellipsoid (rbh_testing.h)
+__global__ void k_prox_ellipsoid(int n, const double* z, const double* mu, const double* xn, EllipsoidParams ep, double* out) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  prox_ellipsoid<double>(z[3 * i], z[3 * i + 1], z[3 * i + 2], mu[3 * i], mu[3 * i + 1], mu[3 * i + 2], xn[i], ep,
+                         out[3 * i], out[3 * i + 1], out[3 * i + 2]);
+}
+
 int grid_for(long n, int block, int maxg = 8192) {
   long g = (n + block - 1) / block;
   return (int)std::max<long>(1, std::min<long>(g, maxg));
@@ -1502,6 +1510,31 @@ int rbh_prefix_sum(rbh_ctx* c, const void* in, int elem_bytes, int n, int cap, i
   if (e != hipSuccess) return fail(c, RBH_E_HIP, std::string("prefix sum: ") + hipGetErrorString(e));
   if (tail[1] & ERR_SCAN) return fail(c, RBH_E_HIP, "prefix sum: a tile's wait for its predecessors timed out");
   *total = tail[0];
+  return 0;
+}
+
+int rbh_prox_ellipsoid(rbh_ctx* c, int n, const double* z, const double* mu, const double* xn, double tolerance,
+                       double expansion, int max_iterations, double* out) {
+  if (!c || !z || !mu || !xn || !out || n <= 0 || n > (1 << 24) || max_iterations < 0)
+    return fail(c, RBH_E_ARG, "bad projection arguments");
+  (void)hipSetDevice(c->device);
+  const size_t v = (size_t)n * 24;   // z, mu, out: 3 n each; xn: n
+  unsigned char* buf = nullptr;
+  HIPCHK(c, hipMalloc(&buf, 3 * v + (size_t)n * 8));
+  double *dz = reinterpret_cast<double*>(buf), *dmu = dz + 3 * (size_t)n, *dout = dmu + 3 * (size_t)n,
+         *dxn = dout + 3 * (size_t)n;
+  hipError_t e = hipMemcpyAsync(dz, z, v, hipMemcpyHostToDevice, c->stream);
+  if (e == hipSuccess) e = hipMemcpyAsync(dmu, mu, v, hipMemcpyHostToDevice, c->stream);
+  if (e == hipSuccess) e = hipMemcpyAsync(dxn, xn, (size_t)n * 8, hipMemcpyHostToDevice, c->stream);
+  if (e == hipSuccess) {
+    hipLaunchKernelGGL(k_prox_ellipsoid, dim3((n + 255) / 256), dim3(256), 0, c->stream, n, dz, dmu, dxn,
+                       EllipsoidParams{tolerance, expansion, max_iterations}, dout);
+    e = hipGetLastError();
+  }
+  if (e == hipSuccess) e = hipMemcpyAsync(out, dout, v, hipMemcpyDeviceToHost, c->stream);
+  if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+  (void)hipFree(buf);
+  if (e != hipSuccess) return fail(c, RBH_E_HIP, std::string("projection: ") + hipGetErrorString(e));
   return 0;
 }
 

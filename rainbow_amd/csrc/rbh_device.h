@@ -315,7 +315,8 @@ __device__ __forceinline__ EllSide ell_side_at(double n1, double n2, double n3, 
   return s;
 }
 
-// 1 / x to about 1e-8 relative or better
+// 1 / x to 3e-15 relative: the estimate is good to 2^-24 (largest seen 2^-24.4,
+// over 6.7e7 arguments), a Newton step squares that and rounds (2^-48.7)
 __device__ __forceinline__ double ell_rcp(double x) {
   const double y = __builtin_amdgcn_rcp(x);
   return __builtin_fma(y, __builtin_fma(-x, y, 1.0), y);
@@ -327,9 +328,12 @@ __device__ __forceinline__ double ell_rcp(double x) {
 // The root by Newton steps on 1 / sqrt(sum) - 1, which is nearly linear in t
 // and converges from t = 0 without overshooting, in FP32, and one in FP64.
 // With g(r) and the slope m = -g'(r) known, convexity puts the true root
-// within 2 |g(r)| / m + rounding of r.  For t below it g(t) >= m (root - t); for
-// t above it |g| is at least what the slope gathers over the first hundredth
-// of (smallest axis squared + r), on which it stays above 0.97 m.
+// within 2 |g(r)| / m + rounding of r (g(r) is a sum near 1 of three terms, each
+// good to 1e-14).  For t below it g(t) >= m (root - t); for t above it |g| is at
+// least what the slope gathers over the first hundredth of (smallest axis
+// squared + r), on which it stays above 0.97 m: hi has to lie within that reach.
+// (It does not where an axis is thin, g(r) is far above the tolerance and the
+// slope is gone before |g| has grown to it.)
 struct EllRoot { double lo, hi; };
 __device__ __forceinline__ EllRoot ell_root(double n1, double n2, double n3, double saa, double sbb, double scc, double tol) {
   const float f1 = (float)n1, f2 = (float)n2, f3 = (float)n3, e1 = (float)saa, e2 = (float)sbb, e3 = (float)scc;
@@ -353,7 +357,7 @@ __device__ __forceinline__ EllRoot ell_root(double n1, double n2, double n3, dou
   const double m = 2.0 * P, eps = fmax(tol, 0.0) + 1e-12;
   const double over = 1.01 * ell_rcp(m) * (2.0 * fabs(g) + 1e-13 + eps / 0.9);
   const double reach = 0.01 * (fmin(saa, fmin(sbb, scc)) + r);
-  const bool ok = r > 0.0 && fabs(g) < 1e-8 && 0.9 * m * reach > eps && over > 0.0 && over < 1e300;
+  const bool ok = r > 0.0 && fabs(g) < 1e-8 && 0.9 * m * reach > eps && over > 0.0 && over <= reach && over < 1e300;
   return EllRoot{ok ? r - over : -INFINITY, ok ? r + over : INFINITY};
 }
 

@@ -118,6 +118,8 @@ _PROTOS = {
     "rbh_get_tuning": [C.c_void_p, C.c_void_p],
     # include/rbh_testing.h
     "rbh_prefix_sum": [C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_void_p, C.POINTER(C.c_int)],
+    "rbh_prox_ellipsoid": [C.c_void_p, C.c_int, C.c_void_p, C.c_void_p, C.c_void_p, C.c_double, C.c_double, C.c_int,
+                           C.c_void_p],
 }
 
 
@@ -230,6 +232,15 @@ class Context:
         self._check(self.lib.rbh_prefix_sum(self.h, a.ctypes.data_as(C.c_void_p), a.dtype.itemsize, n, cap,
                                             out.ctypes.data_as(C.c_void_p), C.byref(tot)))
         return out, tot.value
+
+    def prox_ellipsoid(self, z, mu, xn, tolerance, expansion, max_iterations):
+        """The sweeps' ellipsoid projection of z (n, 3) (a test hook, include/rbh_testing.h)."""
+        xn = _f64(xn)
+        n = len(xn)
+        z, mu, out = _f64(z, 3 * n), _f64(mu, 3 * n), np.empty((n, 3))
+        self._check(self.lib.rbh_prox_ellipsoid(self.h, n, _ptr(z), _ptr(mu), _ptr(xn), float(tolerance),
+                                                float(expansion), int(max_iterations), _ptr(out)))
+        return out
 
     def sdf_build_noalloc(self, V, T, min_coord, max_coord, I, J, K):
         """sdf_build staged in the library's fixed per-GPU array (no device allocation)."""
