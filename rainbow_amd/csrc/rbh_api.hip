@@ -1308,10 +1308,18 @@ template <typename R> int get_contacts(rbh_ctx* c, const SceneHost& s, const Sce
 bool sdf_pruned(const double* V, int nv, int nt, const double* mn, const double* mx, long n) {
   if (n >= (1L << 30) || nt >= (1 << 27) || nv >= (1 << 28)) return false;   // 32-bit indices
   if ((double)nt * std::max(n, 55000L) <= 1.1e7) return false;
-  bool finite = true;
-  for (int i = 0; i < 3 * nv; ++i) finite = finite && std::isfinite(V[i]);
-  for (int a = 0; a < 3; ++a) finite = finite && std::isfinite(mn[a]) && std::isfinite(mx[a]);
-  return finite;   // (boxes and welding need an order)
+  // Finite values (boxes and welding need an order), and of a size whose fourth
+  // powers, which choose the closest point, are far from overflow and underflow:
+  // distances that are wrong for that reason would join nodes across the surface.
+  double most = 0.0;
+  bool in_range = true;
+  auto look = [&](double x) {
+    in_range = in_range && std::fabs(x) <= 1e60;
+    most = std::max(most, std::fabs(x));
+  };
+  for (int i = 0; i < 3 * nv; ++i) look(V[i]);
+  for (int a = 0; a < 3; ++a) { look(mn[a]); look(mx[a]); }
+  return in_range && most >= 1e-60;
 }
 
 constexpr size_t SDF_KEEP_BYTES = (size_t)64 << 20;
