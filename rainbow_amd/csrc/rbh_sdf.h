@@ -75,6 +75,8 @@ __device__ __forceinline__ double solid_angle(double px, double py, double pz, c
 
 // The same sum of solid angles without an arctangent per triangle: the
 // argument of the product of (den + i det), with the turns past pi counted.
+// The half planes are told apart by sign bits, as atan2 does it: a node on a
+// triangle has det = -0 and den < 0 there, an angle of -pi and not pi.
 // The product is kept near 1 by an approximate reciprocal (its length does
 // not matter).  Agrees with the sum of arctangents to rounding.
 struct TurnSum {
@@ -82,9 +84,9 @@ struct TurnSum {
   int turns = 0;
   __device__ __forceinline__ void add(double det, double den) {
     if (det == 0.0 && den == 0.0) return;   // atan2(0, 0): no angle
-    const bool up = !signbit(det), was = im >= 0.0;
+    const bool up = !signbit(det), was = !signbit(im);
     const double r = re * den - im * det, i = re * det + im * den;
-    const bool now = i >= 0.0;
+    const bool now = !signbit(i);
     if (up && was && !now) ++turns;
     if (!up && !was && now) --turns;
     const double s = __builtin_amdgcn_rcp(fabs(r) + fabs(i));

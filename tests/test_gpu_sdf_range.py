@@ -36,3 +36,57 @@ def test_size_of_the_mesh(ctx, exponent):
     assert np.array_equal(np.signbit(got), np.signbit(base))
     if abs(exponent) < 250:
         assert np.array_equal(bits(got), bits(base * s))
+
+
+def winding(P, V, T):
+    """Sum of the solid angles over 4 pi, in the kernels' expressions (signed zeros too)."""
+    with np.errstate(all="ignore"):
+        a, b, c = (V[T[:, k]][None] - P[:, None] for k in range(3))
+        (ax, ay, az), (bx, by, bz), (cx, cy, cz) = (np.moveaxis(x, 2, 0) for x in (a, b, c))
+        la, lb, lc = (np.sqrt((x * x).sum(-1)) for x in (a, b, c))
+        det = ax * (by * cz - bz * cy) + ay * (bz * cx - bx * cz) + az * (bx * cy - by * cx)
+        den = la * lb * lc + (a * b).sum(-1) * lc + (b * c).sum(-1) * la + (c * a).sum(-1) * lb
+    return 2.0 * np.arctan2(det, den).sum(1) / (4.0 * np.pi)
+
+
+def quartered_box(times):
+    """A unit box, its faces quartered `times` times."""
+    V, T = MESH.create_box(1.0, 1.0, 1.0)
+    V, T = [tuple(v) for v in V], np.asarray(T).tolist()
+    for _ in range(times):
+        index, out = {v: i for i, v in enumerate(V)}, []
+
+        def middle(i, j):
+            v = tuple((np.array(V[i]) + np.array(V[j])) / 2.0)
+            if v not in index:
+                index[v] = len(V)
+                V.append(v)
+            return index[v]
+
+        for a, b, c in T:
+            m = middle(a, b), middle(b, c), middle(c, a)
+            out += [(a, m[0], m[2]), (m[0], b, m[1]), (m[2], m[1], c), m]
+        T = out
+    return np.array(V), np.array(T, dtype=np.int32)
+
+
+@pytest.mark.parametrize("seed", range(2))
+@pytest.mark.parametrize("inwards", [False, True])
+@pytest.mark.parametrize("times,n", [(2, 41), (3, 21)])      # 3 and 12 triangles a lane; a spacing of 1/32 and 1/16
+def test_sign_on_the_surface(ctx, seed, inwards, times, n):
+    """Nodes on a box's faces have a winding number of 0, 1/2 or 1, as the signed zeros of their triangles fall; away
+    from 1/2 the sign must be the one of the sum of arctangents, whatever order the triangles come in."""
+    V, T = quartered_box(times)
+    T = T[np.random.default_rng(seed).permutation(len(T))]
+    T = np.ascontiguousarray(T[:, ::-1] if inwards else T)
+    lo, hi = np.full(3, -0.625), np.full(3, 0.625)          # nodes at +-1/2
+    got = ctx.sdf_build(V, T, lo, hi, n, n, n)
+    x = lo[0] + (hi[0] - lo[0]) / (n - 1) * np.arange(n)
+    k, j, i = np.meshgrid(x, x, x, indexing="ij")
+    P = np.stack([i.ravel(), j.ravel(), k.ravel()], 1)
+    on = np.abs(P).max(1) == 0.5
+    assert (got[on] == 0.0).all()
+    w = np.abs(winding(P[on], V, T))
+    sure = np.abs(w - 0.5) > 1e-6
+    assert sure.any()
+    assert np.array_equal(np.signbit(got[on])[sure], (w > 0.5)[sure])
