@@ -1305,9 +1305,11 @@ template <typename R> int get_contacts(rbh_ctx* c, const SceneHost& s, const Sce
 // takes about 0.48 us per triangle up to ~55,000 nodes, in proportion beyond
 // (12 triangles on 32^3: plain 61 us in all; 448 on 32^3: 457 plain, 320
 // pruned; 10,000 on 64^3: 23.4 ms plain, 1.3 pruned).
-bool sdf_pruned(const double* V, int nv, int nt, const double* mn, const double* mx, long n) {
-  if (n >= (1L << 30) || nt >= (1 << 27) || nv >= (1 << 28)) return false;   // 32-bit indices
-  if ((double)nt * std::max(n, 55000L) <= 1.1e7) return false;
+// Returns the largest coordinate of a mesh and grid for the pruned build, 0 for
+// the plain one.
+double sdf_pruned(const double* V, int nv, int nt, const double* mn, const double* mx, long n) {
+  if (n >= (1L << 30) || nt >= (1 << 27) || nv >= (1 << 28)) return 0.0;   // 32-bit indices
+  if ((double)nt * std::max(n, 55000L) <= 1.1e7) return 0.0;
   // Finite values (boxes and welding need an order), and of a size whose fourth
   // powers, which choose the closest point, are far from overflow and underflow:
   // distances that are wrong for that reason would join nodes across the surface.
@@ -1319,7 +1321,7 @@ bool sdf_pruned(const double* V, int nv, int nt, const double* mn, const double*
   };
   for (int i = 0; i < 3 * nv; ++i) look(V[i]);
   for (int a = 0; a < 3; ++a) { look(mn[a]); look(mx[a]); }
-  return in_range && most >= 1e-60;
+  return in_range && most >= 1e-60 ? most : 0.0;
 }
 
 constexpr size_t SDF_KEEP_BYTES = (size_t)64 << 20;
@@ -1329,8 +1331,9 @@ struct SdfLayout {
   size_t V, T, tri, out, box, cnt, pos, vhash, rep, ekey, ebal, flags, uf, roots, sign, total;
   int vtab, etab;
   bool pruned;
+  double most;   // largest coordinate (pruned builds)
   static int pow2(size_t x) { int p = 256; while ((size_t)p < x) p *= 2; return p; }
-  SdfLayout(int nv, int nt, long n, bool pruned_) : pruned(pruned_) {
+  SdfLayout(int nv, int nt, long n, double most_) : pruned(most_ > 0.0), most(most_) {
     size_t o = 0;
     auto part = [&](size_t bytes) { const size_t at = o; o += (bytes + 255) & ~(size_t)255; return at; };
     V = part(24 * (size_t)nv);
@@ -1374,7 +1377,7 @@ hipError_t sdf_run(hipStream_t s, const SdfLayout& lay, unsigned char* buf, cons
     if (e == hipSuccess) e = hipMemcpyAsync(dT, T, 12 * (size_t)nt, hipMemcpyHostToDevice, s);
   }
   if (e != hipSuccess) return e;
-  SdfGrid g{I, J, K, {mn[0], mn[1], mn[2]}, {}, {mx[0], mx[1], mx[2]}};
+  SdfGrid g{I, J, K, {mn[0], mn[1], mn[2]}, {}, {mx[0], mx[1], mx[2]}, SDF_SLACK * lay.most};
   const int dim[3] = {I, J, K};
   for (int a = 0; a < 3; ++a) g.h[a] = (mx[a] - mn[a]) / (dim[a] - 1);
   if (!lay.pruned) {
@@ -1402,7 +1405,7 @@ hipError_t sdf_run(hipStream_t s, const SdfLayout& lay, unsigned char* buf, cons
     hipLaunchKernelGGL(k_sdf_tris, dim3((nt + 255) / 256), dim3(256), 0, s, w, g);
     hipLaunchKernelGGL(k_sdf_cells_scan, dim3(1), dim3(256), 0, s, w);
     hipLaunchKernelGGL(k_sdf_scatter, dim3(grid_for(lay.etab, 256, 1024)), dim3(256), 0, s, w);
-    hipLaunchKernelGGL(k_sdf_boxes, dim3((nt + 255) / 256), dim3(256), 0, s, w);
+    hipLaunchKernelGGL(k_sdf_boxes, dim3((nt + 255) / 256), dim3(256), 0, s, w, g);
     hipLaunchKernelGGL(k_sdf_dist, dim3((unsigned)((blocks + 3) / 4)), dim3(256), 0, s, w, g);
     hipLaunchKernelGGL(k_sdf_climb, dim3(gn), dim3(256), 0, s, w, g, (int)n);
     hipLaunchKernelGGL(k_sdf_roots, dim3(gn), dim3(256), 0, s, w, (int)n);
@@ -1596,7 +1599,7 @@ int rbh_sdf_build_noalloc(rbh_ctx* c, const double* V, int nv, const int* T, int
   HIPCHK(c, hipSetDevice(c->device));
   // the pruned build where its workspace fits the array too (the values are the same either way)
   SdfLayout lay(nv, nt, (long)n, sdf_pruned(V, nv, nt, mn, mx, (long)n));
-  if (lay.total > NOALLOC_SCRATCH_BYTES) lay = SdfLayout(nv, nt, (long)n, false);
+  if (lay.total > NOALLOC_SCRATCH_BYTES) lay = SdfLayout(nv, nt, (long)n, 0.0);
   const hipError_t e = sdf_run(c->stream, lay, c->scratch, V, nv, T, nt, mn, mx, I, J, K, values, nullptr);
   if (e != hipSuccess) return fail(c, RBH_E_HIP, std::string("SDF kernel: ") + hipGetErrorString(e));
   return 0;

@@ -149,12 +149,13 @@ __global__ void __launch_bounds__(SDF_BLOCK) k_sdf(const double* __restrict__ tr
 // triangles: 2.5e9 distances and solid angles, 23.1 ms):
 //  * Distance: triangles are sorted into clusters of SDF_CL along a Morton
 //    curve; a wavefront owns a small block of nodes and takes the exact
-//    distance only to the clusters whose box may hold a nearer triangle.  The
-//    nearest triangle is always among them and its distance is computed by the
-//    same expression, so the minimum is the same.
+//    distance only to the clusters whose box may hold a nearer triangle, with
+//    room for the rounding of those distances (SdfGrid::slack).  The nearest
+//    triangle is always among them and its distance is computed by the same
+//    expression, so the minimum is the same.
 //  * Sign: away from the surface of a closed mesh the winding number is constant.
 //    Two neighbouring nodes lie on the same side if either is farther from the
-//    surface than from the other; nodes are joined so into trees, and the
+//    surface than from the other, rounding included; nodes are joined so into trees, and the
 //    winding number is taken once per tree.  Nodes on the surface itself join
 //    no other.  Closed: every edge (vertices welded by position) is used as
 //    often in one direction as in the other; for any other mesh every node is
@@ -162,9 +163,16 @@ __global__ void __launch_bounds__(SDF_BLOCK) k_sdf(const double* __restrict__ tr
 constexpr int SDF_CL = 32;               // triangles per cluster
 constexpr int SDF_CELLS = 4096;          // Morton cells the triangles are sorted by (16 per axis)
 
+// A computed distance, or that of two neighbouring nodes, is good to a few units
+// in the last place of the largest coordinate, however small it is itself: near
+// the surface of a mesh 10^4 units from the origin, values within 3e-12 of it
+// came out otherwise than the plain build's before the slack was given.
+constexpr double SDF_SLACK = 256.0 * 2.220446049250313e-16;
+
 struct SdfGrid {
   int I, J, K;
   double mn[3], h[3], mx[3];
+  double slack;              // SDF_SLACK of the largest coordinate
   __device__ __forceinline__ double at(int a, int i) const { return mn[a] + h[a] * (double)i; }
 };
 
@@ -260,8 +268,8 @@ __global__ void k_sdf_scatter(SdfWork w) {
     if (w.ebal[i] != 0) w.flags[0] = 1;
 }
 
-// cluster boxes: half a wavefront each
-__global__ void __launch_bounds__(256) k_sdf_boxes(SdfWork w) {
+// cluster boxes, wider by the slack on every side: half a wavefront each
+__global__ void __launch_bounds__(256) k_sdf_boxes(SdfWork w, SdfGrid g) {
   const int t = blockIdx.x * 256 + threadIdx.x;
   const double* p = w.tri + 9 * (size_t)min(t, w.nt - 1);   // (a cluster starts inside the list)
   double b[6];
@@ -275,7 +283,7 @@ __global__ void __launch_bounds__(256) k_sdf_boxes(SdfWork w) {
       b[3 + a] = fmax(b[3 + a], __shfl_xor(b[3 + a], o, 64));
     }
   if (t < w.nt && t % SDF_CL == 0)
-    for (int a = 0; a < 6; ++a) w.box[6 * (size_t)(t / SDF_CL) + a] = b[a];
+    for (int a = 0; a < 6; ++a) w.box[6 * (size_t)(t / SDF_CL) + a] = a < 3 ? b[a] - g.slack : b[a] + g.slack;
 }
 
 __device__ __forceinline__ double wave_min(double v) {
@@ -283,8 +291,7 @@ __device__ __forceinline__ double wave_min(double v) {
   return v;
 }
 
-// squared distance of the box [lo, hi] to a cluster's box, shrunk by a margin
-// far above the rounding of the distances it is compared with
+// squared distance of the box [lo, hi] to a cluster's box
 __device__ __forceinline__ double sdf_box_gap(const double* lo, const double* hi, const double* box) {
   double s = 0.0;
   for (int a = 0; a < 3; ++a) {
@@ -375,7 +382,7 @@ __global__ void k_sdf_climb(SdfWork w, SdfGrid g, int n) {
         if (x[a] + s < 0 || x[a] + s >= dim[a]) continue;
         const int q = p + s * stride[a];
         const double e = w.out[q];
-        if (!(fmax(d, e) > g.h[a] * (1.0 + 1e-9))) continue;
+        if (!(fmax(d, e) > g.h[a] * (1.0 + 1e-9) + g.slack)) continue;
         if (e > top || (e == top && q < to)) { top = e; to = q; }
       }
     w.uf[p] = open ? p : to;

@@ -90,3 +90,24 @@ def test_sign_on_the_surface(ctx, seed, inwards, times, n):
     sure = np.abs(w - 0.5) > 1e-6
     assert sure.any()
     assert np.array_equal(np.signbit(got[on])[sure], (w > 0.5)[sure])
+
+
+@pytest.mark.parametrize("offset,size", [(0.0, None), (0.0, 1e-8), (1e4, None), (1e4, 1e-8), (1e4, 1e-10)])
+def test_pruned_against_plain_bitwise(ctx, offset, size):
+    """The pruned build and the plain one, bit for bit: over the whole mesh and in boxes of `size` around points of its
+    surface, where every distance is small.  (128^3 nodes: the plain build fits the no-allocation array, the pruned
+    one's workspace does not, so sdf_build_noalloc is the plain build.)"""
+    V, T = sphere()
+    q, _ = np.linalg.qr(np.random.default_rng(3).normal(size=(3, 3)))
+    V = np.ascontiguousarray(V @ q + offset)
+    rng = np.random.default_rng(4)
+    for k in range(1 if size is None else 4):
+        if size is None:
+            lo, hi = V.min(0) - 0.2, V.max(0) + 0.2
+        else:   # around a vertex, an edge and the inside of a triangle
+            w = np.array([(1.0, 0.0, 0.0), (0.5, 0.5, 0.0), (0.2, 0.3, 0.5), (0.3, 0.7, 0.0)][k])
+            c = w @ V[T[rng.integers(len(T))]]
+            lo, hi = c - size, c + size * rng.uniform(0.5, 1.5, 3)
+        pruned, plain = ctx.sdf_build(V, T, lo, hi, 128, 128, 128), ctx.sdf_build_noalloc(V, T, lo, hi, 128, 128, 128)
+        bad = bits(pruned) != bits(plain)
+        assert not bad.any(), "%d differ, by up to %g" % (bad.sum(), np.abs(pruned - plain).max())
