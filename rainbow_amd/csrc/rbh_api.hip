@@ -1305,23 +1305,25 @@ template <typename R> int get_contacts(rbh_ctx* c, const SceneHost& s, const Sce
 // takes about 0.48 us per triangle up to ~55,000 nodes, in proportion beyond
 // (12 triangles on 32^3: plain 61 us in all; 448 on 32^3: 457 plain, 320
 // pruned; 10,000 on 64^3: 23.4 ms plain, 1.3 pruned).
-// Returns the largest coordinate of a mesh and grid for the pruned build, 0 for
-// the plain one.
-double sdf_pruned(const double* V, int nv, int nt, const double* mn, const double* mx, long n) {
-  if (n >= (1L << 30) || nt >= (1 << 27) || nv >= (1 << 28)) return 0.0;   // 32-bit indices
-  if ((double)nt * std::max(n, 55000L) <= 1.1e7) return 0.0;
-  // Finite values (boxes and welding need an order), and of a size whose fourth
-  // powers, which choose the closest point, are far from overflow and underflow:
-  // distances that are wrong for that reason would join nodes across the surface.
+bool sdf_pruned(int nv, int nt, long n, double most) {
+  if (n >= (1L << 30) || nt >= (1 << 27) || nv >= (1 << 28)) return false;   // 32-bit indices
+  return most >= 1e-60 && (double)nt * std::max(n, 55000L) > 1.1e7;
+}
+
+// The largest coordinate of a mesh and its grid, 0 if one is not finite or above
+// 1e60.  Between 1e-60 and that, the products of four lengths that choose the
+// closest point are far from overflow and underflow: distances that are wrong
+// for that reason would join nodes across the surface.
+double sdf_extent(const double* V, int nv, const double* mn, const double* mx) {
   double most = 0.0;
-  bool in_range = true;
+  bool bounded = true;
   auto look = [&](double x) {
-    in_range = in_range && std::fabs(x) <= 1e60;
+    bounded = bounded && std::fabs(x) <= 1e60;   // (not for a NaN)
     most = std::max(most, std::fabs(x));
   };
-  for (int i = 0; i < 3 * nv; ++i) look(V[i]);
+  for (size_t i = 0; i < 3 * (size_t)nv; ++i) look(V[i]);
   for (int a = 0; a < 3; ++a) { look(mn[a]); look(mx[a]); }
-  return in_range && most >= 1e-60 ? most : 0.0;
+  return bounded ? most : 0.0;
 }
 
 constexpr size_t SDF_KEEP_BYTES = (size_t)64 << 20;
@@ -1331,9 +1333,9 @@ struct SdfLayout {
   size_t V, T, tri, out, box, cnt, pos, vhash, rep, ekey, ebal, flags, uf, roots, sign, total;
   int vtab, etab;
   bool pruned;
-  double most;   // largest coordinate (pruned builds)
+  double most;   // largest coordinate, 0: not bounded (sdf_extent)
   static int pow2(size_t x) { int p = 256; while ((size_t)p < x) p *= 2; return p; }
-  SdfLayout(int nv, int nt, long n, double most_) : pruned(most_ > 0.0), most(most_) {
+  SdfLayout(int nv, int nt, long n, double most_, bool pruned_) : pruned(pruned_), most(most_) {
     size_t o = 0;
     auto part = [&](size_t bytes) { const size_t at = o; o += (bytes + 255) & ~(size_t)255; return at; };
     V = part(24 * (size_t)nv);
@@ -1382,8 +1384,13 @@ hipError_t sdf_run(hipStream_t s, const SdfLayout& lay, unsigned char* buf, cons
   for (int a = 0; a < 3; ++a) g.h[a] = (mx[a] - mn[a]) / (dim[a] - 1);
   if (!lay.pruned) {
     if (!tri) hipLaunchKernelGGL(k_sdf_gather, dim3(grid_for(9L * nt, 256)), dim3(256), 0, s, dV, dT, nt, dtri);
-    hipLaunchKernelGGL(k_sdf, dim3((unsigned)((n + SDF_BLOCK - 1) / SDF_BLOCK)), dim3(SDF_BLOCK), 0, s, dtri, nt, I, J, K,
-                       mn[0], mn[1], mn[2], g.h[0], g.h[1], g.h[2], dout);
+    const dim3 blocks((unsigned)((n + SDF_BLOCK - 1) / SDF_BLOCK));
+    if (lay.most > 0.0)
+      hipLaunchKernelGGL(k_sdf<true>, blocks, dim3(SDF_BLOCK), 0, s, dtri, nt, I, J, K, mn[0], mn[1], mn[2], g.h[0],
+                         g.h[1], g.h[2], dout);
+    else
+      hipLaunchKernelGGL(k_sdf<false>, blocks, dim3(SDF_BLOCK), 0, s, dtri, nt, I, J, K, mn[0], mn[1], mn[2], g.h[0],
+                         g.h[1], g.h[2], dout);
   } else {
     SdfWork w{};
     w.V = dV; w.T = dT; w.nv = nv; w.nt = nt; w.tri = dtri; w.out = dout;
@@ -1558,7 +1565,8 @@ int rbh_sdf_build(rbh_ctx* c, const double* V, int nv, const int* T, int nt, con
   (void)hipSetDevice(c->device);
   const long n = (long)I * J * K;
   // one buffer for the call, kept by the context up to SDF_KEEP_BYTES
-  const SdfLayout lay(nv, nt, n, sdf_pruned(V, nv, nt, mn, mx, n));
+  const double most = sdf_extent(V, nv, mn, mx);
+  const SdfLayout lay(nv, nt, n, most, sdf_pruned(nv, nt, n, most));
   if (lay.total > c->sdf_buf_bytes) {
     if (c->sdf_buf) (void)hipFree(c->sdf_buf);
     c->sdf_buf = nullptr;
@@ -1598,8 +1606,9 @@ int rbh_sdf_build_noalloc(rbh_ctx* c, const double* V, int nv, const int* T, int
                 "entry point holds " + std::to_string(NOALLOC_SCRATCH_BYTES) + " (use rbh_sdf_build)");
   HIPCHK(c, hipSetDevice(c->device));
   // the pruned build where its workspace fits the array too (the values are the same either way)
-  SdfLayout lay(nv, nt, (long)n, sdf_pruned(V, nv, nt, mn, mx, (long)n));
-  if (lay.total > NOALLOC_SCRATCH_BYTES) lay = SdfLayout(nv, nt, (long)n, 0.0);
+  const double most = sdf_extent(V, nv, mn, mx);
+  SdfLayout lay(nv, nt, (long)n, most, sdf_pruned(nv, nt, (long)n, most));
+  if (lay.total > NOALLOC_SCRATCH_BYTES) lay = SdfLayout(nv, nt, (long)n, most, false);
   const hipError_t e = sdf_run(c->stream, lay, c->scratch, V, nv, T, nt, mn, mx, I, J, K, values, nullptr);
   if (e != hipSuccess) return fail(c, RBH_E_HIP, std::string("SDF kernel: ") + hipGetErrorString(e));
   return 0;

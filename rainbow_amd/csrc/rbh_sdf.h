@@ -20,7 +20,11 @@ constexpr int SDF_TILE = 256;
 // squared distance of p to the triangle t: the closest point is a + e1 t1 + e2 t2
 // from a corner, an edge (t2 = 0) or the face, chosen in the order of the
 // region tests by selects and one division (a branch per region made every
-// wavefront run through most of them, with a division in four)
+// wavefront run through most of them, with a division in four).
+// BOUNDED: no coordinate is infinite and no difference of two overflows, so
+// that an edge times zero is zero; else the edges without a part in the closest
+// point are set to zero.
+template <bool BOUNDED = true>
 __device__ __forceinline__ double tri_sqdist(double px, double py, double pz, const double* t) {
   const double ax = t[0], ay = t[1], az = t[2], bx = t[3], by = t[4], bz = t[5], cx = t[6], cy = t[7], cz = t[8];
   const double abx = bx - ax, aby = by - ay, abz = bz - az;
@@ -47,10 +51,15 @@ __device__ __forceinline__ double tri_sqdist(double px, double py, double pz, co
   const double t1 = corner ? 0.0 : edge ? q : vb * q, t2 = corner || edge ? 0.0 : vc * q;
   const bool from_b = in_b || in_bc;
   const double ox = in_c ? cx : from_b ? bx : ax, oy = in_c ? cy : from_b ? by : ay, oz = in_c ? cz : from_b ? bz : az;
-  const double ex = in_bc ? cx - bx : in_ac ? acx : abx, ey = in_bc ? cy - by : in_ac ? acy : aby,
-               ez = in_bc ? cz - bz : in_ac ? acz : abz;
-  const double dx = px - (ox + ex * t1 + acx * t2), dy = py - (oy + ey * t1 + acy * t2),
-               dz = pz - (oz + ez * t1 + acz * t2);
+  double ex = in_bc ? cx - bx : in_ac ? acx : abx, ey = in_bc ? cy - by : in_ac ? acy : aby,
+         ez = in_bc ? cz - bz : in_ac ? acz : abz;
+  double fx = acx, fy = acy, fz = acz;
+  if (!BOUNDED) {
+    if (corner) ex = ey = ez = 0.0;
+    if (corner || edge) fx = fy = fz = 0.0;
+  }
+  const double dx = px - (ox + ex * t1 + fx * t2), dy = py - (oy + ey * t1 + fy * t2),
+               dz = pz - (oz + ez * t1 + fz * t2);
   return dx * dx + dy * dy + dz * dz;
 }
 
@@ -109,6 +118,7 @@ __global__ void k_sdf_gather(const double* __restrict__ V, const int* __restrict
 }
 
 // tri: 9 doubles per triangle; out[i + I (j + J k)] = signed distance of node (i, j, k)
+template <bool BOUNDED>
 __global__ void __launch_bounds__(SDF_BLOCK) k_sdf(const double* __restrict__ tri, int nt, int I, int J, int K,
                                                    double mnx, double mny, double mnz, double hx, double hy, double hz,
                                                    double* __restrict__ out) {
@@ -131,7 +141,7 @@ __global__ void __launch_bounds__(SDF_BLOCK) k_sdf(const double* __restrict__ tr
     if (node < n) {
       for (int e = 0; e < cnt; ++e) {
         const double* t = st + e * 9;
-        best = fmin(best, tri_sqdist(px, py, pz, t));
+        best = fmin(best, tri_sqdist<BOUNDED>(px, py, pz, t));
         wsum += solid_angle(px, py, pz, t);
       }
     }

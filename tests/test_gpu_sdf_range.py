@@ -111,3 +111,45 @@ def test_pruned_against_plain_bitwise(ctx, offset, size):
         pruned, plain = ctx.sdf_build(V, T, lo, hi, 128, 128, 128), ctx.sdf_build_noalloc(V, T, lo, hi, 128, 128, 128)
         bad = bits(pruned) != bits(plain)
         assert not bad.any(), "%d differ, by up to %g" % (bad.sum(), np.abs(pruned - plain).max())
+
+
+def closest_sq(p, a, b, c):
+    """Squared distance of p to a triangle, region after region (Ericson, "Real-Time Collision Detection" 5.1.5)."""
+    ab, ac, ap, bp, cp = b - a, c - a, p - a, p - b, p - c
+    d1, d2, d3, d4, d5, d6 = ab @ ap, ac @ ap, ab @ bp, ac @ bp, ab @ cp, ac @ cp
+    if d1 <= 0.0 and d2 <= 0.0:
+        return ap @ ap
+    if d3 >= 0.0 and d4 <= d3:
+        return bp @ bp
+    vc, vb, va = d1 * d4 - d3 * d2, d5 * d2 - d1 * d6, d3 * d6 - d5 * d4
+    if vc <= 0.0 and d1 >= 0.0 and d3 <= 0.0:
+        q = a + d1 / (d1 - d3) * ab
+    elif d6 >= 0.0 and d5 <= d6:
+        return cp @ cp
+    elif vb <= 0.0 and d2 >= 0.0 and d6 <= 0.0:
+        q = a + d2 / (d2 - d6) * ac
+    elif va <= 0.0 and d4 - d3 >= 0.0 and d5 - d6 >= 0.0:
+        q = b + (d4 - d3) / ((d4 - d3) + (d5 - d6)) * (c - b)
+    else:
+        den = 1.0 / (va + vb + vc)
+        q = a + ab * (vb * den) + ac * (vc * den)
+    return (p - q) @ (p - q)
+
+
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan, 1.5e308])
+@pytest.mark.parametrize("corner", [0, 1, 2])
+def test_corner_out_of_range(ctx, value, corner):
+    """A triangle with a corner at infinity has a distance where another corner is the closest point."""
+    V = np.array([(0.1, 0.2, 0.0), (0.9, 0.1, 0.2), (0.3, 0.8, 0.1)])
+    T = np.array([(0, 1, 2)], dtype=np.int32)
+    V[corner, 0] = value
+    lo, hi = (-1.0, -1.0, -1.0), (2.0, 2.0, 2.0)
+    n = 6
+    got = np.abs(ctx.sdf_build(V, T, lo, hi, n, n, n))
+    assert np.array_equal(bits(got), bits(np.abs(ctx.sdf_build_noalloc(V, T, lo, hi, n, n, n))))
+    x = lo[0] + (hi[0] - lo[0]) / (n - 1) * np.arange(n)
+    with np.errstate(all="ignore"):
+        ref = np.array([closest_sq(np.array((i, j, k)), *V) for k in x for j in x for i in x])
+    known = ref < np.inf                          # (a NaN or an infinity leaves the minimum at infinity)
+    assert np.abs(got[known] - np.sqrt(ref[known])).max(initial=0.0) < 1e-12
+    assert (got[~known] == np.inf).all()
