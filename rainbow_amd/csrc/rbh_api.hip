@@ -1384,13 +1384,9 @@ hipError_t sdf_run(hipStream_t s, const SdfLayout& lay, unsigned char* buf, cons
   for (int a = 0; a < 3; ++a) g.h[a] = (mx[a] - mn[a]) / (dim[a] - 1);
   if (!lay.pruned) {
     if (!tri) hipLaunchKernelGGL(k_sdf_gather, dim3(grid_for(9L * nt, 256)), dim3(256), 0, s, dV, dT, nt, dtri);
-    const dim3 blocks((unsigned)((n + SDF_BLOCK - 1) / SDF_BLOCK));
-    if (lay.most > 0.0)
-      hipLaunchKernelGGL(k_sdf<true>, blocks, dim3(SDF_BLOCK), 0, s, dtri, nt, I, J, K, mn[0], mn[1], mn[2], g.h[0],
-                         g.h[1], g.h[2], dout);
-    else
-      hipLaunchKernelGGL(k_sdf<false>, blocks, dim3(SDF_BLOCK), 0, s, dtri, nt, I, J, K, mn[0], mn[1], mn[2], g.h[0],
-                         g.h[1], g.h[2], dout);
+    const auto kernel = lay.most > 0.0 && n <= SDF_SELECT_NODES ? k_sdf<true> : k_sdf<false>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)((n + SDF_BLOCK - 1) / SDF_BLOCK)), dim3(SDF_BLOCK), 0, s, dtri, nt, I, J,
+                       K, mn[0], mn[1], mn[2], g.h[0], g.h[1], g.h[2], dout);
   } else {
     SdfWork w{};
     w.V = dV; w.T = dT; w.nv = nv; w.nt = nt; w.tri = dtri; w.out = dout;

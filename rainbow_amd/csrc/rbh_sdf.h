@@ -17,15 +17,57 @@ namespace rbh {
 constexpr int SDF_BLOCK = 256;
 constexpr int SDF_TILE = 256;
 
-// squared distance of p to the triangle t: the closest point is a + e1 t1 + e2 t2
-// from a corner, an edge (t2 = 0) or the face, chosen in the order of the
-// region tests by selects and one division (a branch per region made every
-// wavefront run through most of them, with a division in four).
-// BOUNDED: no coordinate is infinite and no difference of two overflows, so
-// that an edge times zero is zero; else the edges without a part in the closest
-// point are set to zero.
-template <bool BOUNDED = true>
+// squared distance of p to the triangle t, region after region: the form for
+// wavefronts of neighbouring nodes, which mostly agree on the region.
 __device__ __forceinline__ double tri_sqdist(double px, double py, double pz, const double* t) {
+  const double ax = t[0], ay = t[1], az = t[2], bx = t[3], by = t[4], bz = t[5], cx = t[6], cy = t[7], cz = t[8];
+  double abx = bx - ax, aby = by - ay, abz = bz - az;
+  double acx = cx - ax, acy = cy - ay, acz = cz - az;
+  double apx = px - ax, apy = py - ay, apz = pz - az;
+  double d1 = abx * apx + aby * apy + abz * apz;
+  double d2 = acx * apx + acy * apy + acz * apz;
+  double qx, qy, qz;
+  if (d1 <= 0.0 && d2 <= 0.0) { qx = ax; qy = ay; qz = az; goto done; }
+  {
+    double bpx = px - bx, bpy = py - by, bpz = pz - bz;
+    double d3 = abx * bpx + aby * bpy + abz * bpz;
+    double d4 = acx * bpx + acy * bpy + acz * bpz;
+    if (d3 >= 0.0 && d4 <= d3) { qx = bx; qy = by; qz = bz; goto done; }
+    double vc = d1 * d4 - d3 * d2;
+    if (vc <= 0.0 && d1 >= 0.0 && d3 <= 0.0) {
+      double v = d1 / (d1 - d3);
+      qx = ax + v * abx; qy = ay + v * aby; qz = az + v * abz; goto done;
+    }
+    double cpx = px - cx, cpy = py - cy, cpz = pz - cz;
+    double d5 = abx * cpx + aby * cpy + abz * cpz;
+    double d6 = acx * cpx + acy * cpy + acz * cpz;
+    if (d6 >= 0.0 && d5 <= d6) { qx = cx; qy = cy; qz = cz; goto done; }
+    double vb = d5 * d2 - d1 * d6;
+    if (vb <= 0.0 && d2 >= 0.0 && d6 <= 0.0) {
+      double w = d2 / (d2 - d6);
+      qx = ax + w * acx; qy = ay + w * acy; qz = az + w * acz; goto done;
+    }
+    double va = d3 * d6 - d5 * d4;
+    if (va <= 0.0 && (d4 - d3) >= 0.0 && (d5 - d6) >= 0.0) {
+      double w = (d4 - d3) / ((d4 - d3) + (d5 - d6));
+      qx = bx + w * (cx - bx); qy = by + w * (cy - by); qz = bz + w * (cz - bz); goto done;
+    }
+    double den = 1.0 / (va + vb + vc);
+    double v = vb * den, w = vc * den;
+    qx = ax + abx * v + acx * w; qy = ay + aby * v + acy * w; qz = az + abz * v + acz * w;
+  }
+done:
+  double dx = px - qx, dy = py - qy, dz = pz - qz;
+  return dx * dx + dy * dy + dz * dz;
+}
+
+// the same value by selects and one division: the closest point is a + e1 t1 +
+// e2 t2 from a corner, an edge (t2 = 0) or the face, chosen in the order of the
+// region tests.  For wavefronts whose lanes hold different triangles: a branch
+// per region had them run through most of the regions, with a division in four;
+// and for lone wavefronts, whose time is that of the chain of instructions.
+// The coordinates have to be finite (an edge times zero is zero).
+__device__ __forceinline__ double tri_sqdist_select(double px, double py, double pz, const double* t) {
   const double ax = t[0], ay = t[1], az = t[2], bx = t[3], by = t[4], bz = t[5], cx = t[6], cy = t[7], cz = t[8];
   const double abx = bx - ax, aby = by - ay, abz = bz - az;
   const double acx = cx - ax, acy = cy - ay, acz = cz - az;
@@ -51,15 +93,10 @@ __device__ __forceinline__ double tri_sqdist(double px, double py, double pz, co
   const double t1 = corner ? 0.0 : edge ? q : vb * q, t2 = corner || edge ? 0.0 : vc * q;
   const bool from_b = in_b || in_bc;
   const double ox = in_c ? cx : from_b ? bx : ax, oy = in_c ? cy : from_b ? by : ay, oz = in_c ? cz : from_b ? bz : az;
-  double ex = in_bc ? cx - bx : in_ac ? acx : abx, ey = in_bc ? cy - by : in_ac ? acy : aby,
-         ez = in_bc ? cz - bz : in_ac ? acz : abz;
-  double fx = acx, fy = acy, fz = acz;
-  if (!BOUNDED) {
-    if (corner) ex = ey = ez = 0.0;
-    if (corner || edge) fx = fy = fz = 0.0;
-  }
-  const double dx = px - (ox + ex * t1 + fx * t2), dy = py - (oy + ey * t1 + fy * t2),
-               dz = pz - (oz + ez * t1 + fz * t2);
+  const double ex = in_bc ? cx - bx : in_ac ? acx : abx, ey = in_bc ? cy - by : in_ac ? acy : aby,
+               ez = in_bc ? cz - bz : in_ac ? acz : abz;
+  const double dx = px - (ox + ex * t1 + acx * t2), dy = py - (oy + ey * t1 + acy * t2),
+               dz = pz - (oz + ez * t1 + acz * t2);
   return dx * dx + dy * dy + dz * dz;
 }
 
@@ -117,8 +154,13 @@ __global__ void k_sdf_gather(const double* __restrict__ V, const int* __restrict
   }
 }
 
-// tri: 9 doubles per triangle; out[i + I (j + J k)] = signed distance of node (i, j, k)
-template <bool BOUNDED>
+// tri: 9 doubles per triangle; out[i + I (j + J k)] = signed distance of node (i, j, k).
+// SELECT: the closest point by selects.  Up to a wavefront per SIMD (65,536
+// nodes) that is 2 to 5 % faster (126 triangles on 12^3 142 us, by branches 150;
+// on 38^3 167, 170), beyond it the less work of the branches is (448 on 128^3
+// 8.7 ms, by selects 10.1; 500 strewn ones 10.0, 11.0).
+constexpr long SDF_SELECT_NODES = 65536;
+template <bool SELECT>
 __global__ void __launch_bounds__(SDF_BLOCK) k_sdf(const double* __restrict__ tri, int nt, int I, int J, int K,
                                                    double mnx, double mny, double mnz, double hx, double hy, double hz,
                                                    double* __restrict__ out) {
@@ -141,7 +183,7 @@ __global__ void __launch_bounds__(SDF_BLOCK) k_sdf(const double* __restrict__ tr
     if (node < n) {
       for (int e = 0; e < cnt; ++e) {
         const double* t = st + e * 9;
-        best = fmin(best, tri_sqdist<BOUNDED>(px, py, pz, t));
+        best = fmin(best, SELECT ? tri_sqdist_select(px, py, pz, t) : tri_sqdist(px, py, pz, t));
         wsum += solid_angle(px, py, pz, t);
       }
     }
@@ -354,7 +396,7 @@ __global__ void __launch_bounds__(256) k_sdf_dist(SdfWork w, SdfGrid g) {
     const double* src = w.tri + 9 * (size_t)c * SDF_CL;
     for (int e = lane; e < 9 * n; e += 64) st[wave][e] = src[e];
     wave_sync_lds();
-    for (int t = part; t < n; t += SDF_SPLIT) best = fmin(best, tri_sqdist(p[0], p[1], p[2], st[wave] + 9 * t));
+    for (int t = part; t < n; t += SDF_SPLIT) best = fmin(best, tri_sqdist_select(p[0], p[1], p[2], st[wave] + 9 * t));
     wave_sync_lds();
     for (int o = 1; o < SDF_SPLIT; o <<= 1) best = fmin(best, __shfl_xor(best, o, 64));
   };

@@ -153,3 +153,16 @@ def test_corner_out_of_range(ctx, value, corner):
     known = ref < np.inf                          # (a NaN or an infinity leaves the minimum at infinity)
     assert np.abs(got[known] - np.sqrt(ref[known])).max(initial=0.0) < 1e-12
     assert (got[~known] == np.inf).all()
+
+
+def test_plain_forms_bitwise(ctx):
+    """Up to 65,536 nodes the plain build finds closest points by selects, above it by branches: the nodes that two
+    grids on either side of the line share have the same bits."""
+    V, T = quartered_box(1)
+    q, _ = np.linalg.qr(np.random.default_rng(8).normal(size=(3, 3)))
+    V = np.ascontiguousarray(V @ q)
+    lo, h = np.full(3, -1.0), 1.0 / 32.0                     # exact spacing: shared nodes have the same coordinates
+    out = [ctx.sdf_build(V, T, lo, lo + h * (np.array(n) - 1), *n).reshape(n[::-1]) for n in ((64, 32, 32), (66, 32, 32))]
+    assert out[0].size == 65536
+    assert np.array_equal(bits(out[0]), bits(np.ascontiguousarray(out[1][:, :, :64])))
+    assert np.signbit(out[0]).any() and not np.signbit(out[0]).all()
