@@ -1412,7 +1412,7 @@ hipError_t sdf_run(hipStream_t s, const SdfLayout& lay, unsigned char* buf, cons
     hipLaunchKernelGGL(k_sdf_dist, dim3((unsigned)((blocks + 3) / 4)), dim3(256), 0, s, w, g);
     hipLaunchKernelGGL(k_sdf_climb, dim3(gn), dim3(256), 0, s, w, g, (int)n);
     hipLaunchKernelGGL(k_sdf_roots, dim3(gn), dim3(256), 0, s, w, (int)n);
-    hipLaunchKernelGGL(k_sdf_sign, dim3(2048), dim3(256), 0, s, w, g);
+    hipLaunchKernelGGL(k_sdf_sign, dim3(2048), dim3(256), 0, s, w, g, (int)n);
     hipLaunchKernelGGL(k_sdf_apply, dim3(gn), dim3(256), 0, s, w, (int)n);
   }
   e = hipGetLastError();

@@ -210,8 +210,8 @@ __global__ void __launch_bounds__(SDF_BLOCK) k_sdf(const double* __restrict__ tr
 //    surface than from the other, rounding included; nodes are joined so into trees, and the
 //    winding number is taken once per tree.  Nodes on the surface itself join
 //    no other.  Closed: every edge (vertices welded by position) is used as
-//    often in one direction as in the other; for any other mesh every node is
-//    a tree of its own.
+//    often in one direction as in the other; for any other (open) mesh every
+//    node is a tree of its own.
 constexpr int SDF_CL = 32;               // triangles per cluster
 constexpr int SDF_CELLS = 4096;          // Morton cells the triangles are sorted by (16 per axis)
 
@@ -237,7 +237,7 @@ struct SdfWork {
   int* vhash; int vmask;     // welded vertices: table of vertex indices (-1: free)
   int* rep;                  // per vertex: the vertex that stands for its position
   unsigned long long* ekey; int* ebal; int emask;   // edges (lower, upper vertex): uses upwards minus downwards
-  int* flags;                // [0] 1: not closed, [1] roots
+  int* flags;                // [0] 1: open, [1] roots of a closed mesh
   int* uf;                   // per node: parent
   int* roots;                // nodes without a parent
   signed char* sign;         // per root: 1 inside
@@ -422,7 +422,7 @@ __global__ void __launch_bounds__(256) k_sdf_dist(SdfWork w, SdfGrid g) {
 // maxima of the distance, and the nodes next to or on the surface that no
 // neighbour reaches.
 __global__ void k_sdf_climb(SdfWork w, SdfGrid g, int n) {
-  const bool open = w.flags[0] != 0;
+  if (w.flags[0]) return;   // an open mesh
   const int stride[3] = {1, g.I, g.I * g.J}, dim[3] = {g.I, g.J, g.K};
   for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < n; p += gridDim.x * blockDim.x) {
     const int x[3] = {p % g.I, p / g.I % g.J, p / (g.I * g.J)};
@@ -437,12 +437,13 @@ __global__ void k_sdf_climb(SdfWork w, SdfGrid g, int n) {
         if (!(fmax(d, e) > g.h[a] * (1.0 + 1e-9) + g.slack)) continue;
         if (e > top || (e == top && q < to)) { top = e; to = q; }
       }
-    w.uf[p] = open ? p : to;
+    w.uf[p] = to;
   }
 }
 
 // the trees' roots, listed in any order
 __global__ void k_sdf_roots(SdfWork w, int n) {
+  if (w.flags[0]) return;
   for (int p0 = blockIdx.x * blockDim.x; p0 < n; p0 += gridDim.x * blockDim.x) {
     const int p = p0 + (int)threadIdx.x, lane = (int)(threadIdx.x & 63);
     const bool r = p < n && w.uf[p] == p;
@@ -459,23 +460,79 @@ __device__ __forceinline__ void sdf_corners(const SdfWork& w, int t, double* c) 
   for (int e = 0; e < 9; ++e) c[e] = w.V[3 * w.T[3 * t + e / 3] + e % 3];
 }
 
-// |winding number| > 1/2 at a node, from the sum of its solid angles (4 pi wn):
-// a sum in any order decides unless it lies near 1/2; exact() then adds the
-// terms in k_sdf's order
 constexpr double SDF_4PI = 4.0 * 3.14159265358979323846;
-template <typename F> __device__ __forceinline__ bool sdf_inside(double sum, F&& exact) {
-  const double wn = sum / SDF_4PI;
-  if (fabs(fabs(wn) - 0.5) > 1e-6) return fabs(wn) > 0.5;   // (not for a NaN)
-  return fabs(exact() / SDF_4PI) > 0.5;
+
+// sum of the solid angles at p in k_sdf's order, by a wavefront; sh: 64 values
+__device__ __forceinline__ double sdf_angles(const SdfWork& w, double px, double py, double pz, double* sh, int lane) {
+  double wsum = 0.0;
+  for (int t0 = 0; t0 < w.nt; t0 += 64) {
+    const int t = t0 + lane, n = min(64, w.nt - t0);
+    if (t < w.nt) {
+      double c[9];
+      sdf_corners(w, t, c);
+      sh[lane] = solid_angle(px, py, pz, c);
+    }
+    wave_sync_lds();
+    for (int e = 0; e < n; ++e) wsum += sh[e];
+    wave_sync_lds();
+  }
+  return wsum;
 }
 
-// Winding number at each root, a wavefront each (a thread each, for the many
-// roots of a spiky or an open mesh, took 0.4 us a triangle in series).
-__global__ void __launch_bounds__(256) k_sdf_sign(SdfWork w, SdfGrid g) {
-  __shared__ double sh[4][64];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, nr = w.flags[1];
+// Whether |winding number| > 1/2 at the roots (of an open mesh: at every node),
+// from the sum of their solid angles (4 pi wn): a sum in any order decides unless
+// it lies near 1/2 (or is not a number); sdf_angles then adds the terms in k_sdf's
+// order.  A wavefront per root (a thread each took 0.4 us a triangle in series), or,
+// from SDF_MANY roots on, a thread each with the triangles staged in LDS: the threads
+// then hide that chain, and a triangle is read once for 256 nodes and not once for
+// each (408 triangles with a hole on 51^3 1.03 ms by wavefronts, 1.06 by threads; on
+// 58^3 0.96, 0.82; on 128^3 8.3, 6.7; 9,999 on 51^3 7.4, 9.8; on 58^3 10.8, 9.6).
+// What is left over the plain build is least for strewn triangles, which cluster
+// badly: 500 on 128^3 10.2 ms (plain 10.3), 80 on 64^3 0.46 (0.45).
+constexpr int SDF_MANY = 163840;
+__global__ void __launch_bounds__(256) k_sdf_sign(SdfWork w, SdfGrid g, int n) {
+  __shared__ double st[SDF_TILE * 9];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const bool open = w.flags[0] != 0;
+  const int nr = open ? n : w.flags[1];
+  auto inside_by = [](double sum) { return fabs(sum / SDF_4PI) > 0.5; };
+  auto put = [&](int node, bool inside) {
+    if (!open) w.sign[node] = inside ? 1 : 0;
+    else if (inside) w.out[node] = -w.out[node];
+  };
+  auto sure = [](double sum) { return fabs(fabs(sum / SDF_4PI) - 0.5) > 1e-6; };
+  if (nr >= SDF_MANY) {
+    for (int r0 = blockIdx.x * 256; r0 < nr; r0 += gridDim.x * 256) {
+      const int r = r0 + (int)threadIdx.x;
+      const bool have = r < nr;
+      const int node = have ? (open ? r : w.roots[r]) : 0;
+      const double px = g.at(0, node % g.I), py = g.at(1, node / g.I % g.J), pz = g.at(2, node / (g.I * g.J));
+      TurnSum ts;
+      for (int t0 = 0; t0 < w.nt; t0 += SDF_TILE) {
+        const int cnt = min(SDF_TILE, w.nt - t0);
+        for (int e = threadIdx.x; e < 9 * cnt; e += 256) st[e] = w.tri[9 * (size_t)t0 + e];
+        __syncthreads();
+        for (int e = 0; e < cnt; ++e) {
+          double det, den;
+          solid_angle_parts(px, py, pz, st + 9 * e, det, den);
+          ts.add(det, den);
+        }
+        __syncthreads();
+      }
+      const double sum = ts.angle();
+      bool inside = inside_by(sum);
+      for (unsigned long long m = __ballot(have && !sure(sum)); m; m &= m - 1) {
+        const int l = __ffsll((long long)m) - 1;
+        const bool in = inside_by(sdf_angles(w, __shfl(px, l, 64), __shfl(py, l, 64), __shfl(pz, l, 64), st + 64 * wave, lane));
+        if (lane == l) inside = in;
+      }
+      if (have) put(node, inside);
+      __syncthreads();   // st is staged again
+    }
+    return;
+  }
   for (int r = blockIdx.x * 4 + wave; r < nr; r += gridDim.x * 4) {
-    const int node = w.roots[r];
+    const int node = open ? r : w.roots[r];
     const double px = g.at(0, node % g.I), py = g.at(1, node / g.I % g.J), pz = g.at(2, node / (g.I * g.J));
     TurnSum ts;
     for (int t = lane; t < w.nt; t += 64) {
@@ -486,26 +543,13 @@ __global__ void __launch_bounds__(256) k_sdf_sign(SdfWork w, SdfGrid g) {
     }
     double sum = ts.angle();
     for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
-    const bool inside = sdf_inside(sum, [&] {   // (uniform over the wavefront)
-      double wsum = 0.0;
-      for (int t0 = 0; t0 < w.nt; t0 += 64) {
-        const int t = t0 + lane, n = min(64, w.nt - t0);
-        if (t < w.nt) {
-          double c[9];
-          sdf_corners(w, t, c);
-          sh[wave][lane] = solid_angle(px, py, pz, c);
-        }
-        wave_sync_lds();
-        for (int e = 0; e < n; ++e) wsum += sh[wave][e];
-        wave_sync_lds();
-      }
-      return wsum;
-    });
-    if (lane == 0) w.sign[node] = inside ? 1 : 0;
+    if (!sure(sum)) sum = sdf_angles(w, px, py, pz, st + 64 * wave, lane);   // (uniform over the wavefront)
+    if (lane == 0) put(node, inside_by(sum));
   }
 }
 
 __global__ void k_sdf_apply(SdfWork w, int n) {
+  if (w.flags[0]) return;   // (k_sdf_sign has done it)
   for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < n; p += gridDim.x * blockDim.x) {
     int r = p;
     for (int q = w.uf[r]; q != r; q = w.uf[r]) r = q;

@@ -166,3 +166,24 @@ def test_plain_forms_bitwise(ctx):
     assert out[0].size == 65536
     assert np.array_equal(bits(out[0]), bits(np.ascontiguousarray(out[1][:, :, :64])))
     assert np.signbit(out[0]).any() and not np.signbit(out[0]).all()
+
+
+@pytest.mark.parametrize("mesh", ["open255", "open256", "open257", "open408", "box"])
+def test_many_roots_bitwise(ctx, mesh):
+    """Open meshes, whose every node has its own winding number: from 163,840 nodes on a thread takes a node, below a
+    wavefront does.  Two grids on either side of the line agree in the nodes they share, on the faces of a box (winding
+    numbers near 1/2) too, and the larger one has the plain build's values."""
+    if mesh == "box":
+        V, T = quartered_box(3)
+        T = T[1:]
+    else:
+        V, T = sphere()
+        T = T[-int(mesh[4:]):]
+    lo, h = np.full(3, -0.625), 1.0 / 32.0                   # exact spacing: shared nodes have the same coordinates
+    out = [ctx.sdf_build(V, T, lo, lo + h * (np.array(n) - 1), *n).reshape(n[::-1]) for n in ((63, 64, 40), (64, 64, 40))]
+    assert out[1].size == 163840
+    assert np.array_equal(bits(out[0]), bits(np.ascontiguousarray(out[1][:, :, :63])))
+    hi = lo + h * 63
+    many, plain = ctx.sdf_build(V, T, lo, hi, 128, 128, 128), ctx.sdf_build_noalloc(V, T, lo, hi, 128, 128, 128)
+    assert np.array_equal(bits(many), bits(plain))
+    assert np.signbit(plain).any()
