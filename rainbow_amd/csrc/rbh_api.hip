@@ -1562,13 +1562,20 @@ int rbh_sdf_build(rbh_ctx* c, const double* V, int nv, const int* T, int nt, con
   const long n = (long)I * J * K;
   // one buffer for the call, kept by the context up to SDF_KEEP_BYTES
   const double most = sdf_extent(V, nv, mn, mx);
-  const SdfLayout lay(nv, nt, n, most, sdf_pruned(nv, nt, n, most));
-  if (lay.total > c->sdf_buf_bytes) {
+  SdfLayout lay(nv, nt, n, most, sdf_pruned(nv, nt, n, most));
+  for (bool got = lay.total <= c->sdf_buf_bytes; !got;) {
     if (c->sdf_buf) (void)hipFree(c->sdf_buf);
     c->sdf_buf = nullptr;
     c->sdf_buf_bytes = 0;
-    HIPCHK(c, hipMalloc(reinterpret_cast<void**>(&c->sdf_buf), lay.total));
-    c->sdf_buf_bytes = lay.total;
+    got = hipMalloc(reinterpret_cast<void**>(&c->sdf_buf), lay.total) == hipSuccess;
+    if (got) {
+      c->sdf_buf_bytes = lay.total;
+    } else {
+      (void)hipGetLastError();
+      c->sdf_buf = nullptr;
+      if (!lay.pruned) return fail(c, RBH_E_MEMORY, "SDF buffer");
+      lay = SdfLayout(nv, nt, n, most, false);   // half the memory
+    }
   }
   std::vector<double> tri(lay.pruned ? 0 : (size_t)nt * 9);
   for (size_t i = 0; i < tri.size(); ++i) tri[i] = V[3 * (size_t)T[i / 3] + i % 3];

@@ -187,3 +187,19 @@ def test_many_roots_bitwise(ctx, mesh):
     many, plain = ctx.sdf_build(V, T, lo, hi, 128, 128, 128), ctx.sdf_build_noalloc(V, T, lo, hi, 128, 128, 128)
     assert np.array_equal(bits(many), bits(plain))
     assert np.signbit(plain).any()
+
+
+def test_no_memory_for_the_grid():
+    """A grid larger than the device (4,096^3 nodes, 550 GB) is refused as such, and the context goes on."""
+    V, T = sphere()
+    lo, hi = V.min(0) - 0.2, V.max(0) + 0.2
+    ctx = native.Context(0, "fp64")
+    try:
+        before = ctx.sdf_build(V, T, lo, hi, 16, 16, 16)
+        none = np.empty(1)                       # (nothing is written without a buffer on the device)
+        rc = ctx.lib.rbh_sdf_build(ctx.h, native._ptr(V), len(V), native._ptr(T), len(T), native._ptr(lo), native._ptr(hi),
+                                   4096, 4096, 4096, native._ptr(none))
+        assert rc == -3 and ctx.lib.rbh_last_error(ctx.h) == b"SDF buffer"
+        assert np.array_equal(bits(ctx.sdf_build(V, T, lo, hi, 16, 16, 16)), bits(before))
+    finally:
+        ctx.close()
