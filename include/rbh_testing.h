@@ -1,8 +1,8 @@
 /* rbh_testing.h - entry points of librbh.so for tests only.
  *
  * No counterpart in the reference.  They run one internal stage of the step
- * on caller data, so that a test can check the stage's edge cases directly
- * (sizes the step rarely produces).  They allocate device memory per call and
+ * on caller data, or one of its launch rules, so that a test can check its
+ * edge cases directly (sizes the step rarely produces).  They allocate device memory per call and
  * are not meant for production paths.
  */
 #ifndef RBH_TESTING_H
@@ -29,6 +29,16 @@ int rbh_prefix_sum(rbh_ctx* ctx, const void* in, int elem_bytes, int n, int cap,
  * ellipsoid_expansion and ellipsoid_max_iterations; out (3n). */
 int rbh_prox_ellipsoid(rbh_ctx* ctx, int n, const double* z, const double* mu, const double* xn, double tolerance,
                        double expansion, int max_iterations, double* out);
+
+/* How the hinge solve of a batch would be launched (no device needed): n
+ * hinged scenes of bodies[i] bodies in hinges[i] hinges on `cus` compute units.
+ * *staged: 1 if their rows are staged in LDS; *lds: bytes of a workgroup;
+ * rows_at (n): where a scene's staged rows start. */
+int rbh_hinge_launch(int precision_bytes, int cus, int n, const int* bodies, const int* hinges, int* staged,
+                     long long* lds, int* rows_at);
+/* Workgroups (of one wavefront) of the hinge solve that share a compute unit
+ * at `lds` bytes each. */
+int rbh_hinge_occupancy(rbh_ctx* ctx, int staged, long long lds, int* groups_per_cu);
 
 #ifdef __cplusplus
 }

@@ -144,7 +144,7 @@ struct rbh_ctx {
   DBuf h_ids, h_geo, hb_body, hb_inc_off, hb_inc, h_J, h_WJ, h_b, h_r0, d_hmer;
   bool hinges_dirty = false;
   bool any_hinge = false;   // a scene of the batch has hinges (set per run_steps call)
-  size_t hinge_lds = 0;     // dynamic LDS of the hinge solve for the batch (its largest scene)
+  rbh::HingeLaunch hinge{false, 16};   // the batch's hinge solve
   // scenes
   std::vector<SceneHost> scenes;
   std::vector<SceneParams> sp_host;
@@ -845,7 +845,8 @@ hipEvent_t* timing_row(rbh_ctx* c, int i, int todo) {
 template <typename R> void hinge_pass(rbh_ctx* c, const Dev<R>& d, int pass) {
   if (!c->any_hinge) return;
   if (pass == 0) hipLaunchKernelGGL(k_hinge_rows<R>, dim3(c->ns), dim3(64), 0, c->stream, d);
-  hipLaunchKernelGGL(k_hinge_solve<R>, dim3(c->ns), dim3(64), c->hinge_lds, c->stream, d, pass);
+  const auto solve = c->hinge.staged ? k_hinge_solve<R, true> : k_hinge_solve<R, false>;
+  hipLaunchKernelGGL(solve, dim3(c->ns), dim3(64), c->hinge.lds, c->stream, d, pass);
 }
 
 template <typename R> hipError_t launch_step(rbh_ctx* c, double dt, int flags, hipEvent_t* ev, bool multi, int multi_grid) {
@@ -1010,8 +1011,10 @@ template <typename R> int setup_solve_lds(rbh_ctx* c) {
   }
   c->solve_lds_half = half;
   const int hbytes = (int)hinge_lds_bytes<R>(HINGE_BODY_MAX, HINGE_MAX);
-  if (hipFuncSetAttribute(reinterpret_cast<const void*>(k_hinge_solve<R>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                          hbytes) != hipSuccess) {
+  if (hipFuncSetAttribute(reinterpret_cast<const void*>(k_hinge_solve<R, false>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                          hbytes) != hipSuccess ||
+      hipFuncSetAttribute(reinterpret_cast<const void*>(k_hinge_solve<R, true>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                          (int)HINGE_STAGE) != hipSuccess) {
     (void)hipGetLastError();
     return fail(c, RBH_E_HIP, "hinge solve cannot use " + std::to_string(hbytes) + " bytes of LDS");
   }
@@ -1023,15 +1026,15 @@ template <typename R> int setup_solve_lds(rbh_ctx* c) {
 template <typename R> int run_steps(rbh_ctx* c, int n_steps, double dt, int flags) {
   c->any_post = false;
   c->any_hinge = false;
-  c->hinge_lds = 16;
+  std::vector<int> h_bodies, h_hinges;   // of the hinged scenes
   for (int slot : c->batch) {
     const SceneParams& sp = c->sp_host[slot];
     c->any_post = c->any_post || c->scenes[slot].params.use_post_stabilization != 0;
     c->any_hinge = c->any_hinge || sp.h_cnt > 0;
-    if (sp.h_cnt > 0)
-      c->hinge_lds = std::max(c->hinge_lds, hinge_staged<R>(sp.hb_cnt, sp.h_cnt) ? HingeLds<R>::bytes(sp.hb_cnt, sp.h_cnt)
-                                                                                : hinge_lds_bytes<R>(sp.hb_cnt, sp.h_cnt));
+    if (sp.h_cnt > 0) { h_bodies.push_back(sp.hb_cnt); h_hinges.push_back(sp.h_cnt); }
   }
+  if (c->any_hinge)
+    c->hinge = hinge_launch<R>(c->prop.multiProcessorCount, (int)h_bodies.size(), h_bodies.data(), h_hinges.data());
   const bool timing = (flags & RBH_STEP_TIMING) != 0;
   const bool use_graph = (flags & RBH_STEP_GRAPH) != 0;
   const int kflags = flags & RBH_STEP_COUNT_OVERLAPS;
@@ -1524,6 +1527,30 @@ int rbh_prefix_sum(rbh_ctx* c, const void* in, int elem_bytes, int n, int cap, i
   if (e != hipSuccess) return fail(c, RBH_E_HIP, std::string("prefix sum: ") + hipGetErrorString(e));
   if (tail[1] & ERR_SCAN) return fail(c, RBH_E_HIP, "prefix sum: a tile's wait for its predecessors timed out");
   *total = tail[0];
+  return 0;
+}
+
+int rbh_hinge_launch(int precision_bytes, int cus, int n, const int* bodies, const int* hinges, int* staged,
+                     long long* lds, int* rows_at) {
+  if ((precision_bytes != 4 && precision_bytes != 8) || cus < 1 || n < 1 || !bodies || !hinges || !staged || !lds || !rows_at)
+    return RBH_E_ARG;
+  const bool f = precision_bytes == 4;
+  const HingeLaunch h = f ? hinge_launch<float>(cus, n, bodies, hinges) : hinge_launch<double>(cus, n, bodies, hinges);
+  *staged = h.staged ? 1 : 0;
+  *lds = (long long)h.lds;
+  for (int i = 0; i < n; ++i)
+    rows_at[i] = (int)(f ? HingeLds<float>::rows_at(bodies[i], hinges[i]) : HingeLds<double>::rows_at(bodies[i], hinges[i]));
+  return 0;
+}
+
+int rbh_hinge_occupancy(rbh_ctx* c, int staged, long long lds, int* groups_per_cu) {
+  if (!c || !groups_per_cu || lds < 0 || lds > (long long)HINGE_STAGE) return fail(c, RBH_E_ARG, "bad occupancy arguments");
+  (void)hipSetDevice(c->device);
+  const void* k = c->prec == 4 ? (staged ? reinterpret_cast<const void*>(k_hinge_solve<float, true>)
+                                         : reinterpret_cast<const void*>(k_hinge_solve<float, false>))
+                               : (staged ? reinterpret_cast<const void*>(k_hinge_solve<double, true>)
+                                         : reinterpret_cast<const void*>(k_hinge_solve<double, false>));
+  HIPCHK(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(groups_per_cu, k, 64, (size_t)lds));
   return 0;
 }
 

@@ -19,8 +19,8 @@
 // the five rows update from the same w (hinges.py:88), one lane per row, and
 // the twelve body entries of W J^T delta one lane each.  w, the iterate and
 // the accepted solution stay in LDS, and so do the rows of all hinges where
-// they fit HINGE_STAGE; else the rows of the next HINGE_AHEAD hinges are loaded
-// from memory while one updates.
+// hinge_launch has them staged; else the rows of the next HINGE_AHEAD hinges are
+// loaded from memory while one updates.
 // (included inside namespace rbh by rbh_kernels.h)
 #pragma once
 
@@ -204,7 +204,10 @@ template <typename R> __host__ __device__ constexpr size_t hinge_lds_bytes(int h
 // Chains of 5, 16 and 48 cubes, 100 sweeps, four steps: 1.93, 3.71 and 9.30 ms
 // from memory, 1.83, 3.09 and 6.77 staged.
 // Up to 64 KB, so that at least two scenes of a batch share a CU: a chain of 83
-// hinges in FP32, 42 in FP64.
+// hinges in FP32, 42 in FP64 (which of the batches that fit are staged:
+// hinge_launch).  The two paths are kernels of their own: in one, the rows in
+// registers of one and of the other left the path from memory one wavefront a
+// SIMD instead of two (256 links 12.5 ms a step, alone 11.3).
 constexpr size_t HINGE_STAGE = 64 * 1024;
 
 template <typename R> struct HingeLds {
@@ -212,14 +215,16 @@ template <typename R> struct HingeLds {
   int wl, wa, x;             // as in the kernel's layout
   int J, WJ, ids, br, off, inc;   // rows of J (body of lower index first), of W J^T, int4 (parent, child, first, second
                                   // slot), b and r0, the bodies' hinge lists
+  // where the rows start
+  __host__ __device__ static constexpr size_t rows_at(int hb, int nh) { return hinge_lds_bytes<R>(hb, nh); }
   __host__ __device__ static constexpr size_t bytes(int hb, int nh) {
-    return hinge_lds_bytes<R>(hb, nh) + (size_t)nh * (40 * VB + 16 + 10 * SR + 8) + 4 * ((size_t)hb + 1);
+    return rows_at(hb, nh) + (size_t)nh * (40 * VB + 16 + 10 * SR + 8) + 4 * ((size_t)hb + 1);
   }
   __device__ HingeLds(unsigned char* smem, int hb, int nh) {
     wl = lds_addr(smem);
     wa = wl + hb * VB;
     x = wa + hb * VB;
-    J = wl + (int)hinge_lds_bytes<R>(hb, nh);
+    J = wl + (int)rows_at(hb, nh);
     WJ = J + 20 * nh * VB;
     ids = WJ + 20 * nh * VB;
     br = ids + 16 * nh;
@@ -228,9 +233,22 @@ template <typename R> struct HingeLds {
   }
 };
 
-// dynamic LDS of a scene's hinge solve, staged or not
-template <typename R> __host__ __device__ constexpr bool hinge_staged(int hb, int nh) {
-  return HingeLds<R>::bytes(hb, nh) <= HINGE_STAGE;
+// How a batch's hinge solve is launched: the rows of all its scenes staged, or
+// none; the dynamic LDS of a workgroup.
+struct HingeLaunch {
+  bool staged;
+  size_t lds;
+};
+
+// n hinged scenes of bodies[i] bodies in hinges[i] hinges: staged if they all fit.
+template <typename R>
+HingeLaunch hinge_launch(int cus, int n, const int* bodies, const int* hinges) {
+  size_t mem = 16, st = 16;
+  for (int i = 0; i < n; ++i) {
+    mem = std::max(mem, hinge_lds_bytes<R>(bodies[i], hinges[i]));
+    st = std::max(st, HingeLds<R>::bytes(bodies[i], hinges[i]));
+  }
+  return st <= HINGE_STAGE ? HingeLaunch{true, st} : HingeLaunch{false, mem};
 }
 
 template <typename R> __device__ void hinge_stage(const Dev<R>& d, const SceneParams& sp, const HingeLds<R>& L) {
@@ -343,10 +361,9 @@ template <typename R> __device__ __forceinline__ void hinge_sweep_lds(const Hing
 // One wavefront per batch scene.  pass 0 records the hinge merit
 // contributions for the contact solve; pass 1 runs to the joint stop and
 // writes hd0/hd1 (see the top of this file).  w, x and the accepted
-// solution sol live in LDS.
-template <typename R> __global__ void __launch_bounds__(64) k_hinge_solve(Dev<R> d, int pass) {
+// solution sol live in LDS, and, STAGED, the rows too.
+template <typename R, bool STAGED> __global__ void __launch_bounds__(64) k_hinge_solve(Dev<R> d, int pass) {
   extern __shared__ __align__(16) unsigned char hinge_smem[];
-  __shared__ R s_delta[5];
   if (aborted(d.err)) return;
   const int slot = d.bs_slot[blockIdx.x];
   const SceneParams& sp = d.sp[slot];
@@ -364,9 +381,8 @@ template <typename R> __global__ void __launch_bounds__(64) k_hinge_solve(Dev<R>
   R* sol = x + nrow;
   double* res = d.residuals + sp.res_off;
   double* hm = d.h_mer + sp.res_off;
-  const bool staged = hinge_staged<R>(sp.hb_cnt, sp.h_cnt);   // uniform; the launch has room for it
-  const HingeLds<R> L(hinge_smem, sp.hb_cnt, sp.h_cnt);
-  if (staged) hinge_stage(d, sp, L);
+  const HingeLds<R> L(hinge_smem, sp.hb_cnt, sp.h_cnt);   // (STAGED: the launch has room for it)
+  if constexpr (STAGED) hinge_stage(d, sp, L);
   for (int i = lane; i < nrow; i += 64) { x[i] = R(0); sol[i] = R(0); }
   if (own)
     for (int i = lane; i < sp.max_iter; i += 64) res[i] = INFINITY;
@@ -376,12 +392,13 @@ template <typename R> __global__ void __launch_bounds__(64) k_hinge_solve(Dev<R>
   ctl.iters = sp.max_iter;
   for (int it = 0; it < n_it; ++it) {
     const R rs = R(ctl.rscale);
-    if (staged) {
+    if constexpr (STAGED) {
       hinge_body_w_lds(L, sp.hb_cnt, L.x);
       __syncthreads();
       hinge_sweep_lds(L, sp.h_cnt, rs);
       __syncthreads();
     } else {
+      __shared__ R s_delta[5];
       hinge_body_w(d, sp, x, wl, wa);
       // rows of the next HINGE_AHEAD hinges in flight while one updates
       HingeRegs<R> ring[HINGE_AHEAD];
@@ -425,7 +442,7 @@ template <typename R> __global__ void __launch_bounds__(64) k_hinge_solve(Dev<R>
     st.final_merit = ctl.last_merit;
   }
   // finalize_solution (hinges.py:50-57): W J^T sol per body
-  if (staged) hinge_body_w_lds(L, sp.hb_cnt, L.x + nrow * (int)sizeof(R));
+  if constexpr (STAGED) hinge_body_w_lds(L, sp.hb_cnt, L.x + nrow * (int)sizeof(R));
   else hinge_body_w(d, sp, sol, wl, wa);
   __syncthreads();
   for (int j = lane; j < sp.hb_cnt; j += 64) {

@@ -118,6 +118,9 @@ _PROTOS = {
     "rbh_get_tuning": [C.c_void_p, C.c_void_p],
     # include/rbh_testing.h
     "rbh_prefix_sum": [C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_void_p, C.POINTER(C.c_int)],
+    "rbh_hinge_launch": [C.c_int, C.c_int, C.c_int, C.c_void_p, C.c_void_p, C.POINTER(C.c_int),
+                         C.POINTER(C.c_longlong), C.c_void_p],
+    "rbh_hinge_occupancy": [C.c_void_p, C.c_int, C.c_longlong, C.POINTER(C.c_int)],
     "rbh_prox_ellipsoid": [C.c_void_p, C.c_int, C.c_void_p, C.c_void_p, C.c_void_p, C.c_double, C.c_double, C.c_int,
                            C.c_void_p],
 }
@@ -157,6 +160,18 @@ def _f64(a, n=None):
 
 def _i32(a):
     return np.ascontiguousarray(a, dtype=np.int32)
+
+
+def hinge_launch(precision, cus, bodies, hinges):
+    """The hinge solve's launch for scenes of these sizes: (staged, LDS bytes, where each scene's rows start); a
+    test hook (include/rbh_testing.h)."""
+    bodies, hinges = _i32(bodies), _i32(hinges)
+    staged, lds, rows = C.c_int(), C.c_longlong(), np.empty(len(bodies), np.int32)
+    rc = load().rbh_hinge_launch({"fp32": 4, "fp64": 8}[precision], int(cus), len(bodies), _ptr(bodies), _ptr(hinges),
+                                 C.byref(staged), C.byref(lds), _ptr(rows))
+    if rc != 0:
+        raise RbhError(rc, "bad hinge sizes")
+    return bool(staged.value), int(lds.value), rows
 
 
 class Context:
@@ -232,6 +247,12 @@ class Context:
         self._check(self.lib.rbh_prefix_sum(self.h, a.ctypes.data_as(C.c_void_p), a.dtype.itemsize, n, cap,
                                             out.ctypes.data_as(C.c_void_p), C.byref(tot)))
         return out, tot.value
+
+    def hinge_occupancy(self, staged, lds):
+        """Workgroups of the hinge solve per compute unit (a test hook, include/rbh_testing.h)."""
+        n = C.c_int()
+        self._check(self.lib.rbh_hinge_occupancy(self.h, int(staged), int(lds), C.byref(n)))
+        return n.value
 
     def prox_ellipsoid(self, z, mu, xn, tolerance, expansion, max_iterations):
         """The sweeps' ellipsoid projection of z (n, 3) (a test hook, include/rbh_testing.h)."""
