@@ -215,8 +215,10 @@ template <typename R> struct HingeLds {
   int wl, wa, x;             // as in the kernel's layout
   int J, WJ, ids, br, off, inc;   // rows of J (body of lower index first), of W J^T, int4 (parent, child, first, second
                                   // slot), b and r0, the bodies' hinge lists
-  // where the rows start
-  __host__ __device__ static constexpr size_t rows_at(int hb, int nh) { return hinge_lds_bytes<R>(hb, nh); }
+  // where the rows start: a whole vec4 (an odd number of hinges leaves half of one in FP64)
+  __host__ __device__ static constexpr size_t rows_at(int hb, int nh) {
+    return (hinge_lds_bytes<R>(hb, nh) + VB - 1) / VB * VB;
+  }
   __host__ __device__ static constexpr size_t bytes(int hb, int nh) {
     return rows_at(hb, nh) + (size_t)nh * (40 * VB + 16 + 10 * SR + 8) + 4 * ((size_t)hb + 1);
   }
@@ -363,7 +365,7 @@ template <typename R> __device__ __forceinline__ void hinge_sweep_lds(const Hing
 // writes hd0/hd1 (see the top of this file).  w, x and the accepted
 // solution sol live in LDS, and, STAGED, the rows too.
 template <typename R, bool STAGED> __global__ void __launch_bounds__(64) k_hinge_solve(Dev<R> d, int pass) {
-  extern __shared__ __align__(16) unsigned char hinge_smem[];
+  extern __shared__ __align__(32) unsigned char hinge_smem[];
   if (aborted(d.err)) return;
   const int slot = d.bs_slot[blockIdx.x];
   const SceneParams& sp = d.sp[slot];
