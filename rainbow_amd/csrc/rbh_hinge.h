@@ -242,15 +242,34 @@ struct HingeLaunch {
   size_t lds;
 };
 
-// n hinged scenes of bodies[i] bodies in hinges[i] hinges: staged if they all fit.
+// n hinged scenes of bodies[i] bodies in hinges[i] hinges on `cus` compute units.
+//
+// Staged, an update takes 1 / 1.5 of its time from memory as long as a CU has one
+// scene; but a scene's workgroup keeps its rows' LDS, so R = LDS / its bytes of
+// them share a CU, where up to W = 8 (FP64 4, by their registers) share it from
+// memory, at 1.3 + 0.2 w of the staged time for w of them (80 links, 30 sweeps:
+// 256 scenes 1.4 ms a step, 512 1.9, 1,024 2.3, 1,280 2.3, 2,048 2.8; staged, with
+// R = 2, 1.0, 1.1, 1.9, 2.8 and 3.9).  Either way takes as long as the longest
+// scene, or as the CU's scenes R or W at a time; the shorter way is taken.  Short
+// scenes stay staged at any number (2,048 of 40 links 1.4 against 1.6, 4,096 of
+// 20 1.6 against 2.0, 2,048 of 40 in FP64 2.5 against 3.1).
 template <typename R>
 HingeLaunch hinge_launch(int cus, int n, const int* bodies, const int* hinges) {
   size_t mem = 16, st = 16;
+  double all = 0.0, longest = 0.0;
   for (int i = 0; i < n; ++i) {
     mem = std::max(mem, hinge_lds_bytes<R>(bodies[i], hinges[i]));
     st = std::max(st, HingeLds<R>::bytes(bodies[i], hinges[i]));
+    all += hinges[i];
+    longest = std::max(longest, (double)hinges[i]);
   }
-  return st <= HINGE_STAGE ? HingeLaunch{true, st} : HingeLaunch{false, mem};
+  if (st > HINGE_STAGE) return HingeLaunch{false, mem};
+  const double per_cu = all / cus;                                  // updates a CU has to do
+  const double scenes = (double)((n + (long)cus - 1) / cus);        // its scenes
+  const double r = std::floor(160.0 * 1024.0 / (double)st), w = std::min(scenes, sizeof(R) == 4 ? 8.0 : 4.0);
+  const double t_staged = std::max(longest, std::ceil(scenes / r) * per_cu / scenes);
+  const double t_memory = std::max(1.5 * longest, per_cu * (1.3 + 0.2 * w) / w);
+  return t_staged <= t_memory ? HingeLaunch{true, st} : HingeLaunch{false, mem};
 }
 
 template <typename R> __device__ void hinge_stage(const Dev<R>& d, const SceneParams& sp, const HingeLds<R>& L) {
