@@ -30,6 +30,11 @@ int rbh_prefix_sum(rbh_ctx* ctx, const void* in, int elem_bytes, int n, int cap,
 int rbh_prox_ellipsoid(rbh_ctx* ctx, int n, const double* z, const double* mu, const double* xn, double tolerance,
                        double expansion, int max_iterations, double* out);
 
+/* Workgroups of a lone scene's solve (no device needed): `units` colouring
+ * units in the last step seen (0: none), rbh_tuning's lanes_per_group, and the
+ * most workgroups that are resident at once. */
+int rbh_coop_grid(int units, int lanes_per_group, int most);
+
 /* How the hinge solve of a batch would be launched (no device needed): n
  * hinged scenes of bodies[i] bodies in hinges[i] hinges on `cus` compute units.
  * *staged: 1 if their rows are staged in LDS; *lds: bytes of a workgroup;

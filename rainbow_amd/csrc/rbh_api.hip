@@ -821,6 +821,21 @@ template <typename T> bool scan(rbh_ctx* c, const T* in, int* out, const int* n_
   return true;
 }
 
+// Workgroups of a lone scene's cooperative solve, from the unit count of the
+// last step seen (0: none seen, or one without contacts, whose next step may
+// have any number): one lane per workgroup while the device has room for them, so
+// that a lane's wavefront shares its CU's LDS with no other and few groups outgrow
+// the resident layout (4096 spheres: solve 875 us, with four lanes per workgroup
+// 1137); but one workgroup for as many lanes as it has wavefronts, which spares the
+// exchange of the merit through memory (2.5 us of a sweep: 64 boxes in 3 lanes, 100
+// sweeps, 403 us in one workgroup, 447 in three).
+int coop_grid(int units, int lanes_per_group, int most) {
+  if (units <= 0) units = 64;
+  if (lanes_per_group == 0 && units <= SOLVE_BLOCK / 64) return 1;
+  const int per = lanes_per_group > 0 ? lanes_per_group : 1;
+  return std::max(1, std::min((units + per - 1) / per, most));
+}
+
 // steps between re-sizings of a single scene's cooperative solve grid
 constexpr int GRID_REFRESH = 16;
 
@@ -1056,17 +1071,7 @@ template <typename R> int run_steps(rbh_ctx* c, int n_steps, double dt, int flag
   bool multi = c->multi_ok && !use_graph;
   if (flags & RBH_STEP_FORCE_SINGLE) multi = false;
   if ((flags & RBH_STEP_FORCE_MULTI) && c->multi_ok && !use_graph) multi = true;
-  // cooperative grid, from the unit count of the last step seen: one lane per workgroup while the device
-  // has room for them, so that a lane's wavefront shares its CU's LDS with no other and few groups outgrow
-  // the resident layout (4096 spheres: solve 875 us, with four lanes per workgroup 1137); but one workgroup
-  // for as many lanes as it has wavefronts, which spares the exchange of the merit through memory (2.5 us
-  // of a sweep: 64 boxes in 3 lanes, 100 sweeps, 403 us in one workgroup, 447 in three)
-  const int lpw = c->tune.lanes_per_group > 0 ? c->tune.lanes_per_group : 1;
-  auto grid_of = [&](int units) {
-    if (c->tune.lanes_per_group == 0 && units <= SOLVE_BLOCK / 64) return 1;
-    return std::max(1, std::min((units + lpw - 1) / lpw, c->coop_max));
-  };
-  int multi_grid = grid_of(c->last_units > 1 ? c->last_units : 64);
+  int multi_grid = coop_grid(c->last_units, c->tune.lanes_per_group, c->coop_max);
   int done = 0;
   StepEnd end{};
   for (int attempt = 0; attempt < 16 && done < n_steps; ++attempt) {
@@ -1104,7 +1109,7 @@ template <typename R> int run_steps(rbh_ctx* c, int n_steps, double dt, int flag
           int nu = 0;
           HIPCHK(c, hipMemcpyAsync(&nu, c->n_units.p, 4, hipMemcpyDeviceToHost, c->stream));
           HIPCHK(c, hipStreamSynchronize(c->stream));
-          if (nu > 0) multi_grid = grid_of(nu);
+          if (nu > 0) multi_grid = coop_grid(nu, c->tune.lanes_per_group, c->coop_max);
         }
       }
     }
@@ -1133,7 +1138,7 @@ template <typename R> int run_steps(rbh_ctx* c, int n_steps, double dt, int flag
     if (rc) return rc;
   }
   if (done < n_steps) return fail(c, RBH_E_CAPACITY, "step workspace could not grow enough");
-  c->last_units = std::max(1, end.units);
+  c->last_units = end.units;
   for (int i = 0; i < 4; ++i) c->counters[i] = end.counts[i];
   if (timing) {
     // average over the timed steps of the last attempt; a graph replay has no stage marks
@@ -1528,6 +1533,11 @@ int rbh_prefix_sum(rbh_ctx* c, const void* in, int elem_bytes, int n, int cap, i
   if (tail[1] & ERR_SCAN) return fail(c, RBH_E_HIP, "prefix sum: a tile's wait for its predecessors timed out");
   *total = tail[0];
   return 0;
+}
+
+int rbh_coop_grid(int units, int lanes_per_group, int most) {
+  if (units < 0 || lanes_per_group < 0 || most < 1) return RBH_E_ARG;
+  return coop_grid(units, lanes_per_group, most);
 }
 
 int rbh_hinge_launch(int precision_bytes, int cus, int n, const int* bodies, const int* hinges, int* staged,
