@@ -41,7 +41,7 @@ def batch_candidates():
 def single_candidates():
     """Shapes for one scene stepped alone by the cooperative grid (default first)."""
     out = []
-    for lpg, unit in itertools.product((4, 2, 1), (64, 128, 256)):
+    for lpg, unit in itertools.product((0, 4, 2, 1), (64, 128, 256)):   # (0: by the scene's unit count)
         out.append(dict(lanes_per_group=lpg, unit_size=unit))
     return out
 
