@@ -13,6 +13,14 @@
  * caller-owned host memory, C order, FP64 unless stated.  Body indices are
  * local to their scene (insertion order of engine.bodies).  A context owns
  * one HIP stream on one device and is not thread-safe.
+ *
+ * rbh_scene_create, rbh_scene_set_state and rbh_scene_set_step_index copy the
+ * caller's arrays and return with their uploads queued in the context's
+ * stream: the arrays may be reused at once, later calls see the new values,
+ * and a device error may be reported by the next call that waits (one that
+ * reads back, rbh_step, rbh_sync).  Such transfers go through pinned host memory
+ * that the context holds, 1 MiB at first and at most 64 MiB; larger ones are
+ * copied from pageable memory and waited for.
  */
 #ifndef RBH_H
 #define RBH_H

@@ -30,6 +30,9 @@ int rbh_prefix_sum(rbh_ctx* ctx, const void* in, int elem_bytes, int n, int cap,
 int rbh_prox_ellipsoid(rbh_ctx* ctx, int n, const double* z, const double* mu, const double* xn, double tolerance,
                        double expansion, int max_iterations, double* out);
 
+/* Pinned host memory the context holds for its transfers. */
+int rbh_transfer_buffer(rbh_ctx* ctx, unsigned long long* bytes);
+
 /* Workgroups of a lone scene's solve (no device needed): `units` colouring
  * units in the last step seen (0: none), rbh_tuning's lanes_per_group, and the
  * most workgroups that are resident at once. */

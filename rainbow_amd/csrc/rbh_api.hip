@@ -17,6 +17,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstddef>
+#include <cstdlib>
 #include <cstring>
 #include <mutex>
 #include <string>
@@ -248,7 +249,11 @@ int ensure(rbh_ctx* c, DBuf& b, size_t bytes, bool keep = false) {
 // about 5; the whole pass 101 -> 61 ms, one step of five hinges 850 -> 575 us).
 // Uploads are in stream order and not waited for; their bytes
 // stay in the pinned buffer until the stream has been waited for.
+// The context keeps at most PIN_MAX of it.  A larger transfer, or one for which
+// the host has no pinned memory, is copied range by range through
+// memory of its own and waited for.
 constexpr int MOVE_MAX = 16;
+constexpr size_t PIN_MAX = (size_t)64 << 20;
 struct Moves {
   unsigned* dev[MOVE_MAX];
   int words[MOVE_MAX], off[MOVE_MAX];   // 4-byte words, and where they lie in the pinned block
@@ -267,40 +272,52 @@ __global__ void k_moves(Moves m, unsigned* pin, bool up) {
 class Transfer {
  public:
   explicit Transfer(rbh_ctx* c_) : c(c_) {}
+  ~Transfer() { std::free(own); }
+  Transfer(const Transfer&) = delete;
+  Transfer& operator=(const Transfer&) = delete;
   // one more range of `bytes` (a multiple of 4)
   void add(void* dev, size_t bytes) {
-    m.dev[n] = static_cast<unsigned*>(dev);
-    m.words[n] = (int)(bytes / 4);
-    m.off[n] = (int)(total / 4);
+    range[n++] = Range{dev, bytes, total};
     total += (bytes + 31) / 32 * 32;
-    ++n;
   }
-  // room in the pinned buffer for the ranges added
+  // room for the ranges added
   int reserve() {
     HIPCHK(c, hipSetDevice(c->device));   // for the launch: some callers only read, with another device current
     if (c->pin_used + total > c->pin_bytes) {
       HIPCHK(c, hipStreamSynchronize(c->stream));
       c->pin_used = 0;
-      if (total > c->pin_bytes) {
-        const size_t want = std::max<size_t>(total + total / 2, 1 << 20);
+      if (total > c->pin_bytes && total <= PIN_MAX) {
+        const size_t want = std::min(std::max<size_t>(total + total / 2, 1 << 20), PIN_MAX);
         if (c->pin) HIPCHK(c, hipHostFree(c->pin));
         c->pin = nullptr;
         c->pin_bytes = 0;
-        HIPCHK(c, hipHostMalloc(reinterpret_cast<void**>(&c->pin), want, hipHostMallocMapped | hipHostMallocCoherent));
-        c->pin_bytes = want;
+        if (hipHostMalloc(reinterpret_cast<void**>(&c->pin), want, hipHostMallocMapped | hipHostMallocCoherent) == hipSuccess) {
+          c->pin_bytes = want;
+        } else {
+          (void)hipGetLastError();
+          c->pin = nullptr;
+        }
       }
     }
-    base = c->pin + c->pin_used;
-    c->pin_used += total;
-    return 0;
+    if (total <= c->pin_bytes) {
+      base = c->pin + c->pin_used;
+      c->pin_used += total;
+      return 0;
+    }
+    base = own = static_cast<unsigned char*>(std::malloc(total));
+    return own ? 0 : fail(c, RBH_E_MEMORY, "no host memory for a transfer of " + std::to_string(total) + " bytes");
   }
-  template <typename T> T* host(int i) const { return reinterpret_cast<T*>(base + 4 * (size_t)m.off[i]); }
+  template <typename T> T* host(int i) const { return reinterpret_cast<T*>(base + range[i].at); }
   // after the host has written its side
-  int up() { return launch(true); }
-  // the device's side, in the pinned block until the next transfer
+  int up() {
+    const int rc = own ? copy(hipMemcpyHostToDevice) : launch(true);
+    if (!rc && own) HIPCHK(c, hipStreamSynchronize(c->stream));
+    return rc;
+  }
+  // the device's side, until the next transfer
   int down() {
     int rc = reserve();
-    if (!rc) rc = launch(false);
+    if (!rc) rc = own ? copy(hipMemcpyDeviceToHost) : launch(false);
     if (rc) return rc;
     HIPCHK(c, hipStreamSynchronize(c->stream));
     c->pin_used = 0;
@@ -308,14 +325,30 @@ class Transfer {
   }
 
  private:
+  struct Range { void* dev; size_t bytes, at; };   // at: where it lies in the host block
   rbh_ctx* c;
-  Moves m{};
+  Range range[MOVE_MAX];
   int n = 0;
   size_t total = 0;
-  unsigned char* base = nullptr;
+  unsigned char *base = nullptr, *own = nullptr;   // the host block; this transfer's own
+  int copy(hipMemcpyKind kind) {
+    for (int i = 0; i < n; ++i) {
+      void *dev = range[i].dev, *here = base + range[i].at;
+      const bool in = kind == hipMemcpyHostToDevice;
+      if (range[i].bytes > 0)
+        HIPCHK(c, hipMemcpyAsync(in ? dev : here, in ? here : dev, range[i].bytes, kind, c->stream));
+    }
+    return 0;
+  }
   int launch(bool up) {
+    Moves m{};
     int most = 0;
-    for (int i = 0; i < n; ++i) most = std::max(most, m.words[i]);
+    for (int i = 0; i < n; ++i) {
+      m.dev[i] = static_cast<unsigned*>(range[i].dev);
+      m.words[i] = (int)(range[i].bytes / 4);
+      m.off[i] = (int)(range[i].at / 4);
+      most = std::max(most, m.words[i]);
+    }
     if (most == 0) return 0;
     void* dev = nullptr;
     HIPCHK(c, hipHostGetDevicePointer(&dev, base, 0));
@@ -1532,6 +1565,12 @@ int rbh_prefix_sum(rbh_ctx* c, const void* in, int elem_bytes, int n, int cap, i
   if (e != hipSuccess) return fail(c, RBH_E_HIP, std::string("prefix sum: ") + hipGetErrorString(e));
   if (tail[1] & ERR_SCAN) return fail(c, RBH_E_HIP, "prefix sum: a tile's wait for its predecessors timed out");
   *total = tail[0];
+  return 0;
+}
+
+int rbh_transfer_buffer(rbh_ctx* c, unsigned long long* bytes) {
+  if (!c || !bytes) return RBH_E_ARG;
+  *bytes = c->pin_bytes;
   return 0;
 }
 

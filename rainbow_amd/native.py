@@ -118,6 +118,7 @@ _PROTOS = {
     "rbh_get_tuning": [C.c_void_p, C.c_void_p],
     # include/rbh_testing.h
     "rbh_prefix_sum": [C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_void_p, C.POINTER(C.c_int)],
+    "rbh_transfer_buffer": [C.c_void_p, C.POINTER(C.c_ulonglong)],
     "rbh_coop_grid": [C.c_int, C.c_int, C.c_int],
     "rbh_hinge_launch": [C.c_int, C.c_int, C.c_int, C.c_void_p, C.c_void_p, C.POINTER(C.c_int),
                          C.POINTER(C.c_longlong), C.c_void_p],
