@@ -176,7 +176,7 @@ struct rbh_ctx {
   int scan_site = 0;         // scans launched so far in the step being enqueued
   int unit_T = 64;          // contacts per colouring unit (a scene's units are windows of this size)
   rbh_tuning tune{};        // rbh_set_tuning (0 fields: defaults)
-  // resident solve groups: LDS capacities (contacts, bodies, colour offsets) and the launch's dynamic LDS
+  // resident solve groups: most contacts and bodies (rbh_tuning), and the launch's dynamic LDS
   int res_cap_c = 0, res_cap_b = 0;
   size_t solve_lds = 0, solve_lds_half = 0;   // full and half layouts (one or two workgroups per CU)
   int max_iter_batch = 1, coop_max = 0, last_units = 0;

@@ -207,8 +207,8 @@ __global__ void __launch_bounds__(SDF_BLOCK) k_sdf(const double* __restrict__ tr
 //    expression, so the minimum is the same.
 //  * Sign: away from the surface of a closed mesh the winding number is constant.
 //    Two neighbouring nodes lie on the same side if either is farther from the
-//    surface than from the other, rounding included; nodes are joined so into trees, and the
-//    winding number is taken once per tree.  Nodes on the surface itself join
+//    surface than from the other, rounding included; nodes are joined so into
+//    trees, and the winding number is taken once per tree.  Nodes on the surface itself join
 //    no other.  Closed: every edge (vertices welded by position) is used as
 //    often in one direction as in the other; for any other (open) mesh every
 //    node is a tree of its own.
@@ -244,6 +244,7 @@ struct SdfWork {
   double* out;               // per node: distance, then signed
 };
 
+// MurmurHash3's 64-bit finalizer (Austin Appleby, public domain)
 __device__ __forceinline__ unsigned sdf_mix(unsigned long long x) {
   x ^= x >> 33; x *= 0xff51afd7ed558ccdull; x ^= x >> 33; x *= 0xc4ceb9fe1a85ec53ull; x ^= x >> 33;
   return (unsigned)x;

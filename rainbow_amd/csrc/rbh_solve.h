@@ -7,11 +7,12 @@
 // packed into colouring units of at most unit_T contacts that never straddle
 // a scene.  Each unit is coloured by one workgroup with its state in LDS.
 //
-// The sweep order is fixed by the colours alone (colours in increasing value;
-// contacts of one colour share no free body), so two schedules give bitwise
-// the same iterates: one workgroup per scene (batched scenes), or one
-// workgroup per unit with a grid barrier per sweep for the scene-wide merit
-// (a single large scene).
+// Every body's contacts are solved in the order of their colours (contacts of
+// one colour share no free body; serial Gauss-Seidel: of their indices), and the
+// iterates depend on nothing else.  All schedules keep that order, so all give
+// bitwise the same iterates: dependency levels or colours, one workgroup per
+// scene (batched scenes), or lanes spread over many workgroups, whose merits
+// meet once per sweep (a single large scene).
 #pragma once
 // (included inside namespace rbh by rbh_kernels.h)
 
@@ -1250,7 +1251,7 @@ template <typename R> __global__ void k_post_integrate(Dev<R> d) {
   d.q[b] = V4<R>{qn.s, qn.x, qn.y, qn.z};
 }
 
-// colour offsets of lane l: 2 K_l + 2 entries (an island's colours stay below
+// level or colour offsets of lane l: 2 K_l + 2 entries (an island's colours stay below
 // twice its size, which the colouring checks)
 template <typename R> __device__ __forceinline__ const int* lane_coff(const Dev<R>& d, int l) {
   return d.col_off + 2 * ((size_t)d.l_start[l] + l);
@@ -1335,8 +1336,9 @@ __device__ __forceinline__ void order_phases(const Dev<R>& d, int l, int nl, con
 // is one more than the highest level of the earlier contacts of its two free
 // bodies -- which keeps every body's order (so the iterates are bitwise the
 // same) in as few phases as that order allows: the colours of a random
-// colouring leave gaps at every body, 146 colours against 106 levels on a
-// 1,500-sphere pile, 345 against 277 on 48 meshes, and serial Gauss-Seidel has
+// colouring leave gaps at every body (an island of 677 contacts in a
+// 1,500-sphere pile has 114 colours, 93 of them with contacts, and 79 levels;
+// one of 1,255 in 48 meshes 345, 306 and 268), and serial Gauss-Seidel has
 // one "colour" per contact.  Levels are found by one wavefront walking the
 // colours (about 260 cycles each) over LDS tables; a lane too large for them
 // keeps its colours.  l_ncol and the colour offsets then count levels.
@@ -2631,7 +2633,7 @@ __device__ void solve_group_resident(const Dev<R>& d, const int slot, const Grou
 // records of a phase are read from global memory two phases ahead, each lane
 // its own row and block, in three register buffers used in turn; a quad
 // without a contact reads the null record after the last one.  Bound by the
-// phase's chain (phase_update) as long as the records come from L2.  With rows
+// phase's chain (QuadPhase::update) as long as the records come from L2.  With rows
 // loaded one phase ahead, the block's rows in the phase itself and lanes of
 // more than 512 contacts always swept by the workgroup, the solve took: 24
 // scenes of ~2,100 contacts 6859 us (now 1406), 320 of ~330 1960 (977),
@@ -2800,7 +2802,7 @@ template <typename R, int NT, int H> __global__ void __launch_bounds__(NT) k_sol
   SceneState& st = d.ss[slot];
   if (d.post && !(sp.use_post_stab && st.post_active)) return;
   double* res = residual_record(d, sp);
-    for (int i = threadIdx.x; i < sp.max_iter; i += NT) res[i] = INFINITY;
+  for (int i = threadIdx.x; i < sp.max_iter; i += NT) res[i] = INFINITY;
   if (st.k_cnt == 0) {
     if (threadIdx.x == 0) no_contacts<R>(st);
     return;
