@@ -304,7 +304,7 @@ class Transfer {
       c->pin_used += total;
       return 0;
     }
-    base = own = static_cast<unsigned char*>(std::malloc(total));
+    base = own = static_cast<unsigned char*>(std::aligned_alloc(32, total));   // (total: a multiple of 32)
     return own ? 0 : fail(c, RBH_E_MEMORY, "no host memory for a transfer of " + std::to_string(total) + " bytes");
   }
   template <typename T> T* host(int i) const { return reinterpret_cast<T*>(base + range[i].at); }
