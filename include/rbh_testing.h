@@ -30,6 +30,11 @@ int rbh_prefix_sum(rbh_ctx* ctx, const void* in, int elem_bytes, int n, int cap,
 int rbh_prox_ellipsoid(rbh_ctx* ctx, int n, const double* z, const double* mu, const double* xn, double tolerance,
                        double expansion, int max_iterations, double* out);
 
+/* Whether rbh_sdf_build takes its pruned form for these arguments: 1 or 0 (no
+ * device needed). */
+int rbh_sdf_is_pruned(const double* V, int nv, const int* T, int nt, const double* min_coord, const double* max_coord,
+                      int I, int J, int K);
+
 /* Pinned host memory the context holds for its transfers. */
 int rbh_transfer_buffer(rbh_ctx* ctx, unsigned long long* bytes);
 

@@ -1342,13 +1342,70 @@ template <typename R> int get_contacts(rbh_ctx* c, const SceneHost& s, const Sce
 }
 
 // ------------------------------------------------------------ signed distances
-// The pruned build (rbh_sdf.h) has ~100 us of launches and set-up; the plain one
-// takes about 0.48 us per triangle up to ~55,000 nodes, in proportion beyond
-// (12 triangles on 32^3: plain 61 us in all; 448 on 32^3: 457 plain, 320
-// pruned; 10,000 on 64^3: 23.4 ms plain, 1.3 pruned).
-bool sdf_pruned(int nv, int nt, long n, double most) {
+// Whether every edge is used as often in one direction as in the other, of at
+// most SDF_FEW triangles, corners named by id(c); by hashing, without allocation.
+constexpr int SDF_FEW = 384, SDF_TABLE = 2048;   // (a table holds at most 3 nt edges or corners)
+unsigned sdf_table_bits(int nt) {
+  unsigned b = 8;
+  while ((1 << b) < 4 * nt) ++b;
+  return b;
+}
+template <typename Id> bool sdf_balanced(int nt, Id&& id) {
+  const unsigned bits = sdf_table_bits(nt), mask = (1u << bits) - 1u;
+  unsigned long long key[SDF_TABLE];
+  int bal[SDF_TABLE], used[3 * SDF_FEW], n = 0, open = 0;
+  std::memset(key, 0xff, sizeof(key[0]) << bits);
+  for (int t = 0; t < nt; ++t)
+    for (int e = 0; e < 3; ++e) {
+      const unsigned a = (unsigned)id(3 * t + e), b = (unsigned)id(3 * t + (e + 1) % 3);
+      if (a == b) continue;
+      const unsigned long long k = (unsigned long long)std::min(a, b) << 32 | std::max(a, b);
+      unsigned s = (unsigned)((k * 0x9e3779b97f4a7c15ull) >> (64 - bits));
+      while (key[s] != ~0ull && key[s] != k) s = (s + 1) & mask;
+      if (key[s] == ~0ull) { key[s] = k; bal[s] = 0; used[n++] = (int)s; }
+      bal[s] += a < b ? 1 : -1;
+    }
+  for (int i = 0; i < n; ++i) open |= bal[used[i]];
+  return open == 0;
+}
+
+// Whether a mesh of at most SDF_FEW triangles is closed: by its vertices, or with
+// vertices at one position taken as one.
+bool sdf_closed(const double* V, const int* T, int nt) {
+  if (sdf_balanced(nt, [&](int c) { return T[c]; })) return true;
+  const unsigned bits = sdf_table_bits(nt), mask = (1u << bits) - 1u;
+  int first[SDF_TABLE], same[3 * SDF_FEW];   // table of corners; per corner the first of its position
+  bool merged = false;
+  std::fill(first, first + mask + 1, -1);
+  for (int c = 0; c < 3 * nt; ++c) {
+    const double* a = V + 3 * (size_t)T[c];
+    const double x[3] = {a[0] + 0.0, a[1] + 0.0, a[2] + 0.0};   // (-0 as +0)
+    unsigned long long h = 0, word;
+    for (double v : x) { std::memcpy(&word, &v, 8); h = (h ^ word) * 0x9e3779b97f4a7c15ull; h ^= h >> 29; }
+    for (unsigned s = (unsigned)(h >> (64 - bits));; s = (s + 1) & mask) {
+      const double* b = first[s] < 0 ? nullptr : V + 3 * (size_t)T[first[s]];
+      if (!b) first[s] = c;
+      if (!b || (b[0] == a[0] && b[1] == a[1] && b[2] == a[2])) { same[c] = first[s]; break; }
+    }
+    merged = merged || T[same[c]] != T[c];
+  }
+  return merged && sdf_balanced(nt, [&](int c) { return same[c]; });
+}
+
+// Whether a build is the pruned one (rbh_sdf.h).  That has ~100 us of launches and
+// set-up; the plain one takes about 0.48 us per triangle up to ~55,000 nodes, in
+// proportion beyond (12 triangles on 32^3: plain 61 us in all; 448 on 32^3: 457
+// plain, 320 pruned; 10,000 on 64^3: 23.4 ms plain, 1.3 pruned).  Few triangles
+// leave it little to prune: 12 on 128^3 1.22 ms plain, 1.51 pruned; 30 1.54, 1.77;
+// 48 1.89, 1.93; 96 2.66, 2.26; 70 on 54^3 0.24, 0.26.  Of an open mesh every node
+// has its own winding number, so of few triangles it is not worth it either, but
+// on small grids, where the plain build leaves the device idle: 125 on 48^3 0.24
+// plain, 0.32 pruned; 260 strewn ones on 48^3 0.44, 0.50, on 32^3 0.29, 0.24; 500
+// on 48^3 0.78, 0.76.  (The host looks whether one is closed, 2 to 10 us.)
+bool sdf_pruned(const double* V, int nv, const int* T, int nt, long n, double most) {
   if (n >= (1L << 30) || nt >= (1 << 27) || nv >= (1 << 28)) return false;   // 32-bit indices
-  return most >= 1e-60 && (double)nt * std::max(n, 55000L) > 1.1e7;
+  if (most < 1e-60 || nt < 64 || (double)nt * std::max(n, 55000L) <= (nt < 128 ? 1.5e7 : 1.1e7)) return false;
+  return nt > SDF_FEW || n < 48000 || sdf_closed(V, T, nt);
 }
 
 // The largest coordinate of a mesh and its grid, 0 if one is not finite or above
@@ -1568,6 +1625,13 @@ int rbh_prefix_sum(rbh_ctx* c, const void* in, int elem_bytes, int n, int cap, i
   return 0;
 }
 
+int rbh_sdf_is_pruned(const double* V, int nv, const int* T, int nt, const double* mn, const double* mx, int I, int J,
+                      int K) {
+  if (!V || !T || !mn || !mx || nv <= 0 || nt <= 0 || I < 2 || J < 2 || K < 2) return RBH_E_ARG;
+  for (int i = 0; i < 3 * nt; ++i) if (T[i] < 0 || T[i] >= nv) return RBH_E_ARG;
+  return sdf_pruned(V, nv, T, nt, (long)I * J * K, sdf_extent(V, nv, mn, mx)) ? 1 : 0;
+}
+
 int rbh_transfer_buffer(rbh_ctx* c, unsigned long long* bytes) {
   if (!c || !bytes) return RBH_E_ARG;
   *bytes = c->pin_bytes;
@@ -1638,7 +1702,7 @@ int rbh_sdf_build(rbh_ctx* c, const double* V, int nv, const int* T, int nt, con
   const long n = (long)I * J * K;
   // one buffer for the call, kept by the context up to SDF_KEEP_BYTES
   const double most = sdf_extent(V, nv, mn, mx);
-  SdfLayout lay(nv, nt, n, most, sdf_pruned(nv, nt, n, most));
+  SdfLayout lay(nv, nt, n, most, sdf_pruned(V, nv, T, nt, n, most));
   for (bool got = lay.total <= c->sdf_buf_bytes; !got;) {
     if (c->sdf_buf) (void)hipFree(c->sdf_buf);
     c->sdf_buf = nullptr;
@@ -1686,7 +1750,7 @@ int rbh_sdf_build_noalloc(rbh_ctx* c, const double* V, int nv, const int* T, int
   HIPCHK(c, hipSetDevice(c->device));
   // the pruned build where its workspace fits the array too (the values are the same either way)
   const double most = sdf_extent(V, nv, mn, mx);
-  SdfLayout lay(nv, nt, (long)n, most, sdf_pruned(nv, nt, (long)n, most));
+  SdfLayout lay(nv, nt, (long)n, most, sdf_pruned(V, nv, T, nt, (long)n, most));
   if (lay.total > NOALLOC_SCRATCH_BYTES) lay = SdfLayout(nv, nt, (long)n, most, false);
   const hipError_t e = sdf_run(c->stream, lay, c->scratch, V, nv, T, nt, mn, mx, I, J, K, values, nullptr);
   if (e != hipSuccess) return fail(c, RBH_E_HIP, std::string("SDF kernel: ") + hipGetErrorString(e));

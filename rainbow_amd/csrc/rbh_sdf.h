@@ -489,7 +489,7 @@ __device__ __forceinline__ double sdf_angles(const SdfWork& w, double px, double
 // each (408 triangles with a hole on 51^3 1.03 ms by wavefronts, 1.06 by threads; on
 // 58^3 0.96, 0.82; on 128^3 8.3, 6.7; 9,999 on 51^3 7.4, 9.8; on 58^3 10.8, 9.6).
 // What is left over the plain build is least for strewn triangles, which cluster
-// badly: 500 on 128^3 10.2 ms (plain 10.3), 80 on 64^3 0.46 (0.45).
+// badly: 500 on 128^3 10.2 ms (plain 10.3).
 constexpr int SDF_MANY = 163840;
 __global__ void __launch_bounds__(256) k_sdf_sign(SdfWork w, SdfGrid g, int n) {
   __shared__ double st[SDF_TILE * 9];

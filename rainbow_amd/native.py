@@ -118,6 +118,7 @@ _PROTOS = {
     "rbh_get_tuning": [C.c_void_p, C.c_void_p],
     # include/rbh_testing.h
     "rbh_prefix_sum": [C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_void_p, C.POINTER(C.c_int)],
+    "rbh_sdf_is_pruned": [C.c_void_p, C.c_int, C.c_void_p, C.c_int, C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_int],
     "rbh_transfer_buffer": [C.c_void_p, C.POINTER(C.c_ulonglong)],
     "rbh_coop_grid": [C.c_int, C.c_int, C.c_int],
     "rbh_hinge_launch": [C.c_int, C.c_int, C.c_int, C.c_void_p, C.c_void_p, C.POINTER(C.c_int),
@@ -162,6 +163,16 @@ def _f64(a, n=None):
 
 def _i32(a):
     return np.ascontiguousarray(a, dtype=np.int32)
+
+
+def sdf_is_pruned(V, T, min_coord, max_coord, I, J, K):
+    """Whether sdf_build takes its pruned form (a test hook, include/rbh_testing.h)."""
+    V, T = _f64(V), _i32(T)
+    rc = load().rbh_sdf_is_pruned(_ptr(V), len(V), _ptr(T), len(T), _ptr(_f64(min_coord, 3)), _ptr(_f64(max_coord, 3)),
+                                  int(I), int(J), int(K))
+    if rc < 0:
+        raise RbhError(rc, "bad SDF arguments")
+    return rc == 1
 
 
 def hinge_launch(precision, cus, bodies, hinges):

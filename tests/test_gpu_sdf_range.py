@@ -168,7 +168,7 @@ def test_plain_forms_bitwise(ctx):
     assert np.signbit(out[0]).any() and not np.signbit(out[0]).all()
 
 
-@pytest.mark.parametrize("mesh", ["open255", "open256", "open257", "open408", "box"])
+@pytest.mark.parametrize("mesh", ["open511", "open512", "open513", "open719", "box"])   # (tiles of 256 triangles)
 def test_many_roots_bitwise(ctx, mesh):
     """Open meshes, whose every node has its own winding number: from 163,840 nodes on a thread takes a node, below a
     wavefront does.  Two grids on either side of the line agree in the nodes they share, on the faces of a box (winding
@@ -177,11 +177,13 @@ def test_many_roots_bitwise(ctx, mesh):
         V, T = quartered_box(3)
         T = T[1:]
     else:
-        V, T = sphere()
+        V, T = MESH.create_sphere(0.5, 20, 20)
+        V, T = np.ascontiguousarray(V), np.ascontiguousarray(T, dtype=np.int32)
         T = T[-int(mesh[4:]):]
     lo, h = np.full(3, -0.625), 1.0 / 32.0                   # exact spacing: shared nodes have the same coordinates
     out = [ctx.sdf_build(V, T, lo, lo + h * (np.array(n) - 1), *n).reshape(n[::-1]) for n in ((63, 64, 40), (64, 64, 40))]
     assert out[1].size == 163840
+    assert native.sdf_is_pruned(V, T, lo, lo + h * 62, 63, 64, 40)
     assert np.array_equal(bits(out[0]), bits(np.ascontiguousarray(out[1][:, :, :63])))
     hi = lo + h * 63
     many, plain = ctx.sdf_build(V, T, lo, hi, 128, 128, 128), ctx.sdf_build_noalloc(V, T, lo, hi, 128, 128, 128)
