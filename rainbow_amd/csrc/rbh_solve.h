@@ -2813,7 +2813,8 @@ template <typename R, int NT, int H> __global__ void __launch_bounds__(NT) k_sol
 }
 
 // A single scene (its lanes are its colouring units): the lanes split into
-// gridDim.x contiguous blocks, one per workgroup of a cooperative launch.
+// gridDim.x contiguous blocks, one per workgroup: a cooperative launch if there are several,
+// which wait for each other.
 template <typename R> __global__ void __launch_bounds__(SOLVE_BLOCK) k_solve_multi(Dev<R> d) {
   extern __shared__ __align__(32) unsigned char solve_smem[];
   double* sh_red;
