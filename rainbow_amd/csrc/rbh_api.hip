@@ -860,8 +860,8 @@ template <typename T> bool scan(rbh_ctx* c, const T* in, int* out, const int* n_
 // that a lane's wavefront shares its CU's LDS with no other and few groups outgrow
 // the resident layout (4096 spheres: solve 875 us, with four lanes per workgroup
 // 1137); but one workgroup for as many lanes as it has wavefronts, which spares the
-// exchange of the merit through memory (2.5 us of a sweep: 64 boxes in 3 lanes, 100
-// sweeps, 403 us in one workgroup, 447 in three).
+// cooperative launch and the exchange of the merit through memory (64 boxes in 3 lanes,
+// 100 sweeps, 40 steps a call: 570 us a step in one workgroup, 606 in three).
 int coop_grid(int units, int lanes_per_group, int most) {
   if (units <= 0) units = 64;
   if (lanes_per_group == 0 && units <= SOLVE_BLOCK / 64) return 1;
