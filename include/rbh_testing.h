@@ -43,6 +43,10 @@ int rbh_transfer_buffer(rbh_ctx* ctx, unsigned long long* bytes);
  * most workgroups that are resident at once. */
 int rbh_coop_grid(int units, int lanes_per_group, int most);
 
+/* The same for a scene of `bodies` bodies; units is 0 for a last step without
+ * contacts, negative if no step was seen. */
+int rbh_lone_grid(int units, int bodies, int lanes_per_group, int most);
+
 /* How the hinge solve of a batch would be launched (no device needed): n
  * hinged scenes of bodies[i] bodies in hinges[i] hinges on `cus` compute units.
  * *staged: 1 if their rows are staged in LDS; *lds: bytes of a workgroup;

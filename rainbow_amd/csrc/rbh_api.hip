@@ -179,7 +179,7 @@ struct rbh_ctx {
   // resident solve groups: most contacts and bodies (rbh_tuning), and the launch's dynamic LDS
   int res_cap_c = 0, res_cap_b = 0;
   size_t solve_lds = 0, solve_lds_half = 0;   // full and half layouts (one or two workgroups per CU)
-  int max_iter_batch = 1, coop_max = 0, last_units = 0;
+  int max_iter_batch = 1, coop_max = 0, last_units = -1;   // last_units: of the last step seen, -1: none seen
   bool multi_ok = false;
   bool any_post = false;    // a scene of the batch has post-stabilisation on (set per run_steps call)
   long long ws_gen = 0;
@@ -793,7 +793,7 @@ int build_batch(rbh_ctx* c, const int* ids, int n) {
   c->max_iter_batch = max_iter;
   c->multi_ok = n == 1;
   c->unit_T = c->tune.unit_size > 0 ? c->tune.unit_size : 64;
-  c->last_units = 0;
+  c->last_units = -1;
   // initial capacities; they grow when a step reports an overflow
   long long est_pairs = std::min<long long>(pairs_all, 64LL * c->nb + 4096);
   c->cap_pairs = std::max(c->cap_pairs, (int)std::max<long long>(est_pairs, 1));
@@ -855,7 +855,7 @@ template <typename T> bool scan(rbh_ctx* c, const T* in, int* out, const int* n_
 }
 
 // Workgroups of a lone scene's cooperative solve, from the unit count of the
-// last step seen (0: none seen, or one without contacts, whose next step may
+// last step seen (0 or less: none seen, or one without contacts, whose next step may
 // have any number): one lane per workgroup while the device has room for them, so
 // that a lane's wavefront shares its CU's LDS with no other and few groups outgrow
 // the resident layout (4096 spheres: solve 875 us, with four lanes per workgroup
@@ -869,7 +869,19 @@ int coop_grid(int units, int lanes_per_group, int most) {
   return std::max(1, std::min((units + per - 1) / per, most));
 }
 
-// steps between re-sizings of a single scene's cooperative solve grid
+// The same for a scene of `bodies` bodies, units < 0 if no step was seen.  Seen without
+// contacts, a scene of up to IDLE_BODIES bodies gets one workgroup, and no cooperative
+// launch (3 boxes falling, 40 steps a call: 150 us a step, 186 with 64 workgroups).
+// Should contacts arrive before it is looked at again, one workgroup is about as good up
+// to there (64 boxes 404 us a step, a lane a group 459; 64 spheres 971 and 1034; but a
+// dense pile of 16 2.3 ms and 1.0) and not beyond (600 boxes 1.9 ms and 0.6).
+constexpr int IDLE_BODIES = 64;
+int lone_grid(int units, int bodies, int lanes_per_group, int most) {
+  if (units == 0 && bodies <= IDLE_BODIES && lanes_per_group == 0) return 1;
+  return coop_grid(units, lanes_per_group, most);
+}
+
+// steps between re-sizings of a single scene's solve grid
 constexpr int GRID_REFRESH = 16;
 
 // Events of step i of a call of `todo` steps: the last TIMED_STEPS steps are
@@ -1113,7 +1125,7 @@ template <typename R> int run_steps(rbh_ctx* c, int n_steps, double dt, int flag
   bool multi = c->multi_ok && !use_graph;
   if (flags & RBH_STEP_FORCE_SINGLE) multi = false;
   if ((flags & RBH_STEP_FORCE_MULTI) && c->multi_ok && !use_graph) multi = true;
-  int multi_grid = coop_grid(c->last_units, c->tune.lanes_per_group, c->coop_max);
+  int multi_grid = lone_grid(c->last_units, c->nb, c->tune.lanes_per_group, c->coop_max);
   int done = 0;
   StepEnd end{};
   for (int attempt = 0; attempt < 16 && done < n_steps; ++attempt) {
@@ -1147,11 +1159,11 @@ template <typename R> int run_steps(rbh_ctx* c, int n_steps, double dt, int flag
         hipError_t le = launch_step<R>(c, dt, kflags, timing ? timing_row(c, i, todo) : nullptr, multi, multi_grid);
         if (le != hipSuccess) return fail(c, RBH_E_HIP, std::string("step launch: ") + hipGetErrorString(le));
         if (multi && (i + 1) % GRID_REFRESH == 0 && i + 1 < todo) {
-          // re-size the cooperative grid to the scene's current unit count
+          // re-size the grid to the scene's current unit count
           int nu = 0;
           HIPCHK(c, hipMemcpyAsync(&nu, c->n_units.p, 4, hipMemcpyDeviceToHost, c->stream));
           HIPCHK(c, hipStreamSynchronize(c->stream));
-          if (nu > 0) multi_grid = coop_grid(nu, c->tune.lanes_per_group, c->coop_max);
+          if (nu > 0 || c->nb <= IDLE_BODIES) multi_grid = lone_grid(nu, c->nb, c->tune.lanes_per_group, c->coop_max);
         }
       }
     }
@@ -1650,6 +1662,11 @@ int rbh_transfer_buffer(rbh_ctx* c, unsigned long long* bytes) {
 int rbh_coop_grid(int units, int lanes_per_group, int most) {
   if (units < 0 || lanes_per_group < 0 || most < 1) return RBH_E_ARG;
   return coop_grid(units, lanes_per_group, most);
+}
+
+int rbh_lone_grid(int units, int bodies, int lanes_per_group, int most) {
+  if (bodies < 1 || lanes_per_group < 0 || most < 1) return RBH_E_ARG;
+  return lone_grid(units, bodies, lanes_per_group, most);
 }
 
 int rbh_hinge_launch(int precision_bytes, int cus, int n, const int* bodies, const int* hinges, int* staged,

@@ -121,6 +121,7 @@ _PROTOS = {
     "rbh_sdf_is_pruned": [C.c_void_p, C.c_int, C.c_void_p, C.c_int, C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_int],
     "rbh_transfer_buffer": [C.c_void_p, C.POINTER(C.c_ulonglong)],
     "rbh_coop_grid": [C.c_int, C.c_int, C.c_int],
+    "rbh_lone_grid": [C.c_int, C.c_int, C.c_int, C.c_int],
     "rbh_hinge_launch": [C.c_int, C.c_int, C.c_int, C.c_void_p, C.c_void_p, C.POINTER(C.c_int),
                          C.POINTER(C.c_longlong), C.c_void_p],
     "rbh_hinge_occupancy": [C.c_void_p, C.c_int, C.c_longlong, C.POINTER(C.c_int)],
